@@ -41,14 +41,13 @@ def log(msg):
 
 
 def flops_per_bead_step(n, D):
-    """FP64 work the kernel executes per bead-step (no credit for padding).  Transforms:
-    for even N the folded DST-I (two N/2 x N/2 halves per transform, 4 N D for the two
-    transforms of the 2D state columns) plus its pre-fold and recombination (4 D); for odd
-    N the dense N x N transforms (8 N D).  Elementwise kick / rotations / O-step / shifts:
-    21 D.  EVB potential: two wells, each y = W^T (x - xw) and W h (2 x 2 D^2) plus ~13 D."""
-    w_pes = 8 * D * D + 26 * D
-    transforms = 4 * n * D + 4 * D if n % 2 == 0 else 8 * n * D
-    return transforms + 21 * D + w_pes
+    """FP64 work the kernel executes per bead-step (no credit for padding).  One transform of
+    the step's normals, split into odd and even modes (n D) and recombined (2 D); the linear
+    A-O-A step with its closed-form solve along the chain (30 D); the normals by Box-Muller
+    (45 D).  EVB potential: y = W^T (x - xw) and W h once (4 D^2), the second well's difference
+    in the columns of the two exchanged atoms (24 D), and 28 D elementwise."""
+    w_pes = 4 * D * D + 52 * D
+    return n * D + 77 * D + w_pes
 
 
 def build_polymers(sp, ns, ntraj, nlam):

@@ -198,14 +198,16 @@ int rp_batch_get_kick_cursor(rp_batch *b, int64_t *kick_cursor);
 int rp_batch_set_cursor(rp_batch *b, const int64_t *cursor, const int64_t *kick_cursor);
 /* families of equal (n, betan), one fused-kernel launch each: n[f], count[f] */
 int rp_batch_families(rp_batch *b, int *nfam, int *n, int *count);
-/* the fused-kernel instance family `fam` runs: waves per workgroup, MFMA units per wave
- * (a unit is 32 normal modes x 16 dofs of x and p) and whether its transforms are folded
- * into two half-size products (even n) */
+/* launch shape of family `fam`: its wave budget (2, 4 or 8), the MFMA units (32 normal modes x
+ * 16 dofs) per wave of the budget, and whether n is even and the potential not the water
+ * cluster (1 / 0).  A workgroup holds as many polymers as the budget has waves per 32 beads of
+ * one, at least one */
 int rp_batch_family_shape(rp_batch *b, int fam, int *waves, int *units_per_wave, int *folded);
-/* launch shape: steps per launch (>= 1; 0 keeps the current value) and waves per
- * polymer workgroup (2, 4 or 8 for every family; 0 keeps each family's value; 8 applies to
- * families of at most 16 MFMA units, 2 to families of at most 2 units with at most 2 dof
- * tiles, the others take 4).  rp_batch_autotune times, on the live batch (state saved and
+/* launch shape: steps per launch (>= 1; 0 keeps the current value) and the wave budget of a
+ * workgroup (2, 4 or 8 for every family; 0 keeps each family's value; 8 applies to families of
+ * at most 16 MFMA units, 2 to families of at most 2 units with at most 2 dof tiles, the others
+ * take 4).  Until a budget is set, polymers per workgroup are picked by occupancy.
+ * rp_batch_autotune times, on the live batch (state saved and
  * restored), 2, 4 and 8 waves per family from each family's own launch timings, then the
  * steps-per-launch candidates; it keeps the fastest and reports the steps and the most
  * frequent wave count. */

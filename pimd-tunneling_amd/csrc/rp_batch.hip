@@ -19,8 +19,9 @@ struct Family {
   int N = 0, NPAD = 0;
   double betan = 0;
   int first = 0, count = 0;  // polymers [first, first+count) in batch order
-  int waves = 4;             // waves per workgroup of this family's step kernel (4 or 8)
-  DevBuf<double> d_T, d_Tf, d_modes;
+  int waves = 4;             // wave budget of a workgroup (2, 4 or 8)
+  bool waves_set = false;    // by set_launch or autotune, else the launch picks by occupancy
+  DevBuf<double> d_T, d_Tf, d_lam;
 };
 }  // namespace
 
@@ -43,7 +44,7 @@ struct rp_batch {
   DevBuf<uint64_t> d_stream;
   DevBuf<int32_t> d_kicks;
   DevBuf<int> d_flags;
-  int npath = 0;
+  int npath = 0, ncu = 1;
   int64_t kick_cap = 0;
   int64_t steps_done = 0;
   int steps_per_launch = 64;
@@ -77,57 +78,28 @@ static void graph_drop(rp_batch* b) {
   b->graphs.clear();
 }
 
-// Folded halves of T for even N (H = N/2, HPAD = H rounded up to 16): row r of the odd
-// half is mode 2r+1 and row r of the even half mode 2r+2 (1-based), both over beads
-// 1..H.  Because sin(i (N+1-l) pi/(N+1)) = (-1)^(i+1) sin(i l pi/(N+1)), T x splits into
-// odd modes = Todd (x_l + x_{N+1-l}) and even modes = Teven (x_l - x_{N+1-l}), half the
-// multiply-adds; the identity holds to 3.4e-13 relative at N = 256 with the reference's
-// truncated pi.
-// Stored four times, each HPAD x HPAD and zero-padded: [odd^T | even^T | odd | even],
-// the transposes for the forward transform and the halves themselves for the backward one,
-// so both read rows of 16 consecutive entries.
-static void family_folded(const Family& f, const std::vector<double>& T, std::vector<double>& Tf) {
-  const int N = f.N, NP = f.NPAD, H = N / 2, HP = (H + 15) / 16 * 16;
-  const size_t Q = (size_t)HP * HP;
-  Tf.assign(4 * Q, 0.0);
-  for (int r = 0; r < H; ++r)
-    for (int k = 0; k < H; ++k) {
-      const double to = T[(size_t)(2 * r) * NP + k], te = T[(size_t)(2 * r + 1) * NP + k];
-      Tf[(size_t)k * HP + r] = to;
-      Tf[Q + (size_t)k * HP + r] = te;
-      Tf[2 * Q + (size_t)r * HP + k] = to;
-      Tf[3 * Q + (size_t)r * HP + k] = te;
-    }
-}
-
-static void family_tables(const rp_batch* b, const Family& f, std::vector<double>& T,
-                          std::vector<double>& modes) {
-  const int N = f.N, NP = f.NPAD;
+// T lam in two halves, odd and even modes: Tf[half][r][l] = T(2 r + half, l) lam(2 r + half)
+// over beads l < ceil(N/2), each half HP x HP and zero-padded.  Because
+// sin(i (N+1-l) pi/(N+1)) = (-1)^(i+1) sin(i l pi/(N+1)), the other beads' values are the odd
+// modes' sum minus the even modes': half the multiply-adds.  The identity holds to 3.4e-13
+// relative at N = 256 with the reference's truncated pi.
+static void family_tables(const Family& f, std::vector<double>& T, std::vector<double>& Tf,
+                          std::vector<double>& lam) {
+  const int N = f.N, NP = f.NPAD, Hc = (N + 1) / 2, HP = 16 * batch_tiles(N);
   T.assign((size_t)NP * NP, 0.0);
-  modes.assign((size_t)NP * kMODE, 0.0);
-  for (int i = 1; i <= N; ++i)
+  Tf.assign(2 * (size_t)HP * HP, 0.0);
+  lam.assign(NP, 0.0);
+  for (int i = 1; i <= N; ++i) {
+    lam[i - 1] = 2.0 * std::sin((double)i * kPiRef / (double)(2 * N + 2)) / f.betan;
     for (int l = i; l <= N; ++l) {
       double t = std::sin((double)(i * l) * kPiRef / (double)(N + 1)) * std::sqrt(2.0 / (double)(N + 1));
       T[(size_t)(i - 1) * NP + (l - 1)] = t;
       T[(size_t)(l - 1) * NP + (i - 1)] = t;
     }
-  for (int i = 0; i < NP; ++i) {
-    double* md = modes.data() + (size_t)i * kMODE;
-    if (i < N) {
-      const int ii = i + 1;
-      const double lam = 2.0 * std::sin((double)ii * kPiRef / (double)(2 * N + 2)) / f.betan;
-      const double lb = lam * f.betan;
-      const double c = std::sqrt(2.0 / (double)(N + 1)) / (lb * lb);
-      md[MD_MU] = lam * lam;
-      md[MD_IMU] = 1.0 / (lam * lam);
-      md[MD_U] = std::sin((double)ii * kPiRef / (double)(N + 1)) * c;
-      md[MD_W] = std::sin((double)(N * ii) * kPiRef / (double)(N + 1)) * c;
-      md[MD_LAM] = lam;
-    } else {  // padded modes: state stays zero; keep every coefficient finite
-      md[MD_MU] = 1.0;
-      md[MD_IMU] = 1.0;
-    }
   }
+  for (int i = 0; i < N; ++i)
+    for (int l = 0; l < Hc; ++l)
+      Tf[((size_t)(i & 1) * HP + (i >> 1)) * HP + l] = T[(size_t)i * NP + l] * lam[i];
 }
 
 static int batch_flags(rp_batch* b) {
@@ -155,18 +127,12 @@ bool rp::batch_supports(const rp_pes* pes, int n) {
     case PES_COUPLED2D: kind_ok = true; break;
     default: kind_ok = false;  // host potentials and unknown kinds
   }
-  const int npad = (n + 31) / 32 * 32;
-  return kind_ok && batch_lds_bytes(npad, batch_dtiles(pes), batch_pes_lds(pes, n)) <= 160 * 1024;
+  return kind_ok && batch_size_ok(pes, n);
 }
 
-// Waves per workgroup by default: 8 (two per SIMD, which hides the latency of the
-// elementwise phases) from 8 to 16 MFMA units, 4 otherwise.  16 waves (four per SIMD, one
-// unit each) measured slower at every N (8-step launch of 5632 polymers, ms, 8 / 16 waves:
-// N = 128 4.39 / 8.75, 192 7.50 / 11.20, 256 11.31 / 13.59).  Measured on the 27-dof EVB
-// (ms per 8-step launch of 5632 polymers, 4 / 8 waves): 2 units 1.37 / 2.15, 4 units
-// 1.69 / 2.68, 6 units 3.43 / 3.85 (two 4-wave workgroups share a CU), 8 units 5.30 / 4.37,
-// 12 units 8.88 / 7.51, 16 units 13.4 / 11.3.  Four 2-wave workgroups per CU for 2 units (no
-// idle wave) measured 1.45 ms against 1.36 for two 4-wave ones.
+// A family's wave budget as rp_batch_family_shape reports it and rp_batch_set_launch bounds
+// it: 8 from 8 to 16 MFMA units (32 modes x 16 dofs), 2 for at most 2, else 4.  Until a budget
+// is asked for, the launch picks its groups per workgroup by occupancy (launch_batch_kind).
 static int default_waves(int DT, int NPAD) {
   const int units = (NPAD >> 5) * DT;
   if (units <= 2 && DT <= 2) return 2;
@@ -177,33 +143,41 @@ static BatchArgs base_args(rp_batch* b, const Family& f, double h) {
   BatchArgs a;
   memset(&a, 0, sizeof(a));
   a.pes = b->pes->dev();
-  a.waves = f.waves;
+  a.waves = f.waves_set ? f.waves : 0;
   a.N = f.N;
   a.NPAD = f.NPAD;
   a.D = b->D;
   a.ndim = b->ndim;
   a.natom = b->natom;
-  a.LD = 2 * b->DC + 1;
+  a.ncu = b->ncu;
+  if (b->pes->kind == PES_EVB)
+    for (int d = 0; d < b->D; ++d)
+      if (b->pes->ip[d / b->ndim] != d / b->ndim) a.moved |= 1u << (d / 4);
   a.first = f.first;
   a.dt = b->dt;
   a.limit = b->limit;
   a.stdev0 = std::sqrt(1.0 / f.betan);
   a.tau = b->tau;
   const double tau = b->tau;
+  double c, sq, sp;
   if (b->cayley) {
     const double w2 = h * h / (tau * tau);
-    a.c = (4.0 - w2) / (4.0 + w2);
-    a.sq = 4.0 * h / (tau * tau * (4.0 + w2));
-    a.sp = 4.0 * h / (4.0 + w2);
+    c = (4.0 - w2) / (4.0 + w2);
+    sq = 4.0 * h / (tau * tau * (4.0 + w2));
+    sp = 4.0 * h / (4.0 + w2);
   } else {
-    a.c = std::cos(h / tau);
-    a.sq = std::sin(h / tau) / tau;
-    a.sp = tau * std::sin(h / tau);
+    c = std::cos(h / tau);
+    sq = std::sin(h / tau) / tau;
+    sp = tau * std::sin(h / tau);
   }
-  const double c1 = std::exp(-b->gamma * b->dt / tau);
+  const double c1 = std::exp(-b->gamma * b->dt / tau), c1sq = c1 * c1;
   const double c2 = std::sqrt(1.0 - c1 * c1);
-  a.c1sq = c1 * c1;
   a.kappa = tau * c2 * std::sqrt((1.0 + c1 * c1) / f.betan);
+  const double bn2 = f.betan * f.betan, gx = sq * bn2 / (f.N + 1), ck = sp / bn2;
+  a.iG = 1.0 / (f.N + 1);
+  a.rot = Linear{c, gx, 1.0, c, ck, 0.0};
+  a.aoa = Linear{c * c - sq * sp * c1sq, gx, c * (1.0 + c1sq), c * c * c1sq - sp * sq,
+                 ck * c * (1.0 + c1sq), c};
   a.noutput = b->noutput;
   a.seed = b->seed;
   a.state = b->d_state.p;
@@ -212,8 +186,7 @@ static BatchArgs base_args(rp_batch* b, const Family& f, double h) {
   a.stream = b->d_stream.p;
   a.T = f.d_T.p;
   a.Tf = f.d_Tf.p;
-  a.fold = (f.N % 2 == 0) && f.d_Tf.p != nullptr;
-  a.modes = f.d_modes.p;
+  a.lam = f.d_lam.p;
   a.pdata = b->d_pdata.p;
   a.massd = b->d_massd.p;
   a.npath = b->npath;
@@ -271,8 +244,7 @@ extern "C" int rp_batch_create(rp_pes* pes, const double* mass, int npoly,
     if (n < 2 || n > 256) return fail(set_error(RP_ERR_ARG, "polymer %d: n=%d outside 2..256", p, n));
     if (!(desc[p].betan > 0) || !desc[p].a || !desc[p].b || !desc[p].dbdl)
       return fail(set_error(RP_ERR_ARG, "polymer %d: bad descriptor", p));
-    const int npad = (n + 31) / 32 * 32;
-    if (batch_lds_bytes(npad, b->DT, batch_pes_lds(pes, n)) > 160 * 1024)
+    if (!batch_size_ok(pes, n))
       return fail(set_error(RP_ERR_ARG, "polymer %d: n=%d with %d dof needs more LDS than a CU has",
                             p, n, b->D));
   }
@@ -320,6 +292,9 @@ extern "C" int rp_batch_create(rp_pes* pes, const double* mass, int npoly,
   int zf[2] = {0, 0};
   if ((rc = [&]() -> int {
         RP_HIP(hipStreamCreateWithFlags(&b->s, hipStreamNonBlocking));
+        int dev = 0;
+        RP_HIP(hipGetDevice(&dev));
+        RP_HIP(hipDeviceGetAttribute(&b->ncu, hipDeviceAttributeMultiprocessorCount, dev));
         b->fev.assign(2 * b->fam.size(), nullptr);
         for (auto& e : b->fev) RP_HIP(hipEventCreate(&e));
         int r;
@@ -332,16 +307,12 @@ extern "C" int rp_batch_create(rp_pes* pes, const double* mass, int npoly,
         if ((r = b->d_massd.alloc(DC)) || (r = b->d_massd.upload(massd.data(), DC, b->s))) return r;
         if ((r = b->d_flags.alloc(2)) || (r = b->d_flags.upload(zf, 2, b->s))) return r;
         for (Family& f : b->fam) {
-          std::vector<double> T, modes;
-          family_tables(b, f, T, modes);
+          std::vector<double> T, Tf, lam;
+          family_tables(f, T, Tf, lam);
           if ((r = f.d_T.alloc(T.size())) || (r = f.d_T.upload(T.data(), T.size(), b->s))) return r;
-          if (f.N % 2 == 0) {
-            std::vector<double> Tf;
-            family_folded(f, T, Tf);
-            if ((r = f.d_Tf.alloc(Tf.size())) || (r = f.d_Tf.upload(Tf.data(), Tf.size(), b->s))) return r;
-          }
-          if ((r = f.d_modes.alloc(modes.size())) || (r = f.d_modes.upload(modes.data(), modes.size(), b->s)))
-            return r;
+          if ((r = f.d_Tf.alloc(Tf.size())) || (r = f.d_Tf.upload(Tf.data(), Tf.size(), b->s))) return r;
+          if ((r = f.d_lam.alloc(lam.size())) || (r = f.d_lam.upload(lam.data(), lam.size(), b->s))) return r;
+          RP_HIP(hipStreamSynchronize(b->s));  // the host tables are released here
         }
         RP_HIP(hipStreamSynchronize(b->s));
         return RP_OK;
@@ -359,7 +330,7 @@ extern "C" int rp_batch_destroy(rp_batch* b) {
   for (Family& f : b->fam) {
     f.d_T.free();
     f.d_Tf.free();
-    f.d_modes.free();
+    f.d_lam.free();
   }
   for (DevBuf<double>* d : {&b->d_state, &b->d_pf64, &b->d_pdata, &b->d_massd, &b->d_noise, &b->d_pathd})
     d->free();
@@ -440,7 +411,7 @@ __global__ void __launch_bounds__(256) batch_init_kernel(BatchArgs A) {
     const int atom = c / ndim, dim = c - atom * ndim;
     const int64_t idx = cur + (int64_t)(dim * natom + atom) * N + i;
     const double z = A.noise ? A.noise[noff + idx] : philox_normal(A.seed, strm, idx);
-    V[e] = (A.stdev0 * z) * (sqrt(A.massd[c]) * A.modes[i * kMODE + MD_LAM] * A.tau);
+    V[e] = (A.stdev0 * z) * (sqrt(A.massd[c]) * A.lam[i] * A.tau);
   }
   __syncthreads();
   const double xi = A.pf64[(size_t)poly * kPF64 + PF_XI];
@@ -489,7 +460,7 @@ static rp_batch::GraphKey graph_key(const rp_batch* b, size_t fi, int steps, int
   k.kicks = b->d_kicks.p;
   k.pathd = b->d_pathd.p;
   k.npath = b->npath;
-  for (const Family& f : b->fam) k.waves.push_back(f.waves);
+  for (const Family& f : b->fam) k.waves.push_back(f.waves_set ? f.waves : 0);
   return k;
 }
 
@@ -770,7 +741,10 @@ extern "C" int rp_batch_set_launch(rp_batch* b, int steps_per_launch, int waves)
              "rp_batch_set_launch: waves per workgroup must be 2, 4 or 8");
   if (steps_per_launch > 0) b->steps_per_launch = steps_per_launch;
   if (waves)
-    for (Family& f : b->fam) f.waves = fitted_waves(b, f, waves);
+    for (Family& f : b->fam) {
+      f.waves = fitted_waves(b, f, waves);
+      f.waves_set = true;
+    }
   return RP_OK;
 }
 
@@ -813,7 +787,10 @@ extern "C" int rp_batch_autotune(rp_batch* b, int trial_steps, int* best_steps, 
   std::vector<int> best_w(nf, 4);
   double sec = 0.0;
   for (int w : {2, 4, 8}) {
-    for (Family& f : b->fam) f.waves = fitted_waves(b, f, w);
+    for (Family& f : b->fam) {
+      f.waves = fitted_waves(b, f, w);
+      f.waves_set = true;
+    }
     if ((rc = trial(std::min(b->steps_per_launch, trial_steps), fam_ms, sec))) return rc;
     for (size_t fi = 0; fi < nf; ++fi)
       if (b->fam[fi].waves == w && fam_ms[fi] < best_ms[fi]) {
@@ -859,12 +836,11 @@ extern "C" int rp_batch_family_shape(rp_batch* b, int fam, int* waves, int* unit
                                      int* folded) {
   RP_REQUIRE(b && fam >= 0 && fam < (int)b->fam.size(), "rp_batch_family_shape: bad arguments");
   const Family& f = b->fam[fam];
-  // the kernel instance launch_batch_thermo picks: units of 32 modes x 16 dofs (folded: 16
-  // rows of each half x 16 dofs; the same count), dealt over the waves of a workgroup
+  // units of 32 modes x 16 dofs over the wave budget
   const int units = (f.NPAD >> 5) * b->DT;
   if (waves) *waves = f.waves;
   if (units_per_wave) *units_per_wave = (units + f.waves - 1) / f.waves;
-  if (folded) *folded = (f.N % 2 == 0) && f.d_Tf.p != nullptr && b->pes->kind != PES_WATER;
+  if (folded) *folded = (f.N % 2 == 0) && b->pes->kind != PES_WATER;
   return RP_OK;
 }
 

@@ -5,10 +5,9 @@
 
 namespace rp {
 
-
-// f(integral_constant<int, 0..N-1>) expanded at compile time: the accumulator indices
-// stay constants even where a loop body is too large for the unroller, so the
-// accumulators never fall back to scratch memory.
+// f(integral_constant<int, 0..N-1>) expanded at compile time: the state's register indices
+// stay constants even where a loop body is too large for the unroller, so the state never
+// falls back to scratch memory.
 template <typename F, int... I>
 __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
   (f(std::integral_constant<int, I>{}), ...);
@@ -22,471 +21,305 @@ __device__ __forceinline__ d4 mfma_f64(double a, double b, d4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ double batch_draw(const BatchArgs& A, int64_t noff, uint64_t strm,
-                                             int64_t idx) {
-  if (A.noise) return A.noise[noff + idx];
-  return philox_normal(A.seed, strm, idx);
+// DPP moves inside each row of 16 lanes; a lane without a source keeps `old`, or gets zero
+template <int CTRL>
+__device__ __forceinline__ double row_mov(double old, double v) {
+  return __builtin_amdgcn_update_dpp(old, v, CTRL, 0xF, 0xF, false);
+}
+template <int CTRL>
+__device__ __forceinline__ double row_mov0(double v) {
+  return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, true);
+}
+constexpr int kShr = 0x110, kShl = 0x100;  // row_shr:n, row_shl:n
+
+// inclusive sums over each row of 16 lanes, toward higher / lower lanes
+__device__ __forceinline__ double row_prefix(double v) {
+  v += row_mov0<kShr + 1>(v);
+  v += row_mov0<kShr + 2>(v);
+  v += row_mov0<kShr + 4>(v);
+  v += row_mov0<kShr + 8>(v);
+  return v;
+}
+__device__ __forceinline__ double row_suffix(double v) {
+  v += row_mov0<kShl + 1>(v);
+  v += row_mov0<kShl + 2>(v);
+  v += row_mov0<kShl + 4>(v);
+  v += row_mov0<kShl + 8>(v);
+  return v;
 }
 
-// Number of unit slots of this wave that hold a real unit (wave-uniform): slots u < NU.
-template <int UPW, int W>
-__device__ __forceinline__ int active_units(int wave, int units) {
-  return max(0, min(UPW, (units - wave + W - 1) / W));
+__device__ __forceinline__ bool nonfinite(double v) { return !(fabs(v) < INFINITY); }
+
+// The kernel's arguments in the constant segment they arrive in.  A phase reads them through
+// an opaque copy of the segment's address (refresh), so they are scalar loads where they are
+// used: as ordinary arguments the compiler kept all of them, and every lane's LDS addresses,
+// in registers across the step loop, and spilled (160 SGPRs and, on the 27-dof EVB, 200
+// VGPRs beyond the 256 of two waves per SIMD).
+typedef const __attribute__((address_space(4))) BatchArgs KernArgs;
+
+// One polymer group's place in the workgroup: pointers into LDS (batch_lds, rp_batch.h), the
+// wave's half and tile, and the lane's bead.  The half h = 0 counts beads l = 0, 1, ... from
+// the start of the chain, h = 1 from its end; both meet in the middle (the lower half has
+// the middle bead of an odd chain).
+struct Lane {
+  double *Z, *E, *Tot, *Row, *Own;
+  int h, tile, nt;     // wave-uniform: the wave's half and bead tile, tiles per half
+  int own;             // doubles of a wave's own area
+  int wtid, wthreads;  // this thread among the group's threads
+  int m, g;            // MFMA lane coordinates
+  int l, bead;         // bead l of the half, bead N-1-l or l of the chain
+  bool on, last;       // l is a bead of the half; its last one
+};
+
+// LDS place of normal `col` (row of the state) of mode 2 r + half.  The column's bit 4 is
+// flipped on odd r: the four mode rows an MFMA operand load reads then fall in distinct banks.
+template <int DC>
+__device__ __forceinline__ int z_at(int HP, int half, int r, int col) {
+  return (half * HP + r) * DC + (DC > 16 ? col ^ ((r & 1) << 4) : col);
 }
 
-// f(integral_constant<int, nu>) for the wave-uniform nu in [0, UPW]: the GEMMs below are
-// instantiated per active-unit count, so a wave issues no MFMA for an empty slot.
-template <int UPW, typename F>
-__device__ __forceinline__ void with_units(int nu, F&& f) {
-  static_for<UPW + 1>([&](auto NU) __attribute__((always_inline)) {
-    if (nu == decltype(NU)::value) f(NU);
-  });
-}
-
-// acc = T S for the first NU units of this wave (see rp_batch.h for the unit layout);
-// accumulators of the other slots are zero and are dropped by the consumers.  Measured on
-// the 27-dof EVB at N = 192 (12 units in 16 slots of 8 waves): 8.64 -> 7.70 ms per 8-step
-// launch against recomputing the last unit in the empty slots.
-template <int DT, int UPW, int W, int NU>
-__device__ __forceinline__ void gemm_T_n(const double* __restrict__ T, int NPAD, const double* S,
-                                         int LD, int wave, int m, int g, d4 (&acc)[UPW][4]) {
-#pragma unroll
-  for (int u = 0; u < UPW; ++u)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc[u][c] = d4{0.0, 0.0, 0.0, 0.0};
-  if constexpr (NU > 0) {
-    const int nk = NPAD >> 2;  // a multiple of 8: NPAD is a multiple of 32
-    // Two register sets in ping-pong: the fragments of K-chunk kc+1 are loaded into one
-    // set while the MFMAs of chunk kc read the other, so a load has a whole chunk of
-    // MFMAs (16 x NU x 4 cycles x 16) to arrive and no register copy sits between them.
-    const int units = (NPAD >> 5) * DT;
-    int toff[NU], soff[NU];
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      const int unit = min(wave + u * W, units - 1);
-      const int rp = unit / DT, dtile = unit - rp * DT;
-      toff[u] = g * NPAD + rp * 32 + m;
-      soff[u] = g * LD + dtile * 16 + m;
+// The normals of one O-step (or, `resample`, of a momentum resample: blocks of N in (dim
+// outer, atom inner) order, verletmodule.f90:102-106, 211-215) into Z.  A thread makes the
+// Philox blocks of one row: both normals of a block belong to consecutive modes.  Lanes run
+// over the rows, so the LDS writes of a wave are consecutive.  N draws from position s take
+// N/2 blocks when N and s are even (`whole`, in every row), else N/2 + 1.  PACK: cur counts
+// from each polymer's own position.
+template <int DC, bool PACK>
+__device__ __forceinline__ void make_noise(KernArgs& A, const Lane& L, int R, int64_t cur,
+                                           uint64_t strm, int64_t noff, bool whole,
+                                           bool resample) {
+  const int N = A.N, D = A.D, HP = 16 * L.nt;
+  const int NB = whole ? N >> 1 : (N >> 1) + 1;
+  int row = L.wtid % R, q = L.wtid / R;
+  const int drow = L.wthreads % R, dq = L.wthreads / R;
+  while (q < NB) {
+    int d = row;
+    int64_t c = cur;
+    uint64_t st = strm;
+    if constexpr (PACK) {
+      const int pol = row / D;
+      d = row - pol * D;
+      const int64_t* ci = reinterpret_cast<const int64_t*>(L.Row + RW_CUR * DC);
+      c = ci[pol] + cur;
+      st = (uint64_t)ci[DC + pol];
     }
-    double a0[2][NU], a1[2][NU], bx[2][NU], bp[2][NU];
-    auto load = [&](int set, int kc) __attribute__((always_inline)) {
-      const double* Tk = T + (size_t)(4 * kc) * NPAD;  // wave-uniform chunk base
-      const double* Sk = S + 4 * kc * LD;
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        a0[set][u] = Tk[toff[u]];
-        a1[set][u] = Tk[toff[u] + 16];
-        bx[set][u] = Sk[soff[u]];
-        bp[set][u] = Sk[soff[u] + DT * 16];
-      }
-    };
-    auto mma = [&](int set) __attribute__((always_inline)) {
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        acc[u][0] = mfma_f64(a0[set][u], bx[set][u], acc[u][0]);
-        acc[u][1] = mfma_f64(a0[set][u], bp[set][u], acc[u][1]);
-        acc[u][2] = mfma_f64(a1[set][u], bx[set][u], acc[u][2]);
-        acc[u][3] = mfma_f64(a1[set][u], bp[set][u], acc[u][3]);
-      }
-    };
-    load(0, 0);
-    for (int kc = 0; kc < nk; kc += 2) {
-      load(1, kc + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      mma(0);
-      __builtin_amdgcn_sched_barrier(0);
-      load(0, kc + 2 < nk ? kc + 2 : kc + 1);  // the last prefetch re-reads a valid chunk
-      __builtin_amdgcn_sched_barrier(0);
-      mma(1);
-      __builtin_amdgcn_sched_barrier(0);
+    const int blk = resample ? (d % A.ndim) * A.natom + d / A.ndim : d;
+    const int64_t s = c + (int64_t)blk * N;
+    const uint64_t b = (uint64_t)(s >> 1) + (uint64_t)q;
+    const int i0 = (int)(2 * (int64_t)b - s), i1 = i0 + 1;  // -1 <= i0 <= N
+    double z0, z1;
+    if (A.noise) {
+      z0 = (i0 >= 0 && i0 < N) ? A.noise[noff + s + i0] : 0.0;
+      z1 = (i1 < N) ? A.noise[noff + s + i1] : 0.0;
+    } else {
+      philox_normal2(A.seed, st, b, z0, z1);
     }
-  }
-}
-
-template <int DT, int UPW, int W>
-__device__ __forceinline__ void gemm_T(const double* __restrict__ T, int NPAD, const double* S,
-                                       int LD, int wave, int m, int g, d4 (&acc)[UPW][4]) {
-  if constexpr (UPW == 1) {
-    // one slot: a wave past the last unit recomputes the last unit (its result is dropped
-    // by the consumers); the branch-free form keeps the one-unit kernels' registers
-    gemm_T_n<DT, 1, W, 1>(T, NPAD, S, LD, wave, m, g, acc);
-  } else {
-    const int units = (NPAD >> 5) * DT;
-    with_units<UPW>(active_units<UPW, W>(wave, units), [&](auto NU) __attribute__((always_inline)) {
-      gemm_T_n<DT, UPW, W, decltype(NU)::value>(T, NPAD, S, LD, wave, m, g, acc);
-    });
-  }
-}
-
-// The folded transforms (even N, H = N/2, HP = H padded to 16).  A unit is a block of 16
-// rows r of both halves and one dof tile; acc[u][0..1] hold the x / p columns of the odd
-// half, acc[u][2..3] those of the even half.
-//   forward:  odd r  (mode 2r+1) = sum_k Todd[r][k]  (x_k + x_{N-1-k})
-//             even r (mode 2r+2) = sum_k Teven[r][k] (x_k - x_{N-1-k})
-//             the sum and difference are formed from the two S rows as they are loaded;
-//   backward: P_l = sum_r Todd[r][l] y_{2r},  Q_l = sum_r Teven[r][l] y_{2r+1}   (S rows = modes)
-//             x_l = P_l + Q_l, x_{N-1-l} = P_l - Q_l                       (store_fold)
-// The loop is the ping-pong of gemm_T over HP/4 K-chunks: half of gemm_T's MFMAs.
-template <int DT, int UPW, int W, bool BWD, int NU>
-__device__ __forceinline__ void gemm_fold_n(const double* __restrict__ Tf, int N, const double* S,
-                                            int LD, int wave, int m, int g, d4 (&acc)[UPW][4]) {
-  const int HP = ((N >> 1) + 15) / 16 * 16;
-  const size_t Q = (size_t)HP * HP;
-  const double* To = Tf + (BWD ? 2 * Q : 0);
-  const double* Te = To + Q;
-#pragma unroll
-  for (int u = 0; u < UPW; ++u)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc[u][c] = d4{0.0, 0.0, 0.0, 0.0};
-  if constexpr (NU > 0) {
-    const int nk = HP >> 2;  // a multiple of 4
-    const int units = (HP >> 4) * DT;
-    int toff[NU], soff[NU];
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      const int unit = min(wave + u * W, units - 1);
-      const int rp = unit / DT, dtile = unit - rp * DT;
-      toff[u] = g * HP + rp * 16 + m;
-      soff[u] = dtile * 16 + m;
-    }
-    // T fragments (global, long latency) in ping-pong; S fragments (LDS) loaded just before
-    // their MFMAs, which keeps the operand registers at 8 per unit
-    double ao[2][NU], ae[2][NU];
-    auto loadA = [&](int set, int kc) __attribute__((always_inline)) {
-      const size_t tb = (size_t)(4 * kc) * HP;  // wave-uniform chunk base
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        ao[set][u] = To[tb + toff[u]];
-        ae[set][u] = Te[tb + toff[u]];
-      }
-    };
-    auto mma = [&](int set, int kc) __attribute__((always_inline)) {
-      const int k = 4 * kc + g;
-      const int ro = BWD ? 2 * k : k;                       // odd-half operand row
-      const int re = BWD ? 2 * k + 1 : max(N - 1 - k, 0);   // even-half operand row
-      double xo[NU], po[NU], xe[NU], pe[NU];
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        xo[u] = S[ro * LD + soff[u]];
-        po[u] = S[ro * LD + DT * 16 + soff[u]];
-        xe[u] = S[re * LD + soff[u]];
-        pe[u] = S[re * LD + DT * 16 + soff[u]];
-        if constexpr (!BWD) {
-          // the fold in registers: rows k and N-1-k -> their sum (odd half) and difference
-          // (even half).  Rows k >= H meet zero columns of the tables.
-          const double sx = xo[u] + xe[u], dx = xo[u] - xe[u];
-          const double sp = po[u] + pe[u], dp = po[u] - pe[u];
-          xo[u] = sx;
-          xe[u] = dx;
-          po[u] = sp;
-          pe[u] = dp;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        acc[u][0] = mfma_f64(ao[set][u], xo[u], acc[u][0]);
-        acc[u][1] = mfma_f64(ao[set][u], po[u], acc[u][1]);
-        acc[u][2] = mfma_f64(ae[set][u], xe[u], acc[u][2]);
-        acc[u][3] = mfma_f64(ae[set][u], pe[u], acc[u][3]);
-      }
-    };
-    loadA(0, 0);
-    for (int kc = 0; kc < nk; kc += 2) {
-      loadA(1, kc + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      mma(0, kc);
-      __builtin_amdgcn_sched_barrier(0);
-      loadA(0, kc + 2 < nk ? kc + 2 : kc + 1);  // the last prefetch re-reads a valid chunk
-      __builtin_amdgcn_sched_barrier(0);
-      mma(1, kc + 1);
-      __builtin_amdgcn_sched_barrier(0);
+    if (i0 >= 0 && i0 < N) L.Z[z_at<DC>(HP, i0 & 1, i0 >> 1, row)] = z0;
+    if (i1 < N) L.Z[z_at<DC>(HP, i1 & 1, i1 >> 1, row)] = z1;
+    row += drow;
+    q += dq;
+    if (row >= R) {
+      row -= R;
+      ++q;
     }
   }
 }
 
-template <int DT, int UPW, int W, bool BWD>
-__device__ __forceinline__ void gemm_fold(const double* __restrict__ Tf, int N, const double* S,
-                                          int LD, int wave, int m, int g, d4 (&acc)[UPW][4]) {
-  if constexpr (UPW == 1) {
-    gemm_fold_n<DT, 1, W, BWD, 1>(Tf, N, S, LD, wave, m, g, acc);  // as in gemm_T
-  } else {
-    const int HP = ((N >> 1) + 15) / 16 * 16;
-    const int units = (HP >> 4) * DT;
-    with_units<UPW>(active_units<UPW, W>(wave, units), [&](auto NU) __attribute__((always_inline)) {
-      gemm_fold_n<DT, UPW, W, BWD, decltype(NU)::value>(Tf, N, S, LD, wave, m, g, acc);
-    });
-  }
-}
-
-// S <- the backward folded accumulators: x_l = P + Q, x_{N-1-l} = P - Q (x and/or p).
-template <int DT, int UPW, int W>
-__device__ __forceinline__ void store_fold(double* S, int LD, int N, int wave, int m, int g,
-                                           const d4 (&acc)[UPW][4], bool store_x) {
-  const int H = N >> 1, HP = (H + 15) / 16 * 16;
-  const int units = (HP >> 4) * DT;
-  constexpr int DC = DT * 16;
+// r = T (lambda z) for this wave's beads.  sin(i (N+1-l) pi/(N+1)) = -(-1)^i sin(i l pi/(N+1))
+// splits the product into its odd modes P and even modes Q, half the multiply-adds: the lower
+// half's beads get P + Q, the upper half's P - Q.  The two waves of a tile share that work:
+// each makes P and Q of half the dof tiles (of one dof tile, the lower wave P and the upper
+// Q) and hands over the other wave's part through LDS.  The tables carry the factor lambda_i;
+// their fragments (L2) are loaded one K-chunk ahead of the MFMAs.
+template <int DT>
+__device__ __forceinline__ void noise_gemm(KernArgs& A, const Lane& L, double (&r)[DT][4]) {
+  constexpr int DC = 16 * DT, ND = DT == 1 ? 1 : DT / 2, NQ = DT == 1 ? 1 : 2;
+  const int HP = 16 * L.nt, lane = L.g * 16 + L.m;
+  const double* __restrict__ T0 = A.Tf + (DT == 1 ? (size_t)L.h * HP * HP : 0);
+  const int toff = L.g * HP + L.tile * 16 + L.m;
+  // operand address of the first K-chunk: z_at's column swizzle is the same in every chunk
+  const double* z0 = L.Z + z_at<DC>(HP, DT == 1 ? L.h : 0, L.g, (DT == 1 ? 0 : 16 * ND * L.h) + L.m);
+  d4 acc[ND][NQ];
 #pragma unroll
-  for (int u = 0; u < UPW; ++u) {
-    const int unit = wave + u * W;
-    if (unit < units) {
-      const int rp = unit / DT, dtile = unit - rp * DT;
-      const int col = dtile * 16 + m;
+  for (int e = 0; e < ND; ++e)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int l = rp * 16 + g + 4 * j;
-        if (l < H) {
-          if (store_x) {
-            S[l * LD + col] = acc[u][0][j] + acc[u][2][j];
-            S[(N - 1 - l) * LD + col] = acc[u][0][j] - acc[u][2][j];
-          }
-          S[l * LD + DC + col] = acc[u][1][j] + acc[u][3][j];
-          S[(N - 1 - l) * LD + DC + col] = acc[u][1][j] - acc[u][3][j];
-        }
+    for (int q = 0; q < NQ; ++q) acc[e][q] = d4{0.0, 0.0, 0.0, 0.0};
+  const int nk = HP >> 2;  // a multiple of 4
+  double b[2][NQ];
+  auto load = [&](int set, int kc) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) b[set][q] = (T0 + (size_t)(q * HP + 4 * kc) * HP)[toff];
+  };
+  auto mma = [&](int set, int kc) __attribute__((always_inline)) {
+    const double* z = z0 + 4 * kc * DC;
+#pragma unroll
+    for (int e = 0; e < ND; ++e)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        // dof tile 16 e further: bit 4 of the column flips with e when the swizzle is on
+        const double* ze = z + q * HP * DC;
+        const double a = ND == 1 ? ze[0] : ze[(L.g & 1) ? (e ^ 1) * 16 - 16 : e * 16];
+        acc[e][q] = mfma_f64(a, b[set][q], acc[e][q]);
       }
-    }
+  };
+  load(0, 0);
+  for (int kc = 0; kc < nk; kc += 2) {
+    load(1, kc + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(0, kc);
+    __builtin_amdgcn_sched_barrier(0);
+    load(0, kc + 2 < nk ? kc + 2 : kc + 1);  // the last prefetch re-reads a valid chunk
+    __builtin_amdgcn_sched_barrier(0);
+    mma(1, kc + 1);
+    __builtin_amdgcn_sched_barrier(0);
   }
-}
-
-// S <- acc (x and/or p columns)
-template <int DT, int UPW, int W>
-__device__ __forceinline__ void store_acc(double* S, int LD, int NPAD, int wave, int m, int g,
-                                          const d4 (&acc)[UPW][4], bool store_x) {
-  const int units = (NPAD >> 5) * DT;
+  double* out = L.Own + lane;
+  const double* in = L.Own + (L.h ? -L.own : L.own) + lane;  // the tile's other wave
 #pragma unroll
-  for (int u = 0; u < UPW; ++u) {
-    const int unit = wave + u * W;
-    if (unit < units) {
-      const int rp = unit / DT, dtile = unit - rp * DT;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int i = rp * 32 + h * 16 + g + 4 * j;
-          if (store_x) S[i * LD + dtile * 16 + m] = acc[u][2 * h][j];
-          S[i * LD + DT * 16 + dtile * 16 + m] = acc[u][2 * h + 1][j];
-        }
-    }
-  }
-}
-
-// The normals of one unit's two row halves: z[h][j] for lane group g at modes
-// i = 32 rp + 16 h + g + 4 j of one dof (folded units: i = 2 (16 rp + g + 4 j) + h), draw
-// index base + i.  When N is even the draws of
-// modes (i, i+1) share one Philox block, so lane groups (2k, 2k+1) split the blocks of
-// their pairs and swap halves with the partner lane 16 away: half the Philox/Box-Muller
-// work.  The four blocks of a lane are independent chains, made side by side.
-template <bool FOLD>
-__device__ __forceinline__ void noise8(const BatchArgs& A, int64_t noff, uint64_t strm,
-                                       int64_t base, int rp, int g, bool real_dof,
-                                       double (&z)[2][4]) {
-  const int N = A.N;
-  if (A.noise || (N & 1)) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int i = FOLD ? 2 * (rp * 16 + g + 4 * j) + h : rp * 32 + 16 * h + g + 4 * j;
-        z[h][j] = (real_dof && i < N) ? batch_draw(A, noff, strm, base + i) : 0.0;
-      }
-    return;
-  }
-  // base is even (the cursor and dof*N are multiples of N): pair (i even, i+1) = one block
-  if constexpr (FOLD) {
-    // folded units hold modes 2r and 2r+1 in the same lane: one block gives both
+  for (int e = 0; e < ND; ++e)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int i0 = 2 * (rp * 16 + g + 4 * j);
-      double z0 = 0.0, z1 = 0.0;
-      if (real_dof && i0 < N) philox_normal2(A.seed, strm, (uint64_t)(base + i0) >> 1, z0, z1);
-      z[0][j] = z0;
-      z[1][j] = z1;
+      const double P = acc[e][0][j], Q = acc[e][NQ - 1][j];
+      out[(e * 4 + j) * 64] = DT == 1 ? P : L.h ? P + Q : P - Q;
+      r[e][j] = DT == 1 ? P : L.h ? P - Q : P + Q;
     }
-    return;
-  }
-  const int ibase = rp * 32;
-  const bool odd = g & 1;
-  double mine[2][2], other[2][2];
+  __syncthreads();
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int e = 0; e < ND; ++e)
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      // even lane: j = 0, 1; odd lane: j = 2, 3
-      const int ie = ibase + 16 * h + (g & ~1) + 4 * (odd ? 2 + t : t);
-      double z0 = 0.0, z1 = 0.0;
-      if (real_dof && ie < N) philox_normal2(A.seed, strm, (uint64_t)(base + ie) >> 1, z0, z1);
-      mine[h][t] = odd ? z1 : z0;
-      other[h][t] = odd ? z0 : z1;
-    }
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const double r0 = __shfl_xor(other[h][0], 16), r1 = __shfl_xor(other[h][1], 16);
-    if (!odd) {
-      z[h][0] = mine[h][0]; z[h][1] = mine[h][1]; z[h][2] = r0; z[h][3] = r1;
-    } else {
-      z[h][0] = r0; z[h][1] = r1; z[h][2] = mine[h][0]; z[h][3] = mine[h][1];
-    }
-  }
-}
-
-// Normal-mode phase on the forward-transform accumulators: q = acc_x - beadvec,
-// A(dt/2) [O A(dt/2)] per element, then S <- [q + beadvec | p~].
-template <int DT, int UPW, int W, bool FOLD>
-__device__ __forceinline__ void nm_phase(const BatchArgs& A, double* S, const double* MT,
-                                         int wave, int m, int g, d4 (&acc)[UPW][4],
-                                         const double* __restrict__ pa, int64_t noff,
-                                         uint64_t strm, int64_t cur, bool with_o, bool& nan) {
-  const int N = A.N, D = A.D, LD = A.LD;
-  const int units = (A.NPAD >> 5) * DT;
-  const double c = A.c, sq = A.sq, sp = A.sp;
-  static_for<UPW>([&](auto U) __attribute__((always_inline)) {
-    constexpr int u = decltype(U)::value;
-    const int unit = wave + u * W;
-    if (unit < units) {
-      const int rp = unit / DT, dtile = unit - rp * DT;
-      const int dof = dtile * 16 + m;
-      const bool dreal = dof < D;
-      const double mc = A.massd[dof], imc = 1.0 / mc, sqm = sqrt(mc);
-      const double av = pa[dof], bvv = pa[DT * 16 + dof];
-      double zz[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
-      if (with_o) noise8<FOLD>(A, noff, strm, cur + (int64_t)dof * N, rp, g, dreal, zz);
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const double* z = zz[h];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int i = FOLD ? 2 * (rp * 16 + g + 4 * j) + h : rp * 32 + h * 16 + g + 4 * j;
-          const double* md = MT + i * kMODE;
-          const double wm = mc * md[MD_MU], iwm = imc * md[MD_IMU];
-          const double bv = av * md[MD_U] + bvv * md[MD_W];
-          double q = acc[u][2 * h][j] - bv;
-          double pt = acc[u][2 * h + 1][j];
-          double q1 = c * q + (sq * iwm) * pt;
-          double p1 = -(sp * wm) * q + c * pt;
-          nan |= (p1 != p1);
-          if (with_o) {
-            const double p2 = A.c1sq * p1 + (sqm * md[MD_LAM] * A.kappa) * z[j];
-            q = c * q1 + (sq * iwm) * p2;
-            pt = -(sp * wm) * q1 + c * p2;
-            nan |= (pt != pt);
-          } else {
-            q = q1;
-            pt = p1;
-          }
-          S[i * LD + dof] = q + bv;
-          S[i * LD + DT * 16 + dof] = pt;
-        }
+    for (int j = 0; j < 4; ++j) {
+      const double own = r[e][j], got = in[(e * 4 + j) * 64];
+      if constexpr (DT == 1) {
+        r[e][j] = L.h ? got - own : own + got;
+      } else {
+        r[e][j] = L.h ? got : own;
+        r[ND + e][j] = L.h ? own : got;
       }
     }
+}
+
+// The wave's edge beads, for the neighbours of the adjacent tiles: slot tile + 1 holds
+// [lower m = 0 | lower m = 15 | upper m = 0 | upper m = 15]; slot 0 holds the fixed ends at
+// the places of m = 15, slot nt + 1 each half's last bead, where the halves meet.
+template <int DT>
+__device__ __forceinline__ void publish_edges(const Lane& L, const double (&x)[DT][4]) {
+  constexpr int DC = 16 * DT;
+  auto put = [&](int slot) __attribute__((always_inline)) {
+    double* e = L.E + slot * DC + L.g;
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) e[16 * d + 4 * j] = x[d][j];
+  };
+  if (L.m == 0 || L.m == 15) put((L.tile + 1) * 4 + 2 * L.h + (L.m == 15));
+  if (L.last) put((L.nt + 1) * 4 + L.h);
+}
+
+// First part of the linear step (Linear, rp_batch.h): p', and x' without the other tiles'
+// share of K^-1; the tile's sums go to Tot.  K^-1 in closed form, with k = 1..N the bead and
+// G = N + 1:
+//   (K^-1 u)_k = betan^2 / G [ (G - k) sum_{j<=k} j u_j + k sum_{j>k} (G - j) u_j ].
+// With w = l + 1 the lower half's bead is k = w and the upper half's k = G - w, so each half
+// takes a prefix sum of w u and a suffix sum of (G - w) u over its own beads, and the other
+// half enters as one number, the total of its w u.  Every term enters with its own sign only:
+// no difference of large partial sums.
+template <int DT, bool NOISE>
+__device__ __forceinline__ void linear_local(KernArgs& A, const Lane& L,
+                                             const __attribute__((address_space(4))) Linear& C,
+                                             double (&x)[DT][4], double (&p)[DT][4], const double (&r)[DT][4]) {
+  constexpr int DC = 16 * DT;
+  const double w = (double)(L.l + 1), v = (double)(A.N - L.l), wf = w * A.iG;
+  const double* ea = L.E + (2 * L.h + 1) * DC + L.g;  // this half's fixed end
+  const double* eb = L.E + (3 - 2 * L.h) * DC + L.g;  // the other one
+  const double* meet = L.E + ((L.nt + 1) * 4 + (L.h ^ 1)) * DC + L.g;
+  // the edge slot a lane's row move has no source for: the tile before (m = 0) or after
+  const double* en = L.E + ((L.m == 0 ? L.tile * 4 + 1 : (L.tile + 2) * 4) + 2 * L.h) * DC + L.g;
+  const double* Row = L.Row + L.g;
+  const bool edge = L.m == 0 || L.m == 15;
+  double* tot = L.Tot + (L.tile * 2 + L.h) * DC * 2 + 2 * L.g + (L.m ? 0 : 1);
+  static_for<DT>([&](auto Dx) __attribute__((always_inline)) {
+    constexpr int d = decltype(Dx)::value;
+    static_for<4>([&](auto J) __attribute__((always_inline)) {
+      constexpr int j = decltype(J)::value, row = 16 * d + 4 * j;
+      const double xi = x[d][j], pi = p[d][j];
+      double ri = 0.0;
+      if constexpr (NOISE) ri = Row[RW_SK * DC + row] * r[d][j];
+      // neighbours l - 1 and l + 1; the halves meet at their last beads
+      const double e = en[row];
+      const double prev = row_mov<kShr + 1>(e, xi);
+      double next = row_mov<kShl + 1>(e, xi);
+      next = L.last ? meet[row] : next;
+      // K^-1 of the tile's own beads
+      const double u = L.on ? (NOISE ? fma(C.cu, pi, ri) : pi) : 0.0;
+      const double f = v * u;
+      const double a = row_prefix(w * u), b = row_suffix(f);
+      if (edge) tot[2 * row] = L.m ? a : b;  // prefix total in lane 15, suffix total in lane 0
+      const double s = v * a + w * (b - f);
+      const double xa = ea[row], xeq = xa + (eb[row] - xa) * wf;
+      double xn = xeq + C.cy * (xi - xeq) + (C.gx * Row[RW_IM * DC + row]) * s;
+      double pn = C.cp * pi - (C.ck * Row[RW_M * DC + row]) * ((xi - prev) + (xi - next));
+      if constexpr (NOISE) pn += C.cr * ri;
+      // computed here: sunk past the next element's branches they would hold its inputs
+      asm volatile("" : "+v"(xn), "+v"(pn));
+      x[d][j] = xn;
+      p[d][j] = pn;
+      if constexpr (j & 1) __builtin_amdgcn_sched_barrier(0);  // two elements at a time: bounded registers
+    });
   });
 }
 
-// B for the water cluster with one (bead, atom) per thread: the atom's gradient from its own
-// molecule's Morse bonds and HOH bend and from every atom of the other molecules (charges,
-// and Lennard-Jones between oxygens), the positions read from LDS.  Each pair term is made
-// by both of its atoms (twice the pair arithmetic of one evaluation per bead), and a thread
-// holds one atom's three components instead of a bead's 3 x 18: nothing spills.  The terms
-// are those of water_eval (rp_pes.h).
-template <int NMOL, int DT, int W>
-__device__ __forceinline__ void water_kick_atoms(const BatchArgs& A, double* S, int tid, bool& nan) {
-  const double* dp = A.pes.dp;
-  const double De = dp[0], al = dp[1], re = dp[2], kb = dp[3], th0 = dp[4], eps = dp[5],
-               sig = dp[6], qH = dp[7];
-  constexpr int NA = 3 * NMOL;
-  const int N = A.N, LD = A.LD;
-  for (int it = tid; it < N * NA; it += W * 64) {
-    const int b = it / NA, i = it - b * NA;
-    const int m = i / 3, ai = i - 3 * m;  // molecule, and 0 = O, 1 / 2 = H
-    const double* xb = S + b * LD;
-    const double* xm = xb + 9 * m;
-    // own molecule: bonds u_h = H_h - O and the bend
-    double u[2][3], r[2], dEdr[2];
+// Second part: the other tiles' share of K^-1.  Each wave sums the tiles' totals for its own
+// place: prefix totals of the tiles before it, suffix totals of those after it plus the other
+// half's total, one (row, kind) per lane, through a wave-private LDS area.
+template <int DT>
+__device__ __forceinline__ void linear_carry(KernArgs& A, const Lane& L,
+                                             const __attribute__((address_space(4))) Linear& C,
+                                             double (&x)[DT][4]) {
+  constexpr int DC = 16 * DT;
+  const int lane = L.g * 16 + L.m;
+  double* car = L.Own;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      double rr = 0.0;
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        u[h][d] = xm[3 * (h + 1) + d] - xm[d];
-        rr += u[h][d] * u[h][d];
+  for (int q = 0; q < (DT + 1) / 2; ++q) {
+    const int c = lane + 64 * q;  // of 2 DC columns (row, kind)
+    if (c < 2 * DC) {
+      double s = 0.0;
+      for (int t = 0; t < L.nt; ++t) {
+        const double* T = L.Tot + (2 * t + L.h) * DC * 2 + c;
+        const double* To = L.Tot + (2 * t + (L.h ^ 1)) * DC * 2 + c;
+        if (c & 1) {
+          s += (t > L.tile ? T[0] : 0.0) + To[-1];  // suffix, and the other half's prefix total
+        } else if (t < L.tile) {
+          s += T[0];
+        }
       }
-      r[h] = sqrt(rr);
-      const double e = exp(-al * (r[h] - re)), om = 1.0 - e;
-      dEdr[h] = (2.0 * De * al) * om * e / r[h];
-    }
-    const double dot = u[0][0] * u[1][0] + u[0][1] * u[1][1] + u[0][2] * u[1][2];
-    const double ir01 = 1.0 / (r[0] * r[1]);
-    const double cs = dot * ir01;
-    const double dth = acos(cs) - th0;
-    const double dEdc = -kb * dth / sqrt(1.0 - cs * cs);
-    const double i00 = cs / (r[0] * r[0]), i11 = cs / (r[1] * r[1]);
-    double g[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const double t0 = dEdr[0] * u[0][d], t1 = dEdr[1] * u[1][d];
-      const double d0 = dEdc * (u[1][d] * ir01 - i00 * u[0][d]);
-      const double d1 = dEdc * (u[0][d] * ir01 - i11 * u[1][d]);
-      g[d] = ai == 0 ? -(t0 + t1) - (d0 + d1) : (ai == 1 ? t0 + d0 : t1 + d1);
-    }
-    // the other molecules
-    const double si = ai == 0 ? -2.0 : 1.0;
-    const double xi0 = xb[3 * i], xi1 = xb[3 * i + 1], xi2 = xb[3 * i + 2];
-    for (int j = 0; j < NA; ++j) {
-      if (j / 3 == m) continue;
-      const double dx0 = xi0 - xb[3 * j], dx1 = xi1 - xb[3 * j + 1], dx2 = xi2 - xb[3 * j + 2];
-      const double rr = dx0 * dx0 + dx1 * dx1 + dx2 * dx2;
-      const double ir2 = 1.0 / rr, ir = sqrt(ir2);
-      const double sij = si * ((j % 3 == 0) ? -2.0 : 1.0);
-      double dEr = (-qH * qH * sij) * ir2 * ir;  // (dE/dr) / r
-      if (ai == 0 && j % 3 == 0) {
-        const double s2 = (sig * sig) * ir2, s6 = s2 * s2 * s2;
-        dEr += (4.0 * eps) * (-12.0 * s6 * s6 + 6.0 * s6) * ir2;
-      }
-      g[0] += dEr * dx0;
-      g[1] += dEr * dx1;
-      g[2] += dEr * dx2;
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      double* pp = S + b * LD + DT * 16 + 3 * i + d;
-      const double np = *pp - g[d] * A.dt;
-      nan |= (np != np);
-      *pp = np;
+      car[c] = s;
     }
   }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const double w = (double)(L.l + 1), v = (double)(A.N - L.l);
+  const double* Row = L.Row + L.g;
+  const double* k = car + 2 * L.g;
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = 16 * d + 4 * j;
+      x[d][j] += (C.gx * Row[RW_IM * DC + row]) * (v * k[2 * row] + w * k[2 * row + 1]);
+    }
 }
 
-// B: p -= dt grad V(x) for every bead (verletmodule.f90:565-585)
-template <int KIND, int MAXD, int DT, int W>
-__device__ __forceinline__ void pes_kick(const BatchArgs& A, double* S, const double* PL, int tid,
-                                         bool& nan) {
-  static_assert(KIND != PES_EVB, "the EVB kick runs on the matrix cores (evb_kick_mfma)");
-  (void)PL;
-  if constexpr (KIND == PES_WATER) {
-    water_kick_atoms<MAXD / 9, DT, W>(A, S, tid, nan);
-    return;
-  }
-  const int N = A.N, D = A.D, LD = A.LD;
-  for (int b = tid; b < N; b += W * 64) {
-    double xs[MAXD], gs[MAXD];
-#pragma unroll
-    for (int d = 0; d < MAXD; ++d) xs[d] = (d < D) ? S[b * LD + d] : 0.0;
-    (void)eval_kind<KIND, MAXD>(A.pes, xs, gs);
-#pragma unroll
-    for (int d = 0; d < MAXD; ++d) {
-      if (d < D) {
-        double np = S[b * LD + DT * 16 + d] - gs[d] * A.dt;
-        nan |= (np != np);
-        S[b * LD + DT * 16 + d] = np;
-      }
-    }
-  }
-}
+// ---------------------------------------------------------------- the kick, p -= dt grad V
+// (verletmodule.f90:565-585)
 
 // The EVB parameter block (evb_eval_at's layout, stride M) -> the kick's LDS layout
 // (evb_kick_lds_size): vectors and matrices zero-padded to DC = 16 DT, matrix rows of
 // stride DC + 1 (the y GEMM reads a column of 16 rows per lane group: an odd stride puts
-// them in distinct banks).
-template <int M, int DT, int W>
-__device__ __forceinline__ void stage_evb_kick(const double* __restrict__ dp, double* PL, int tid) {
+// them in distinct banks).  The second matrix is the difference WtB - WtA: the wells differ by
+// a permutation of atoms, so its columns are zero at every atom the permutation leaves.
+template <int M, int DT>
+__device__ __forceinline__ void stage_evb_kick(const double* __restrict__ dp, double* PL, uint32_t moved,
+                                               int tid, int nthreads) {
   constexpr int DC = DT * 16, LW = DC + 1, NV = 2 + 4 * DC;
   const double* WA = dp + 1;
   const double* cA = WA + M * M;
@@ -494,7 +327,8 @@ __device__ __forceinline__ void stage_evb_kick(const double* __restrict__ dp, do
   const double* cB = WB + M * M;
   const double* lam = cB + M;
   const double* cub = lam + M;
-  for (int e = tid; e < evb_kick_lds_size(DC); e += W * 64) {
+  const int ld = evb_diff_stride(moved);
+  for (int e = tid; e < evb_kick_lds_size(DC, moved); e += nthreads) {
     double v = 0.0;
     if (e == 0) {
       v = dp[0];
@@ -503,204 +337,524 @@ __device__ __forceinline__ void stage_evb_kick(const double* __restrict__ dp, do
       const double* vec = k == 0 ? cA : k == 1 ? cB : k == 2 ? lam : cub;
       if (i < M) v = vec[i];
     } else if (e >= NV) {
-      const int f = e - NV, w = f / (DC * LW), r = f - w * (DC * LW);
-      const int i = r / LW, j = r - i * LW;
-      if (i < M && j < M) v = (w ? WB : WA)[i * M + j];
+      const int f = e - NV, w = f >= DC * LW, r = f - w * (DC * LW);
+      const int i = r / (w ? ld : LW), j = r - i * (w ? ld : LW);
+      if (i < M && j < M) v = w ? WB[i * M + j] - WA[i * M + j] : WA[i * M + j];
     }
     PL[e] = v;
   }
 }
 
-// B for the EVB on the matrix cores.  For a tile of 16 beads, both wells' coordinates
-// y = Wt x - cw are one GEMM (rows: 2 x 16*RT well rows; K: the dofs) and the mixed
-// gradient wa WtA^T hA + wb WtB^T hB is a second GEMM (rows: dofs; K: both wells' rows)
-// whose B operand is the first GEMM's accumulators, scaled in place: item j of row tile
-// rt holds row 16 rt + g + 4 j of bead m, exactly the operand of K-chunk 4 rt + j.
-// The per-bead well energies are reduced over the four lane groups with two xor
-// shuffles.  Tiles are dealt to waves round-robin.  The matrices come zero-padded from
-// stage_evb_kick, so padded rows give y = h = 0 and padded dofs no gradient.
-template <int M, int DT, int W>
-__device__ __forceinline__ void evb_kick_mfma(const BatchArgs& A, double* S, const double* PL,
-                                              int wave, int m, int g, bool& nan) {
-  constexpr int RT = DT;             // row tiles per well
-  constexpr int KY = 4 * RT;         // K-chunks of the y GEMM (dofs, padded to 16 RT)
-  constexpr int KG = 8 * RT;         // K-chunks of the gradient GEMM (both wells' rows)
+// The EVB on the matrix cores, 16 beads of a wave, from registers to registers.  Both wells'
+// coordinates are y_A = WtA x - cA (one GEMM whose B operand is x as the state holds it: item
+// j of dof tile d is dof 16 d + g + 4 j of bead m, the operand of K-chunk 4 d + j) and
+// y_B = y_A + cA - cB + (WtB - WtA) x, over the K-chunks in `moved` only: those with a dof that
+// the wells' permutation moves.  The mixed gradient is likewise
+// WtA^T (wa hA + wb hB) + (WtB - WtA)^T wb hB, the second product for the dof tiles with a
+// moved dof; its B operand is the first GEMMs' accumulators, scaled in place, and its result
+// has the layout of p.  With two hydrogens exchanged (dofs 0-5 of 27) that is 39 MFMAs per 16
+// beads; both wells in full take 56.  K-chunks beyond M are left out.  The per-bead well
+// energies are reduced over the four lane groups with two xor shuffles.
+template <int M, int DT>
+__device__ __forceinline__ void evb_kick(const double* PL, const Lane& L, double dt, uint32_t moved,
+                                         const double (&x)[DT][4], double (&p)[DT][4]) {
   constexpr int DC = DT * 16, LW = DC + 1;
-  const int N = A.N, D = A.D, LD = A.LD;
+  const int m = L.m, g = L.g;
   const double kappa = PL[0];
-  const double* cA = PL + 2;
+  const double* cA = PL + 2 + g;
   const double* cB = cA + DC;
   const double* lam = cB + DC;
   const double* cub = lam + DC;
-  const double* WA = cub + DC;
-  const double* WB = WA + DC * LW;
-  const int ntile = A.NPAD >> 4;
-  for (int t = wave; t < ntile; t += W) {
-    const int b0 = t * 16;
-    d4 ay[2 * RT];
+  const double* WA = PL + 2 + 4 * DC;
+  const double* WD = WA + DC * LW;
+  const int ld = evb_diff_stride(moved);
+  d4 ya[DT], yb[DT];
 #pragma unroll
-    for (int r = 0; r < 2 * RT; ++r) ay[r] = d4{0.0, 0.0, 0.0, 0.0};
+  for (int r = 0; r < DT; ++r) ya[r] = d4{0.0, 0.0, 0.0, 0.0};
+  static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
+    constexpr int kc = decltype(K)::value;
+    if constexpr (4 * kc < M) {
 #pragma unroll
-    for (int kc = 0; kc < KY; ++kc) {
-      // keep at most two K-chunks of operands in flight: the kick's registers stay below the
-      // budget of two workgroups per CU
-      if (kc % 2 == 0) __builtin_amdgcn_sched_barrier(0);
-      const int j = 4 * kc + g;
-      const double bx = S[(b0 + m) * LD + j];
+      for (int r = 0; r < DT; ++r)
+        ya[r] = mfma_f64(WA[(r * 16 + m) * LW + 4 * kc + g], x[kc / 4][kc % 4], ya[r]);
+    }
+  });
 #pragma unroll
-      for (int r = 0; r < 2 * RT; ++r) {
-        const double* Wt = r < RT ? WA : WB;
-        ay[r] = mfma_f64(Wt[((r % RT) * 16 + m) * LW + j], bx, ay[r]);
+  for (int r = 0; r < DT; ++r) yb[r] = ya[r];
+  static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
+    constexpr int kc = decltype(K)::value;
+    if constexpr (4 * kc < M) {
+      if ((moved >> kc) & 1) {  // wave-uniform
+#pragma unroll
+        for (int r = 0; r < DT; ++r)
+          yb[r] = mfma_f64(WD[(r * 16 + m) * ld + 4 * kc + g], x[kc / 4][kc % 4], yb[r]);
       }
     }
-    // h = lam y + 3 c y^2 and the well energies, per bead m
-    double va = 0.0, vb = 0.0;
+  });
+  // h = lam y + 3 c y^2 and the well energies, per bead m
+  double va = 0.0, vb = 0.0;
 #pragma unroll
-    for (int r = 0; r < 2 * RT; ++r)
+  for (int r = 0; r < DT; ++r)
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int i = (r % RT) * 16 + g + 4 * jj;
-        const double li = lam[i], ci = cub[i];
-        const double y = ay[r][jj] - (r < RT ? cA[i] : cB[i]), y2 = y * y;
-        const double v = (0.5 * li) * y2 + ci * y2 * y;
-        if (r < RT)
-          va += v;
-        else
-          vb += v;
-        ay[r][jj] = li * y + (3.0 * ci) * y2;
-      }
-    va += __shfl_xor(va, 16);
-    va += __shfl_xor(va, 32);
-    vb += __shfl_xor(vb, 16);
-    vb += __shfl_xor(vb, 32);
-    const double dl = va - vb, R = sqrt(0.25 * dl * dl + kappa * kappa), f = dl / (4.0 * R);
-    const double wa = 0.5 - f, wb = 0.5 + f;
-#pragma unroll
-    for (int r = 0; r < 2 * RT; ++r) ay[r] *= (r < RT ? wa : wb);
-    // gradient: G[dof][bead] = sum over both wells' rows i of Wt[i][dof] h_i
-    d4 ag[DT];
-#pragma unroll
-    for (int d = 0; d < DT; ++d) ag[d] = d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int kc = 0; kc < KG; ++kc) {
-      if (kc % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-      const int r = kc / 4, jj = kc % 4;
-      const int i = (r % RT) * 16 + 4 * jj + g;
-      const double* Wt = r < RT ? WA : WB;
-      const double bh = ay[r][jj];
-#pragma unroll
-      for (int d = 0; d < DT; ++d) ag[d] = mfma_f64(Wt[i * LW + d * 16 + m], bh, ag[d]);
+    for (int jj = 0; jj < 4; ++jj) {
+      if (r * 16 + 4 * jj >= M) continue;  // padded rows
+      const int i = r * 16 + 4 * jj;
+      const double li = lam[i], ci = cub[i];
+      auto well = [&](double y, double& v, double& h) __attribute__((always_inline)) {
+        const double t = ci * y;
+        v += (y * y) * fma(0.5, li, t);
+        h = y * fma(3.0, t, li);
+      };
+      double ha, hb;
+      well(ya[r][jj] - cA[i], va, ha);
+      well(yb[r][jj] - cB[i], vb, hb);
+      ya[r][jj] = ha;
+      yb[r][jj] = hb;
     }
-    const int bead = b0 + m;
+  va += __shfl_xor(va, 16);
+  va += __shfl_xor(va, 32);
+  vb += __shfl_xor(vb, 16);
+  vb += __shfl_xor(vb, 32);
+  const double dl = va - vb, R = sqrt(0.25 * dl * dl + kappa * kappa), f = dl / (4.0 * R);
+  const double wa = -dt * (0.5 - f), wb = -dt * (0.5 + f);
 #pragma unroll
-    for (int d = 0; d < DT; ++d)
+  for (int r = 0; r < DT; ++r) {
+    yb[r] *= wb;
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int dof = d * 16 + g + 4 * jj;
-        if (bead < N && dof < D) {
-          const double np = S[bead * LD + DC + dof] - ag[d][jj] * A.dt;
-          nan |= (np != np);
-          S[bead * LD + DC + dof] = np;
+    for (int jj = 0; jj < 4; ++jj) ya[r][jj] = fma(wa, ya[r][jj], yb[r][jj]);
+  }
+  d4 ag[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) ag[d] = d4{0.0, 0.0, 0.0, 0.0};
+  static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
+    constexpr int kc = decltype(K)::value;
+    if constexpr (4 * kc < M) {
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+        ag[d] = mfma_f64(WA[(4 * kc + g) * LW + d * 16 + m], ya[kc / 4][kc % 4], ag[d]);
+    }
+  });
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+    if ((moved >> (4 * d)) & 15u) {  // wave-uniform
+      static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
+        constexpr int kc = decltype(K)::value;
+        if constexpr (4 * kc < M)
+          ag[d] = mfma_f64(WD[(4 * kc + g) * ld + d * 16 + m], yb[kc / 4][kc % 4], ag[d]);
+      });
+    }
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) p[d][jj] += ag[d][jj];
+}
+
+// Elementwise potentials, one state element at a time.  COUPLED2D pairs row 2 q (x) with row
+// 2 q + 1 (y), which sits 16 lanes away.
+template <int KIND, int DT>
+__device__ __forceinline__ void simple_kick(KernArgs& A, const Lane& L,
+                                            const double (&x)[DT][4], double (&p)[DT][4]) {
+  constexpr int DC = 16 * DT;
+  const double* dp = A.pes.dp;
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const double xi = x[d][j];
+      double gr;
+      if constexpr (KIND == PES_QUARTIC) {
+        const double h = dp[0], x0 = dp[1], ix2 = 1.0 / (x0 * x0);
+        gr = (xi * xi * ix2 - 1.0) * (4.0 * h) * xi * ix2;
+      } else if constexpr (KIND == PES_HARMONIC) {
+        const int row = 16 * d + L.g + 4 * j;
+        gr = L.Row[RW_K * DC + row] * (xi - L.Row[RW_C * DC + row]);
+      } else {
+        static_assert(KIND == PES_COUPLED2D, "elementwise potentials only");
+        const double V0 = dp[0], a = dp[1], mm = dp[2], om = dp[3], c = dp[4];
+        const double ia2 = 1.0 / (a * a), mw2 = mm * om * om;
+        const double xo = __shfl_xor(xi, 16);
+        const bool isy = L.g & 1;
+        const double x0 = isy ? xo : xi, x1 = isy ? xi : xo;
+        const double s = x1 + c * x0 * x0, t = x0 * x0 * ia2 - 1.0;
+        gr = isy ? mw2 * s : (4.0 * V0) * t * x0 * ia2 + mw2 * s * (2.0 * c) * x0;
+      }
+      p[d][j] -= gr * A.dt;
+    }
+}
+
+// 1/sqrt(x), x > 0: the hardware estimate y (about 26 bits) and one third-order step on the
+// residual 1 - x y^2, taken with the product's rounding error: within an ulp, in place of a
+// division and a square root
+__device__ __forceinline__ double rsqrt_ref(double x) {
+  const double y = __builtin_amdgcn_rsq(x), t = x * y, tl = fma(x, y, -t);
+  const double e = fma(-tl, y, fma(-t, y, 1.0));
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// The water cluster for the 16 beads of a wave, positions in the wave's own part of LDS: a
+// lane takes bead m and, round by round, the atoms g, g + 4, ... for the terms with the other
+// molecules (charges, and Lennard-Jones between oxygens; each pair is made by both of its
+// atoms, but a lane holds one atom's three components: nothing spills), then the molecules
+// g, g + 4 for the Morse bonds and the HOH bend.  The gradients of a lane's atoms stay in
+// registers until the positions are done with, then replace them, so the kick needs no
+// barrier.  (A thread per (bead, atom) that made its molecule's own terms three times over,
+// between barriers: 15.9 ms per 8-step launch of 11,264 polymers of 6 molecules and 128
+// beads; this 11.4.)  The terms are those of water_eval (rp_pes.h); X: [16][DX].
+template <int NMOL, int DT>
+__device__ __forceinline__ void water_kick(KernArgs& A, const Lane& L, double* X,
+                                           const double (&x)[DT][4], double (&p)[DT][4]) {
+  constexpr int NA = 3 * NMOL, D = 3 * NA, DX = water_stride(D), NR = (NA + 3) / 4;
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  double* xb = X + L.m * DX;
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = 16 * d + 4 * j + L.g;
+      if (row < D) xb[row] = x[d][j];
+    }
+  wave_sync();
+  const double* dp = A.pes.dp;
+  double gp[NR][3];
+  if constexpr (NMOL > 1) {
+    const double eps = dp[5], sig2 = dp[6] * dp[6], q2 = dp[7] * dp[7];
+    static_for<NR>([&](auto Rr) __attribute__((always_inline)) {
+      constexpr int r = decltype(Rr)::value;
+      const int i = min(4 * r + L.g, NA - 1), mol = i / 3;
+      const bool oxy = i == 3 * mol;
+      const double x0 = xb[3 * i], x1 = xb[3 * i + 1], x2 = xb[3 * i + 2];
+      const double qo = oxy ? -4.0 * q2 : 2.0 * q2, qh = oxy ? 2.0 * q2 : -q2;  // -q_i q_O, -q_i q_H
+      double g0 = 0.0, g1 = 0.0, g2 = 0.0;
+#pragma unroll 1
+      for (int k = 1; k < NMOL; ++k) {
+        const int mj = mol + k < NMOL ? mol + k : mol + k - NMOL;
+        const double* y = xb + 9 * mj;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const double d0 = x0 - y[3 * a], d1 = x1 - y[3 * a + 1], d2 = x2 - y[3 * a + 2];
+          const double ir = rsqrt_ref(d0 * d0 + d1 * d1 + d2 * d2), ir2 = ir * ir;
+          double f = (a ? qh : qo) * ir;  // r dE/dr
+          if (a == 0) {
+            const double s2 = sig2 * ir2, s6 = s2 * s2 * s2;
+            const double lj = (24.0 * eps) * (s6 - 2.0 * s6 * s6);
+            f += oxy ? lj : 0.0;
+          }
+          f *= ir2;
+          g0 += f * d0;
+          g1 += f * d1;
+          g2 += f * d2;
         }
       }
+      gp[r][0] = g0;
+      gp[r][1] = g1;
+      gp[r][2] = g2;
+      __builtin_amdgcn_sched_barrier(0);
+    });
   }
-}
-
-// NM-space momenta of a resample / init_path (verletmodule.f90:102-109, 211-219):
-// v_i = sqrt(1/betan) z sqrt(beadmass_i), draws in (dim outer, atom inner) blocks of N.
-template <int DT, int W>
-__device__ __forceinline__ void write_resample(const BatchArgs& A, double* S, const double* MT,
-                                               int tid, int64_t noff, uint64_t strm,
-                                               int64_t cur) {
-  constexpr int DC = DT * 16;
-  const int N = A.N, NPAD = A.NPAD, D = A.D, LD = A.LD, natom = A.natom, ndim = A.ndim;
-  for (int e = tid; e < NPAD * DC; e += W * 64) {
-    const int c = e / NPAD, i = e - c * NPAD;
-    double v = 0.0;
-    if (i < N && c < D) {
-      const int atom = c / ndim, dim = c - atom * ndim;
-      const double z = batch_draw(A, noff, strm, cur + (int64_t)(dim * natom + atom) * N + i);
-      v = (A.stdev0 * z) * (sqrt(A.massd[c]) * MT[i * kMODE + MD_LAM] * A.tau);
+  constexpr int NM = (NMOL + 3) / 4;
+  double gm[NM][9];
+  const double De = dp[0], al = dp[1], re = dp[2], kb = dp[3], th0 = dp[4];
+  static_for<NM>([&](auto Rr) __attribute__((always_inline)) {
+    constexpr int r = decltype(Rr)::value;
+    const double* xm = xb + 9 * min(4 * r + L.g, NMOL - 1);
+    double u[2][3], rr[2], dEdr[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      double s = 0.0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        u[h][d] = xm[3 * (h + 1) + d] - xm[d];
+        s += u[h][d] * u[h][d];
+      }
+      rr[h] = sqrt(s);
+      const double e = exp(-al * (rr[h] - re)), om = 1.0 - e;
+      dEdr[h] = (2.0 * De * al) * om * e / rr[h];
     }
-    S[i * LD + DC + c] = v;
+    const double dot = u[0][0] * u[1][0] + u[0][1] * u[1][1] + u[0][2] * u[1][2];
+    const double ir01 = 1.0 / (rr[0] * rr[1]);
+    const double cs = dot * ir01;
+    const double dth = acos(cs) - th0;
+    const double dEdc = -kb * dth / sqrt(1.0 - cs * cs);
+    const double i00 = cs / (rr[0] * rr[0]), i11 = cs / (rr[1] * rr[1]);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const double a = dEdr[0] * u[0][d] + dEdc * (u[1][d] * ir01 - i00 * u[0][d]);
+      const double b = dEdr[1] * u[1][d] + dEdc * (u[0][d] * ir01 - i11 * u[1][d]);
+      gm[r][d] = -(a + b);
+      gm[r][3 + d] = a;
+      gm[r][6 + d] = b;
+    }
+  });
+  wave_sync();  // every lane has read the positions
+  if constexpr (NMOL > 1) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if (4 * r + L.g < NA)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) xb[3 * (4 * r + L.g) + d] = gp[r][d];
+    wave_sync();
   }
+#pragma unroll
+  for (int r = 0; r < NM; ++r)
+    if (4 * r + L.g < NMOL)
+#pragma unroll
+      for (int d = 0; d < 9; ++d) {
+        double* o = xb + 9 * (4 * r + L.g) + d;
+        *o = (NMOL > 1 ? *o : 0.0) + gm[r][d];
+      }
+  wave_sync();
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = 16 * d + 4 * j + L.g;
+      if (row < D) p[d][j] -= A.dt * xb[row];
+    }
 }
 
-// Phases of one step.  Every phase is: pre-op, sync, acc = T S, sync, post-op, sync.
-//   Langevin (time_step_pile):  [kick] T [NM: A O A] T [store]
-//   Andersen (time_step_nm):    ([resample] T [store p]) T [NM: A] T [store] [kick]
-//                               T [NM: A] T [store]
-//   re-initialisation:          [resample] T [store p, path spline -> x]
-enum : int { PH_FWD_PILE = 0, PH_FWD_A = 1, PH_BWD = 2, PH_RESAMPLE = 3, PH_REINIT = 4 };
+// ---------------------------------------------------------------- the step kernel
+enum : int { kPile = 0, kLimit, kPack, kAndersen };
 
-// One-unit 4-wave kernels (small bead counts, whose workgroups need little LDS) are held to
-// two waves per SIMD so that two polymers share a CU.
-template <int KIND, int MAXD, int DT, int UPW, int W, bool LANGEVIN, bool FOLD>
-__global__ void __launch_bounds__(W * 64, (W <= 4 && UPW == 1) ? 2 : 1)
-    batch_kernel(BatchArgs A) {
+// One workgroup holds a.groups polymer groups of 2 nt waves each; a group is one polymer, or
+// (PACK, at most 8 dofs) a.pack polymers side by side in the 16 rows of an MFMA tile.  The
+// state x, p lives in registers in the MFMA accumulator layout for all nsteps steps: item
+// (d, j) of lane (m, g) is row 16 d + g + 4 j (a dof, or PACK a polymer's dof) of bead
+// l = 16 tile + m of the wave's half.
+//
+// Langevin (time_step_pile): kick, normals -> LDS | T (lambda z) | linear step | carries.
+// Andersen (time_step_nm): [resample] A(dt/2), kick, A(dt/2).  Bars are barriers.
+//
+// MODE: kPile, kLimit (with dHdrlimit re-initialisations), kPack or kAndersen.
+//
+// FP64 MFMAs and FP64 vector instructions share one pipe (256 workgroups of 8 waves: MFMA
+// alone 2.29 ms, as many FMAs alone 2.90 ms, both on different waves 5.29 ms), so the step's
+// bound is the sum of both; the normals' integer rounds do overlap the kick's MFMAs, so half
+// of the waves take the two in the other order.
+template <int KIND, int MAXD, int DT, int MODE>
+__global__ void __launch_bounds__(DT > 2 ? 512 : 1024, DT > 2 ? 2 : 4) batch_kernel(BatchArgs) {
   extern __shared__ double S[];
-  __shared__ int s_flag;
   constexpr int DC = DT * 16;
-  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
-  (void)m;  // lane coordinates of the MFMA fragments: unused by the opaque-copy instances
-  (void)g;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
-  const int poly = A.first + blockIdx.x;
-  const int N = A.N, NPAD = A.NPAD, D = A.D, LD = A.LD;
-  double* MT = S + NPAD * LD;
-  double* PL = MT + NPAD * kMODE;  // EVB block (stage_evb_kick's layout), KIND == PES_EVB only
-  int64_t* pi = A.pi64 + (size_t)poly * kPI64;
-  double* st = A.state + pi[PI_STATE_OFF];
-  const double* pa = A.pdata + (size_t)poly * 3 * DC;
-  const uint64_t strm = A.stream[poly];
+  constexpr bool LANGEVIN = MODE != kAndersen, PACK = MODE == kPack;
+  KernArgs* const args = (KernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  const int tid = threadIdx.x;
+  // wave-uniform values, in SGPRs
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nwave = 2 * batch_tiles(args->N);
+  const int grp0 = wave / nwave, wave0 = wave - grp0 * nwave;
+  const double* PL = S;  // EVB block (stage_evb_kick's layout), KIND == PES_EVB only
+  // the lane's place, derived afresh from opaque copies in each phase of a step
+  auto place = [&](KernArgs& A) __attribute__((always_inline)) -> Lane {
+    int lane = tid & 63, grp = grp0, wv = wave0;
+    asm volatile("" : "+v"(lane));
+    asm volatile("" : "+s"(grp), "+s"(wv));
+    const int N = A.N;
+    const BatchLds B = batch_lds(N, DT, KIND == PES_EVB ? evb_kick_lds_size(DC, A.moved) : 0,
+                                 KIND == PES_WATER ? A.D : 0);
+    Lane L;
+    L.nt = batch_tiles(N);
+    L.h = wv & 1;
+    L.tile = wv >> 1;
+    L.wthreads = L.nt * 128;
+    L.wtid = wv * 64 + lane;
+    L.m = lane & 15;
+    L.g = lane >> 4;
+    L.l = L.tile * 16 + L.m;
+    L.bead = L.h ? N - 1 - L.l : L.l;
+    const int nh = L.h ? N >> 1 : (N + 1) >> 1;  // beads of this half
+    L.on = L.l < nh;
+    L.last = L.l == nh - 1;
+    double* base = S + B.shared + grp * B.group;
+    L.Z = base;
+    L.E = base + B.e;
+    L.Tot = base + B.tot;
+    L.Row = base + B.row;
+    L.own = wave_lds(DT, KIND == PES_WATER ? MAXD : 0);
+    L.Own = base + B.ex + wv * L.own;
+    return L;
+  };
+  auto refresh = [&]() __attribute__((always_inline)) -> KernArgs& {
+    KernArgs* a = args;
+    asm volatile("" : "+s"(a));
+    return *a;
+  };
+  // the group's polymers; a group past the family's last polymer repeats it without storing
+  const int npk = PACK ? args->pack : 1;
+  const int want = ((int)blockIdx.x * args->groups + grp0) * npk;
+  const bool live = want < args->count;
+  const int q0 = live ? want : args->count - 1;                // first polymer of the group
+  const int npol = PACK ? min(npk, args->count - q0) : 1;
+  const int poly = args->first + q0;
+  const int R = PACK ? npol * args->D : args->D;               // rows in use
+  const uint64_t strm = args->stream[poly];
+  int64_t* const pi = args->pi64 + (size_t)poly * kPI64;
   const int64_t noff = pi[PI_NOISE_OFF];
-  // the thermostat is a compile-time choice: each kernel carries one step sequence only
-  constexpr bool langevin = LANGEVIN;
-  int64_t cur = pi[PI_CURSOR];
-  bool nan = false;
-  // state -> LDS (zero padding); per-mode table -> LDS
-  for (int e = tid; e < NPAD * 2 * DC; e += W * 64) {
-    const int c = e / NPAD, i = e - c * NPAD;
-    const int d = c < DC ? c : c - DC;
-    double v = 0.0;
-    if (i < N && d < D) v = st[(c < DC ? 0 : (size_t)D * N) + (size_t)d * N + i];
-    S[i * LD + c] = v;
+  int64_t cur = PACK ? 0 : pi[PI_CURSOR];  // PACK: draws since the launch began
+  bool whole = !(args->N & 1);
+  for (int k = 0; k < npol; ++k) whole &= !(pi[(size_t)k * kPI64 + PI_CURSOR] & 1);
+  auto each = [&](const Lane& L, auto&& f) __attribute__((always_inline)) {
+    static_for<DT>([&](auto Dx) __attribute__((always_inline)) {
+      static_for<4>([&](auto J) __attribute__((always_inline)) {
+        constexpr int d = decltype(Dx)::value, j = decltype(J)::value;
+        f(std::integral_constant<int, d>{}, std::integral_constant<int, j>{}, 16 * d + L.g + 4 * j);
+      });
+    });
+  };
+  // x column of a row in use, in the state's global memory
+  auto state_of = [&](KernArgs& A, int row) __attribute__((always_inline)) -> double* {
+    const int pol = PACK ? row / A.D : 0, d = row - pol * A.D;
+    return A.state + A.pi64[(size_t)(poly + pol) * kPI64 + PI_STATE_OFF] + (size_t)d * A.N;
+  };
+  double x[DT][4], p[DT][4];
+  {
+    // staging: the EVB block, zeroed normals and edges, row tables; state -> registers
+    KernArgs& A = refresh();
+    const Lane L = place(A);
+    const int N = A.N, D = A.D;
+    if constexpr (KIND == PES_EVB) stage_evb_kick<MAXD, DT>(A.pes.dp, S, A.moved, tid, blockDim.x);
+    for (int e = L.wtid; e < (int)(L.Tot - L.Z); e += L.wthreads) L.Z[e] = 0.0;  // Z and E
+    __syncthreads();
+    for (int row = L.wtid; row < DC; row += L.wthreads) {
+      const int pol = PACK ? row / D : 0, d = row - pol * D;
+      const bool real = row < R;
+      const double* pa = A.pdata + (size_t)(poly + (real ? pol : 0)) * 3 * DC;
+      const double mass = real ? A.massd[d] : 1.0;
+      L.Row[RW_M * DC + row] = mass;
+      L.Row[RW_IM * DC + row] = 1.0 / mass;
+      L.Row[RW_SK * DC + row] = real ? sqrt(mass) * A.kappa : 0.0;
+      L.Row[RW_SV * DC + row] = real ? sqrt(mass) * A.stdev0 * A.tau : 0.0;
+      L.Row[RW_MDB * DC + row] = real ? mass * pa[2 * DC + d] : 0.0;
+      L.E[1 * DC + row] = real ? pa[d] : 0.0;       // fixed start a
+      L.E[3 * DC + row] = real ? pa[DC + d] : 0.0;  // fixed end b
+      if constexpr (KIND == PES_HARMONIC) {
+        L.Row[RW_K * DC + row] = real ? A.pes.dp[d] : 0.0;
+        L.Row[RW_C * DC + row] = real ? A.pes.dp[D + d] : 0.0;
+      }
+      if constexpr (PACK) {  // one entry per polymer
+        int64_t* ci = reinterpret_cast<int64_t*>(L.Row + RW_CUR * DC);
+        const int k = min(row, npol - 1);
+        ci[row] = A.pi64[(size_t)(poly + k) * kPI64 + PI_CURSOR];
+        ci[DC + row] = (int64_t)A.stream[poly + k];
+      }
+    }
+    each(L, [&](auto Dx, auto J, int row) __attribute__((always_inline)) {
+      constexpr int d = decltype(Dx)::value, j = decltype(J)::value;
+      const bool real = row < R && L.on;
+      const double* st = state_of(A, row < R ? row : 0) + (L.on ? L.bead : 0);
+      x[d][j] = real ? st[0] : 0.0;
+      p[d][j] = real ? st[(size_t)D * N] : 0.0;
+    });
   }
-  for (int e = tid; e < NPAD * kMODE; e += W * 64) MT[e] = A.modes[e];
-  if constexpr (KIND == PES_EVB) stage_evb_kick<MAXD, DT, W>(A.pes.dp, PL, tid);
-  if (tid == 0) s_flag = 0;
+  bool bad = false;
+  auto check = [&]() __attribute__((always_inline)) {  // NaN or infinity in the real beads
+    const Lane L = place(refresh());
+    each(L, [&](auto Dx, auto J, int row) __attribute__((always_inline)) {
+      constexpr int d = decltype(Dx)::value, j = decltype(J)::value;
+      bad |= L.on && row < R && (nonfinite(x[d][j]) || nonfinite(p[d][j]));
+    });
+  };
   double tisum = 0.0;
+  d4 tirow[DT];  // PACK: one running sum per row
+#pragma unroll
+  for (int d = 0; d < DT; ++d) tirow[d] = d4{0.0, 0.0, 0.0, 0.0};
   int64_t ticnt = 0, nre = 0;
   int64_t acount = 0, rkick = 0, kcur = 0;
-  if (!langevin) {
+  if constexpr (!LANGEVIN) {
     acount = pi[PI_ACOUNT];
     rkick = pi[PI_RKICK];
     kcur = pi[PI_KCURSOR];
   }
-  const int64_t koff = pi[PI_KICK_OFF];
-  const int64_t need = (int64_t)N * D;  // draws per O-step / resample / re-initialisation
+  const bool lead = wave0 == 1;  // the wave that holds bead N (upper half, l = 0): it keeps the TI sums
+  const int64_t need = (int64_t)args->N * args->D;  // draws per O-step / resample / re-init
+
+  auto kick = [&]() __attribute__((always_inline)) {
+    KernArgs& A = refresh();
+    const Lane L = place(A);
+    if constexpr (KIND == PES_EVB) {
+      evb_kick<MAXD, DT>(PL, L, A.dt, A.moved, x, p);
+    } else if constexpr (KIND == PES_WATER) {
+      water_kick<MAXD / 9, DT>(A, L, L.Own, x, p);
+    } else {
+      simple_kick<KIND, DT>(A, L, x, p);
+    }
+  };
+  auto noise = [&](bool resample) __attribute__((always_inline)) {
+    KernArgs& A = refresh();
+    make_noise<DC, PACK>(A, place(A), R, cur, strm, noff, whole, resample);
+  };
+  // p = sqrt(1/betan) z sqrt(beadmass) in normal modes, transformed back (:102-115, 211-228)
+  auto resample_p = [&]() __attribute__((always_inline)) {
+    noise(true);
+    KernArgs& A = refresh();
+    const Lane L = place(A);
+    __syncthreads();
+    double r[DT][4];
+    noise_gemm<DT>(A, L, r);
+    each(L, [&](auto Dx, auto J, int row) __attribute__((always_inline)) {
+      constexpr int d = decltype(Dx)::value, j = decltype(J)::value;
+      p[d][j] = L.Row[RW_SV * DC + row] * r[d][j];
+    });
+    cur += need;
+  };
+  // the linear step: A(dt/2) O A(dt/2) with the normals in Z (AOA), or A(dt/2) alone
+  auto linear = [&](auto AOA) __attribute__((always_inline)) {
+    constexpr bool aoa = decltype(AOA)::value;
+    {
+      const Lane L = place(refresh());
+      publish_edges<DT>(L, x);
+      __syncthreads();
+    }
+    double r[DT][4];
+    if constexpr (aoa) {
+      KernArgs& A = refresh();
+      noise_gemm<DT>(A, place(A), r);
+    }
+    {
+      KernArgs& A = refresh();
+      linear_local<DT, aoa>(A, place(A), aoa ? A.aoa : A.rot, x, p, r);
+      __syncthreads();
+    }
+    KernArgs& A = refresh();
+    linear_carry<DT>(A, place(A), aoa ? A.aoa : A.rot, x);
+  };
+
   __syncthreads();
   bool stop = false;
-  const int64_t step0 = A.step0p ? *A.step0p : A.step0;
-  for (int s = 0; s < A.nsteps; ++s) {
+  const int64_t step0 = args->step0p ? *args->step0p : args->step0;
+#pragma unroll 1
+  for (int s = 0; s < args->nsteps; ++s) {
     const int64_t ii = step0 + s + 1;  // the reference's step counter
-    // the step's phase list, 4 bits per phase in one register (an indexed array would live
-    // in scratch memory): at most 6 phases
-    uint32_t ph = 0;
-    int nph = 0;
-    auto push = [&](int p) __attribute__((always_inline)) { ph |= (uint32_t)p << (4 * nph++); };
-    bool resample = false;
-    if (langevin) {
-      if (A.noise && cur + need > A.noise_cap) { stop = true; break; }
-      push(PH_FWD_PILE);
-      push(PH_BWD);
+    if constexpr (LANGEVIN) {
+      KernArgs& A = refresh();
+      if (A.noise && cur + need > A.noise_cap) {
+        stop = true;
+        break;
+      }
+#pragma unroll 1
+      for (int k = 0; k < 2; ++k) {
+        if ((k ^ (wave >> 2)) & 1)
+          noise(false);
+        else
+          kick();
+      }
+      linear(std::true_type{});
+      cur += need;
     } else {
       // propagate_pimd_nm (verletmodule.f90:202-234): Poisson-timed resample first
+      KernArgs& A = refresh();
+      auto interval = [&]() -> int64_t {
+        const int64_t k = kcur++;
+        return A.kicks ? A.kicks[pi[PI_KICK_OFF] + k]
+                       : philox_poisson(A.seed, strm, k, (double)A.noutput);
+      };
       if (rkick < 0) {
-        if (A.kicks && kcur >= A.kick_cap) { stop = true; break; }
-        rkick = A.kicks ? A.kicks[koff + kcur]
-                        : philox_poisson(A.seed, strm, kcur, (double)A.noutput);
-        ++kcur;
+        if (A.kicks && kcur >= A.kick_cap) {
+          stop = true;
+          break;
+        }
+        rkick = interval();
       }
       acount = acount + 1;
       if (acount >= rkick) {
@@ -708,128 +862,113 @@ __global__ void __launch_bounds__(W * 64, (W <= 4 && UPW == 1) ? 2 : 1)
           stop = true;
           break;
         }
-        resample = true;
-        push(PH_RESAMPLE);
+        resample_p();
+        rkick = interval();
+        acount = 0;
       }
-      push(PH_FWD_A);
-      push(PH_BWD);
-      push(PH_FWD_A);
-      push(PH_BWD);
+      linear(std::false_type{});
+      kick();
+      linear(std::false_type{});
     }
-    int nbwd = 0;
-    bool ti_done = false;
-#pragma unroll 1
-    for (int k = 0; k < nph; ++k) {
-      const int p = (int)((ph >> (4 * k)) & 15u);
-      // With two or more units per wave, the lane indices are re-derived from an opaque
-      // copy in every phase: the per-lane LDS addresses are then recomputed where they are
-      // used instead of being hoisted out of the step loop and spilled (measured: 16 % less
-      // time per launch at N = 256, and under 256 VGPRs for two workgroups per CU at N = 96).
-      // One-unit waves keep the hoisted addresses: the opaque copy removes their few spill
-      // slots (254 -> 237 VGPRs on the 27-dof EVB) but costs 4-5 % per launch at N = 32-128.
-      int lane_k = lane;
-      if constexpr (UPW >= 2 || !LANGEVIN) asm volatile("" : "+v"(lane_k));
-      const int m = lane_k & 15, g = lane_k >> 4, tid = wave * 64 + lane_k;
-      if (p == PH_FWD_PILE || (p == PH_FWD_A && nbwd == 1)) {
-        if constexpr (KIND == PES_EVB) {  // B(dt) on the matrix cores
-          evb_kick_mfma<MAXD, DT, W>(A, S, PL, wave, m, g, nan);
-        } else {
-          pes_kick<KIND, MAXD, DT, W>(A, S, PL, tid, nan);
-        }
-        __syncthreads();
-      } else if (p == PH_RESAMPLE || p == PH_REINIT) {
-        write_resample<DT, W>(A, S, MT, tid, noff, strm, cur);
-        __syncthreads();
-      }
-      d4 acc[UPW][4];
-      const bool fwd = p == PH_FWD_PILE || p == PH_FWD_A;
-      if constexpr (FOLD) {
-        if (fwd) {
-          gemm_fold<DT, UPW, W, false>(A.Tf, N, S, LD, wave, m, g, acc);
-        } else {
-          gemm_fold<DT, UPW, W, true>(A.Tf, N, S, LD, wave, m, g, acc);
-        }
+    // TI estimator after the step (verletmodule.f90:397-410, 236-244): sum over dofs of
+    // m (-x_N) db/dxi; bead N is the upper bead of l = 0 (the sum's order differs from the
+    // reference's only in rounding)
+    KernArgs& A = refresh();
+    if (ii > A.imin) {
+      const Lane L = place(A);
+      if constexpr (PACK) {
+        each(L, [&](auto Dx, auto J, int row) __attribute__((always_inline)) {
+          constexpr int d = decltype(Dx)::value, j = decltype(J)::value;
+          tirow[d][j] -= L.Row[RW_MDB * DC + row] * x[d][j];
+        });
+        ++ticnt;
       } else {
-        gemm_T<DT, UPW, W>(A.T, NPAD, S, LD, wave, m, g, acc);
-      }
-      __syncthreads();
-      if (p == PH_FWD_PILE || p == PH_FWD_A) {
-        nm_phase<DT, UPW, W, FOLD>(A, S, MT, wave, m, g, acc, pa, noff, strm, cur, p == PH_FWD_PILE, nan);
-        if (p == PH_FWD_PILE) cur += need;
-      } else {
-        if constexpr (FOLD)
-          store_fold<DT, UPW, W>(S, LD, N, wave, m, g, acc, p == PH_BWD);
-        else
-          store_acc<DT, UPW, W>(S, LD, NPAD, wave, m, g, acc, p == PH_BWD);
-        if (p == PH_BWD) ++nbwd;
-        if (p == PH_REINIT) {
-          // init_path positions: x_k = splint(path, (k-1) xi/(n-1)) (verletmodule.f90:40-48)
-          const double xi = A.pf64[(size_t)poly * kPF64 + PF_XI];
-          const double* lampath = A.pathd;
-          for (int e = tid; e < N * D; e += W * 64) {
-            const int cc = e / N, i = e - cc * N;
-            const double xe = (double)i * xi / (double)(N - 1);
-            S[i * LD + cc] = splint_dev(lampath, lampath + A.npath + (size_t)cc * A.npath,
-                                        lampath + A.npath * (1 + D) + (size_t)cc * A.npath,
-                                        A.npath, xe);
-          }
+        double contr = 0.0;
+        if (lead) {
+          each(L, [&](auto Dx, auto J, int row) __attribute__((always_inline)) {
+            constexpr int d = decltype(Dx)::value, j = decltype(J)::value;
+            contr -= L.Row[RW_MDB * DC + row] * x[d][j];
+          });
+          contr += __shfl_xor(contr, 16);
+          contr += __shfl_xor(contr, 32);
         }
-        if (p == PH_RESAMPLE || p == PH_REINIT) cur += need;
-      }
-      __syncthreads();
-      // TI estimator after the step (verletmodule.f90:397-410, 236-244)
-      if (k == nph - 1 && !ti_done && ii > A.imin) {
-        ti_done = true;
-        if (wave == 0) {
-          // sum over dofs of m (-x_N) db/dxi: one dof per lane, then an xor-shuffle reduction
-          // (the reference's dim-outer order differs only in rounding)
-          double contr = 0.0;
-          for (int d = lane; d < D; d += 64) contr += A.massd[d] * (-S[(N - 1) * LD + d]) * pa[2 * DC + d];
-#pragma unroll
-          for (int o = 32; o > 0; o >>= 1) contr += __shfl_xor(contr, o);
-          const bool ok = !langevin || fabs(contr) < A.limit || A.limit < 0.0;
-          if (ok) {
-            tisum = tisum + contr;
-            ++ticnt;
-          }
-          if (lane == 0) s_flag = ok ? 0 : 1;
-        }
-        if (langevin && A.limit >= 0.0) {
+        if constexpr (MODE == kLimit) {
+          // dHdrlimit: a step whose term is too large is not counted and the path is
+          // re-initialised (:398-408)
+          int* flag = reinterpret_cast<int*>(L.Row + RW_FLAG * DC);
+          if (lead && (tid & 63) == 0) *flag = fabs(contr) < A.limit ? 0 : 1;
           __syncthreads();
-          if (s_flag) {
+          if (!*flag) {
+            tisum += contr;
+            ++ticnt;
+          } else {
             if (A.noise && cur + need > A.noise_cap) {
               stop = true;
-            } else {
-              push(PH_REINIT);  // one more phase: re-initialise the path
-              ++nre;
+              break;
             }
+            ++nre;
+            check();
+            resample_p();
+            // init_path positions: x_k = splint(path, (k-1) xi/(n-1)) (:40-48)
+            const double xi = A.pf64[(size_t)poly * kPF64 + PF_XI];
+            const double* lam = A.pathd;
+            const int N = A.N, np = A.npath;
+            each(L, [&](auto Dx, auto J, int row) __attribute__((always_inline)) {
+              constexpr int d = decltype(Dx)::value, j = decltype(J)::value;
+              if (row < A.D && L.on) {
+                const double* yy = lam + np + (size_t)row * np;
+                const double* y2 = lam + np * (1 + A.D) + (size_t)row * np;
+                x[d][j] = splint_dev(lam, yy, y2, np, (double)L.bead * xi / (double)(N - 1));
+              }
+            });
           }
+          __syncthreads();
+        } else {
+          tisum += contr;
+          ++ticnt;
         }
       }
     }
-    if (stop) break;
-    if (resample) {
-      rkick = A.kicks ? A.kicks[koff + kcur] : philox_poisson(A.seed, strm, kcur, (double)A.noutput);
-      ++kcur;
-      acount = 0;
+  }
+  check();
+  if (!live) return;
+  KernArgs& A = refresh();
+  const Lane L = place(A);
+  const int N = A.N, D = A.D;
+  if (stop && L.wtid == 0) atomicOr(&A.flags[1], 1);
+  if (bad) atomicOr(&A.flags[0], 1);
+  // registers -> state
+  each(L, [&](auto Dx, auto J, int row) __attribute__((always_inline)) {
+    constexpr int d = decltype(Dx)::value, j = decltype(J)::value;
+    if (row < R && L.on) {
+      double* st = state_of(A, row) + L.bead;
+      st[0] = x[d][j];
+      st[(size_t)D * N] = p[d][j];
     }
-  }
-  if (stop && tid == 0) atomicOr(&A.flags[1], 1);
-  __syncthreads();
-  // LDS -> state
-  for (int e = tid; e < N * 2 * D; e += W * 64) {
-    const int c = e / N, i = e - c * N;
-    const int d = c < D ? c : c - D;
-    const int sc = c < D ? d : DC + d;
-    st[(c < D ? 0 : (size_t)D * N) + (size_t)d * N + i] = S[i * LD + sc];
-  }
-  if (nan) atomicOr(&A.flags[0], 1);
-  if (tid == 0) {
+  });
+  if constexpr (PACK) {
+    // each polymer's rows summed by one lane
+    if (!lead) return;
+    if (L.m == 0)
+      each(L, [&](auto Dx, auto J, int row) __attribute__((always_inline)) {
+        L.Z[row] = tirow[decltype(Dx)::value][decltype(J)::value];
+      });
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int q = tid & 63;
+    if (q < npol) {
+      double t = 0.0;
+      for (int d = 0; d < D; ++d) t += L.Z[q * D + d];
+      A.pf64[(size_t)(poly + q) * kPF64 + PF_TISUM] += t;
+      pi[(size_t)q * kPI64 + PI_TICNT] += ticnt;
+      pi[(size_t)q * kPI64 + PI_CURSOR] += cur;
+    }
+  } else if (lead && (tid & 63) == 0) {
     A.pf64[(size_t)poly * kPF64 + PF_TISUM] += tisum;
     pi[PI_TICNT] += ticnt;
     pi[PI_NREINIT] += nre;
     pi[PI_CURSOR] = cur;
-    if (!langevin) {
+    if constexpr (!LANGEVIN) {
       pi[PI_ACOUNT] = acount;
       pi[PI_RKICK] = rkick;
       pi[PI_KCURSOR] = kcur;
@@ -837,48 +976,65 @@ __global__ void __launch_bounds__(W * 64, (W <= 4 && UPW == 1) ? 2 : 1)
   }
 }
 
-template <int KIND, int MAXD, int DT, bool LANG, bool FOLD>
-int launch_batch_thermo(const BatchArgs& a, int npoly, hipStream_t s) {
-  const int units = (a.NPAD >> 5) * DT;
-  const size_t lds = batch_lds_bytes(a.NPAD, DT, KIND == PES_EVB ? evb_kick_lds_size(DT * 16) : 0);
-  auto go = [&](auto kern, int waves) -> int {
+// How a family is dealt to workgroups.  A polymer takes one wave per 16 beads of each half.
+//  * PACK (Langevin without re-initialisation, at most 8 dofs): as many polymers share the 16
+//    rows of a tile as fit, but no more than leaves a workgroup for every CU.
+//  * Groups per workgroup, for plain Langevin, where every group of a workgroup runs the same
+//    steps: the fewest that keep a CU busiest by the score below, or a.waves (set_launch) over
+//    the tiles of a half; and no more than leaves a workgroup for every CU.  Otherwise one: resamples and re-initialisations fall
+//    differently.
+template <int KIND, int MAXD, int DT>
+int launch_batch_kind(const BatchArgs& a0, int thermostat, int npoly, hipStream_t s) {
+  BatchArgs a = a0;
+  const bool lang = thermostat == RP_THERMO_LANGEVIN, plain = lang && a.limit < 0.0 && !a.noise;
+  const int nt = batch_tiles(a.N);
+  a.count = npoly;
+  a.pack = a.groups = 1;
+  constexpr bool packs =
+      DT == 1 && (KIND == PES_QUARTIC || KIND == PES_HARMONIC || KIND == PES_COUPLED2D);
+  if (packs && plain && a.D <= 8)
+    a.pack = std::max(1, std::min(16 / a.D, (npoly + a.ncu - 1) / a.ncu));
+  const BatchLds B = batch_lds(a.N, DT, KIND == PES_EVB ? evb_kick_lds_size(DT * 16, a.moved) : 0,
+                               KIND == PES_WATER ? a.D : 0);
+  const int units = (npoly + a.pack - 1) / a.pack;
+  constexpr int kWaves = DT > 2 ? 8 : 16;  // of a workgroup (launch bound)
+  auto go = [&](auto kern) -> int {
+    auto lds_of = [&](int g) { return (B.shared + (size_t)g * B.group) * sizeof(double); };
     RP_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)lds));
-    kern<<<npoly, waves * 64, lds, s>>>(a);
+                               (int)std::min(kBatchLds, lds_of(kWaves))));
+    if (plain) {
+      const int most = std::min({kWaves / (2 * nt), (units + a.ncu - 1) / a.ncu,
+                                 a.waves ? std::max(1, a.waves / nt) : kWaves});
+      double best = 0.0;
+      for (int g = 1; g <= most && lds_of(g) <= kBatchLds; ++g) {
+        int per_cu = 0;
+        const int w = 2 * nt * g;
+        RP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, w * 64, lds_of(g)));
+        // waves of a CU, less where a workgroup is alone on it (nothing fills its barriers) and
+        // where its waves do not divide over the four SIMDs.  Measured on the 27-dof EVB, ms
+        // per 8-step launch of 5632 polymers: N = 32, 2 groups (3 workgroups, 12 waves) 0.52,
+        // 7 groups (1 workgroup, 14 waves) 0.72; N = 96, 2 groups (1 workgroup, 12 waves) 1.74,
+        // 1 group (2 workgroups of 6 waves) 2.03; N = 64, 2 groups (2 workgroups, 16 waves)
+        // 1.00, 1 group (3 workgroups, 12 waves) 1.30
+        const double score = per_cu * w * (per_cu > 1 ? 1.0 : 0.74) * (w % 4 ? 0.7 : 1.0);
+        if (a.waves || score > best) {
+          a.groups = g;
+          best = score;
+        }
+      }
+    }
+    const size_t lds = lds_of(a.groups);
+    RP_REQUIRE(lds <= kBatchLds, "batch: n=%d with %d dof needs %zu bytes of LDS", a.N, a.D, lds);
+    kern<<<(units + a.groups - 1) / a.groups, nt * a.groups * 128, lds, s>>>(a);
     RP_HIP(hipGetLastError());
     return RP_OK;
   };
-  if constexpr (DT <= 2) {
-    // one unit per wave, four 2-wave workgroups per CU (at most 256 VGPRs each): small
-    // polymers whose 2 units would leave half of a 4-wave workgroup idle
-    if (a.waves == 2 && units <= 2) return go(batch_kernel<KIND, MAXD, DT, 1, 2, LANG, FOLD>, 2);
+  if (!lang) return go(batch_kernel<KIND, MAXD, DT, kAndersen>);
+  if constexpr (packs) {
+    if (a.pack > 1) return go(batch_kernel<KIND, MAXD, DT, kPack>);
   }
-  if (a.waves == 8) {  // two waves per SIMD: units spread over 8 waves, at most 2 each
-    const int upw = (units + 7) / 8;
-    if (upw <= 1) return go(batch_kernel<KIND, MAXD, DT, 1, 8, LANG, FOLD>, 8);
-    if (upw <= 2) return go(batch_kernel<KIND, MAXD, DT, 2, 8, LANG, FOLD>, 8);
-    return set_error(RP_ERR_ARG, "batch: %d MFMA units are too many for 8 waves", units);
-  }
-  const int upw = (units + 3) / 4;
-  if (upw <= 1) return go(batch_kernel<KIND, MAXD, DT, 1, 4, LANG, FOLD>, 4);
-  if (upw <= 2) return go(batch_kernel<KIND, MAXD, DT, 2, 4, LANG, FOLD>, 4);
-  if (upw <= 3) return go(batch_kernel<KIND, MAXD, DT, 3, 4, LANG, FOLD>, 4);
-  if (upw <= 4) return go(batch_kernel<KIND, MAXD, DT, 4, 4, LANG, FOLD>, 4);
-  return set_error(RP_ERR_ARG, "batch: %d MFMA units per wave is more than supported", upw);
-}
-
-// ALLOW_FOLD = false keeps a potential on the full transforms (fewer kernel instances).
-template <int KIND, int MAXD, int DT, bool ALLOW_FOLD = true>
-int launch_batch_kind(const BatchArgs& a, int thermostat, int npoly, hipStream_t s) {
-  const bool lang = thermostat == RP_THERMO_LANGEVIN;
-  if constexpr (ALLOW_FOLD) {
-    if (a.fold) {
-      if (lang) return launch_batch_thermo<KIND, MAXD, DT, true, true>(a, npoly, s);
-      return launch_batch_thermo<KIND, MAXD, DT, false, true>(a, npoly, s);
-    }
-  }
-  if (lang) return launch_batch_thermo<KIND, MAXD, DT, true, false>(a, npoly, s);
-  return launch_batch_thermo<KIND, MAXD, DT, false, false>(a, npoly, s);
+  if (a.limit >= 0.0) return go(batch_kernel<KIND, MAXD, DT, kLimit>);
+  return go(batch_kernel<KIND, MAXD, DT, kPile>);
 }
 
 }  // namespace rp
