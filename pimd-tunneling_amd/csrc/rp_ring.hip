@@ -42,11 +42,12 @@ __device__ __forceinline__ void lds_sync() {
   }
 }
 
+template <int NT = kRingThreads>
 __device__ __forceinline__ double block_sum(double v, double* red) {
   const int tid = threadIdx.x;
   red[tid] = v;
   __syncthreads();
-  for (int s = kRingThreads / 2; s > 0; s >>= 1) {
+  for (int s = NT / 2; s > 0; s >>= 1) {
     if (tid < s) red[tid] += red[tid + s];
     __syncthreads();
   }
@@ -535,13 +536,34 @@ __device__ __forceinline__ double pivot_recip(double x) {
   return fma(r, fma(-x, r, 1.0), r);
 }
 
-// One wave per chain.  Lane l owns the elements e = l + 64 q (q < P) of every D x D block, so
-// the Hessian block of the next bead is loaded into registers while the current one is
-// eliminated, and the Schur update uses the previous inverse where it sits in LDS.  The
-// Gauss-Jordan inverse runs without pivoting, double-buffered in LDS (one barrier per pair
-// of eliminations): the pivot of elimination k is the k-th pivot of the matrix's LDL^T
-// factorisation (a ratio of leading principal minors), so their logs sum to log|det| and
-// their signs give the inertia (Sylvester).
+// f(integral_constant<int, 0..N-1>) expanded at compile time (tile and item indices stay
+// constants, so the tiles stay in registers)
+template <typename F, int... I>
+__device__ __forceinline__ void static_unroll_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_unroll(F&& f) {
+  static_unroll_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+__device__ __forceinline__ double read_lane(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// A raw buffer over [p, p + bytes): its loads take the lane's byte offset in a VGPR and a
+// uniform byte offset in an SGPR, so a step's loads need no 64-bit address per lane.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const double* p, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(p), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ double buffer_ld(__amdgpu_buffer_rsrc_t b, int voff, int soff) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, voff, soff, 0));
+}
+
+#include "rp_ring_factor.h"
+
+// The factorisation for more than 32 dofs, from bead 0 to bead n-1.
 // T threads per chain.  Thread t owns the elements e = t + T q (q < P) of every D x D block,
 // so the Hessian block of the next bead is loaded into registers while the current one is
 // eliminated, and the Schur update uses the previous inverse where it sits in LDS.  The
@@ -793,24 +815,26 @@ __global__ void __launch_bounds__(kRingThreads) ring_gersh_kernel(
   }
 }
 
-// threads and per-thread element count of ring_logdet_kernel for D (D*D <= T P)
+// the factorisation kernel for D and its threads
 template <typename F>
 int with_logdet_kernel(int D, F&& f) {
-  if (D * D <= 64) return f(ring_logdet_kernel<1, 64>, 64);
-  if (D * D <= 256) return f(ring_logdet_kernel<1, 256>, 256);
-  if (D * D <= 768) return f(ring_logdet_kernel<2, 256, true, 3>, 256);  // D (D + 1) / 2 <= 512
+  if (D <= 16) return f(ring_factor_kernel<1>, 128);
+  if (D <= 32) return f(ring_factor_kernel<2>, 128);
   if (D * D <= 1536) return f(ring_logdet_kernel<4, 256, true, 6>, 256);  // D (D + 1) / 2 <= 1024
   return f(ring_logdet_kernel<7, 256, true, 13>, 256);  // D (D + 1) / 2 <= 1792
 }
+// the middle bead of its elimination
+__host__ __device__ inline int ring_middle(int D, int n) { return D <= 32 ? (n - 1) >> 1 : n - 1; }
 
-// The block solve y = H^-1 v through the stored factors S_i^-1 (the off-diagonal blocks are
-// -c I and bead 0 is coupled to no other bead), in two sweeps whose serial path never waits
-// for global memory:
-//   forward  (m = 0 .. n-1): t_m = S_m^-1 z_m, with z_0 = v_0, z_1 = v_1 and
-//                            z_{m+1} = v_{m+1} + c t_m for m >= 1;
-//   backward (i = n-2 .. 1): y_i = t_i + c S_i^-1 y_{i+1}, with y_{n-1} = t_{n-1}, y_0 = t_0.
+// The block solve y = H^-1 v through the stored factors S_i^-1 of an elimination from both
+// ends to bead h (the off-diagonal blocks are -c I and bead 0 is coupled to no other bead), in
+// two sweeps whose serial path never waits for global memory:
+//   forward:  t_i = S_i^-1 z_i toward h from both ends, z_0 = v_0, z_{n-1} = v_{n-1}, and the
+//             next bead's z = v + c t where the two are coupled; z_h takes both sides' c t;
+//   backward: y_h = t_h, y_i = t_i + c S_i^-1 y_{i +- 1} outward from h, y_0 = t_0.
+// Half of the threads take each side (HALVES = 2); from one end only, h = n-1 and HALVES = 1.
 // The running vector (z or y, D values) sits in LDS, double-buffered; what a step reads from
-// global memory (its block, and v_{m+1} or t_i) does not depend on it, so it is loaded P steps
+// global memory (its block, and v or t) does not depend on it, so it is loaded P steps
 // ahead into registers, and the per-step barrier orders LDS only, which leaves those loads in
 // flight across it.  Lanes: Q per block row (row r = tid / Q, lane q), each holding the KPL
 // columns k = q + Q j of its row; a row's sum is a DPP butterfly inside its Q lanes.  The LDS
@@ -829,35 +853,31 @@ __device__ __forceinline__ double row_sum(double s) {
   return s;
 }
 
-// A raw buffer over [p, p + bytes): its loads take the lane's byte offset in a VGPR and a
-// uniform byte offset in an SGPR, so a step's loads need no 64-bit address per lane.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const double* p, int64_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(p), 0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ double buffer_ld(__amdgpu_buffer_rsrc_t b, int voff, int soff) {
-  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, voff, soff, 0));
-}
-
-// One sweep; returns the LDS buffer that holds its last vector (t_{n-1} after the forward
-// sweep, which is y_{n-1}).  src: v (forward) or the t the forward sweep left in dst
-// (backward).  Byte offsets within a chain fit 31 bits (the host checks n D^2 8 < 2^31).
-template <int Q, int KPL, int P, bool FWD>
-__device__ __forceinline__ int solve_sweep(int D, int n, double c, const double* __restrict__ S,
+// One sweep of a side (side 0: beads below h, side 1: above), K steps of this side in Kmax of the
+// workgroup; returns the LDS buffer (of the side's two, zb) that holds its last vector.  src: v
+// (forward) or the t the forward sweep left in dst (backward).  Byte offsets within a chain fit
+// 31 bits (the host checks n D^2 8 < 2^31).
+template <int Q, int KPL, int P, int NT, bool FWD>
+__device__ __forceinline__ int solve_sweep(int D, int n, int h, int side, int K, int Kmax, int ht,
+                                           double c, const double* __restrict__ S,
                                            const double* src, double* dst, double* zb, int cur) {
   constexpr int QK = Q * KPL;
-  const int tid = threadIdx.x, r = tid / Q, q = tid - r * Q;
+  const int r = ht / Q, q = ht - r * Q;
   const int rr = min(r, D - 1);
   const bool wr = q == 0 && r < D;
-  const int K = FWD ? n : n - 2, DD8 = D * D * 8, D8 = D * 8;
+  const int DD8 = D * D * 8, D8 = D * 8;
   const __amdgpu_buffer_rsrc_t Sb = raw_buffer(S, (int64_t)n * DD8);
   const __amdgpu_buffer_rsrc_t Eb = raw_buffer(src, (int64_t)n * D8);
   int ko[KPL];
 #pragma unroll
   for (int j = 0; j < KPL; ++j) ko[j] = (rr * D + min(q + Q * j, D - 1)) * 8;
   const int eo = rr * 8;
-  // bead of step k, and the bead of the row value it reads (clamped past the end)
-  auto bead = [&](int k) { return FWD ? min(k, n - 1) : max(n - 2 - k, 0); };
-  auto ebead = [&](int k) { return FWD ? min(k + 1, n - 1) : max(n - 2 - k, 0); };
+  // bead of step k, and the bead of the row value it reads (clamped to the chain)
+  auto bead = [&](int k) {
+    const int i = FWD ? (side ? n - 1 - k : k) : (side ? h + 1 + k : h - 1 - k);
+    return min(max(i, 0), n - 1);
+  };
+  auto ebead = [&](int k) { return FWD ? min(max(bead(k) + (side ? -1 : 1), 0), n - 1) : bead(k); };
   double a[P][KPL], e[P];
 #pragma unroll
   for (int s = 0; s < P; ++s) {
@@ -866,38 +886,42 @@ __device__ __forceinline__ int solve_sweep(int D, int n, double c, const double*
     for (int j = 0; j < KPL; ++j) a[s][j] = buffer_ld(Sb, ko[j], so);
     e[s] = buffer_ld(Eb, eo, ebead(s) * D8);
   }
-  for (int k0 = 0; k0 < K; k0 += P) {
+  for (int k0 = 0; k0 < Kmax; k0 += P) {
 #pragma unroll
     for (int s = 0; s < P; ++s) {
       const int k = k0 + s;
-      if (k < K) {  // block-uniform
-        const double* u = zb + cur * QK;
-        double t0 = 0.0, t1 = 0.0;
+      if (k < Kmax) {  // block-uniform
+        if (k < K) {   // the side's waves
+          const double* u = zb + cur * QK;
+          double t0 = 0.0, t1 = 0.0;
 #pragma unroll
-        for (int j = 0; j < KPL; j += 2) {
-          t0 += a[s][j] * u[q + Q * j];
-          if (j + 1 < KPL) t1 += a[s][j + 1] * u[q + Q * (j + 1)];
-        }
-        const double t = row_sum<Q>(t0 + t1), ev = e[s];
-        const int so = bead(k + P) * DD8;
+          for (int j = 0; j < KPL; j += 2) {
+            t0 += a[s][j] * u[q + Q * j];
+            if (j + 1 < KPL) t1 += a[s][j + 1] * u[q + Q * (j + 1)];
+          }
+          const double t = row_sum<Q>(t0 + t1), ev = e[s];
+          const int so = bead(k + P) * DD8, i = bead(k);
 #pragma unroll
-        for (int j = 0; j < KPL; ++j) a[s][j] = buffer_ld(Sb, ko[j], so);
-        e[s] = buffer_ld(Eb, eo, ebead(k + P) * D8);
-        double* nz = zb + (cur ^ 1) * QK;
-        if (FWD) {
-          if (wr) {
-            dst[(int64_t)k * D + r] = t;
-            nz[r] = k + 1 < n ? (k >= 1 ? ev + c * t : ev) : t;
+          for (int j = 0; j < KPL; ++j) a[s][j] = buffer_ld(Sb, ko[j], so);
+          e[s] = buffer_ld(Eb, eo, ebead(k + P) * D8);
+          double* nz = zb + (cur ^ 1) * QK;
+          if (FWD) {
+            if (wr) {
+              dst[(int64_t)i * D + r] = t;
+              // side 1 brings its c t alone to the middle bead, which side 0 gives its v
+              const bool coupled = side || k >= 1, own = !(side && k == K - 1);
+              nz[r] = (own ? ev : 0.0) + (coupled ? c * t : 0.0);
+            }
+          } else {
+            const double y = ev + c * t;
+            if (wr) {
+              dst[(int64_t)i * D + r] = y;
+              nz[r] = y;
+            }
           }
-        } else {
-          const double y = ev + c * t;
-          if (wr) {
-            dst[(int64_t)(n - 2 - k) * D + r] = y;
-            nz[r] = y;
-          }
+          cur ^= 1;
         }
-        cur ^= 1;
-        lds_sync<kRingThreads>();
+        lds_sync<NT>();
       }
     }
   }
@@ -910,49 +934,77 @@ __device__ __forceinline__ int solve_sweep(int D, int n, double c, const double*
 // otherwise the previous v is continued.  Stops after iters iterations, or earlier once eta
 // changes by at most tol relative; chains with act[c] == 0 are left as they are.
 // D <= Q KPL.
-template <int Q, int KPL, int P>
-__global__ void __launch_bounds__(kRingThreads) ring_eta1_kernel(
+template <int Q, int KPL, int P, int HALVES>
+__global__ void __launch_bounds__(HALVES * kRingThreads) ring_eta1_kernel(
     int D, const int* __restrict__ nn, const int64_t* __restrict__ boff,
     const double* __restrict__ betan, const double* __restrict__ sinv, double* __restrict__ work,
     const double* __restrict__ shift, int iters, int fresh, double tol,
     const int* __restrict__ act, double* __restrict__ eta1) {
   static_assert(Q * (kRingThreads / Q) == kRingThreads && (Q == 2 || Q == 4 || Q == 8), "lanes per row");
-  __shared__ double red[kRingThreads];
-  __shared__ double zb[2 * Q * KPL];
+  constexpr int NT = HALVES * kRingThreads, QK = Q * KPL;
+  __shared__ double red[NT];
+  __shared__ double zbs[HALVES][2 * QK], zm[QK];
   const int cix = blockIdx.x, n = nn[cix], tid = threadIdx.x;
   if (act && !act[cix]) return;  // block-uniform
+  const int side = HALVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / kRingThreads);
+  const int ht = tid - side * kRingThreads, h = ring_middle(D, n);
   const int64_t tot = (int64_t)n * D;
   const double c = 1.0 / (betan[cix] * betan[cix]);
   double* v = work + 2 * boff[cix] * D;
   double* y = v + tot;
   const double* S = sinv + (size_t)boff[cix] * D * D;
   const double sig = shift ? shift[cix] : 0.0;
-  if (tid < 2 * Q * KPL) zb[tid] = 0.0;
+  double* zb = zbs[side];
+  if (ht < 2 * QK) zb[ht] = 0.0;
+  if (tid < QK) zm[tid] = 0.0;
   double nrm = 0.0;
-  for (int64_t e = tid; e < tot; e += blockDim.x) {
+  for (int64_t e = tid; e < tot; e += NT) {
     const double t = fresh ? 1.0 + 0.37 * (double)((e * 7919) % 101) / 101.0 : v[e];
     v[e] = t;
     nrm += t * t;
   }
-  nrm = sqrt(block_sum(nrm, red));
-  for (int64_t e = tid; e < tot; e += blockDim.x) v[e] /= nrm;
+  nrm = sqrt(block_sum<NT>(nrm, red));
+  for (int64_t e = tid; e < tot; e += NT) v[e] /= nrm;
   __syncthreads();
   double eta = 0.0, prev = 0.0;
+  const int nup = h, ndn = n - 1 - h;
   for (int it = 0; it < iters; ++it) {
-    if (tid < D) zb[tid] = v[tid];  // z_0 = v_0 in buffer 0
+    if (ht < D) zb[ht] = v[side ? tot - D + ht : ht];  // z_0 and z_{n-1} in the sides' buffers 0
     __syncthreads();
-    int cur = solve_sweep<Q, KPL, P, true>(D, n, c, S, v, y, zb, 0);
-    __syncthreads();  // the t of every lane, in y, before the backward sweep reads them
-    solve_sweep<Q, KPL, P, false>(D, n, c, S, y, y, zb, cur);
+    const int cur = solve_sweep<Q, KPL, P, NT, true>(D, n, h, side, side ? ndn : nup, max(nup, ndn), ht, c,
+                                               S, v, y, zb, 0);
+    // the middle bead: z_h from both sides, y_h = S_h^-1 z_h by side 0, for both sides' way back
+    if (!side && ht < D) zm[ht] = zb[cur * QK + ht];
+    __syncthreads();
+    if (side && h >= 1 && ht < D) zm[ht] += zb[cur * QK + ht];
+    if (HALVES == 2) __syncthreads();
+    if (!side) {
+      const int r = ht / Q, q = ht - r * Q;
+      const double* Sh = S + ((int64_t)h * D + min(r, D - 1)) * D;
+      double t = 0.0;
+#pragma unroll
+      for (int j = 0; j < KPL; ++j) t += Sh[min(q + Q * j, D - 1)] * zm[q + Q * j];
+      t = row_sum<Q>(t);
+      if (q == 0 && r < D) {
+        y[(int64_t)h * D + r] = t;
+#pragma unroll
+        for (int b = 0; b < HALVES; ++b) zbs[b][r] = t;
+      }
+    }
+    __syncthreads();  // and the t of every lane, in y, before the backward sweep reads them
+    // y_0 = t_0, and nothing comes back to side 1 where h = 0: bead 0 is coupled to no other
+    const int kup = max(nup - 1, 0), kdn = h ? ndn : 0;
+    solve_sweep<Q, KPL, P, NT, false>(D, n, h, side, side ? kdn : kup, max(kup, kdn), ht, c, S, y, y,
+                                      zb, 0);
     __syncthreads();
     double mu = 0.0, yy = 0.0;
-    for (int64_t e = tid; e < tot; e += blockDim.x) {
+    for (int64_t e = tid; e < tot; e += NT) {
       mu += v[e] * y[e];
       yy += y[e] * y[e];
     }
-    mu = block_sum(mu, red);
-    yy = sqrt(block_sum(yy, red));
-    for (int64_t e = tid; e < tot; e += blockDim.x) v[e] = y[e] / yy;
+    mu = block_sum<NT>(mu, red);
+    yy = sqrt(block_sum<NT>(yy, red));
+    for (int64_t e = tid; e < tot; e += NT) v[e] = y[e] / yy;
     __syncthreads();
     eta = sig + 1.0 / mu;
     if (it > 2 && fabs(eta - prev) <= tol * fabs(eta)) break;  // block-uniform
@@ -1412,11 +1464,12 @@ int ring_lowest_eigen(rp_ring* r, const std::vector<int>& ng, double* eta) {
     cleanup();
     return rc;
   }
-  // lanes per block row and prefetch depth of the block solve: 8 x 4 columns, 12 steps ahead
-  // for D <= 32; 4 x 16 columns, 4 steps ahead up to kMaxD (the registers of a deeper ring)
+  // lanes per block row, prefetch depth and sides of the block solve: 8 x 4 columns, 12 steps
+  // ahead, from both ends for D <= 32; 4 x 16 columns, 4 steps ahead (the registers of a deeper
+  // ring) up to kMaxD
   auto eta1 = [&](const double* shift, int iters, int fresh, double tol, const int* act) -> int {
-    auto kern = r->D <= 32 ? ring_eta1_kernel<8, 4, 12> : ring_eta1_kernel<4, 16, 4>;
-    kern<<<C, kRingThreads, 0, r->s>>>(r->D, r->d_n.p, r->d_boff.p, r->d_betan.p, r->d_sinv.p,
+    auto kern = r->D <= 32 ? ring_eta1_kernel<8, 4, 12, 2> : ring_eta1_kernel<4, 16, 4, 1>;
+    kern<<<C, kRingThreads * (r->D <= 32 ? 2 : 1), 0, r->s>>>(r->D, r->d_n.p, r->d_boff.p, r->d_betan.p, r->d_sinv.p,
                                        r->d_work.p, shift, iters, fresh, tol, act, r->d_eta.p);
     RP_HIP(hipGetLastError());
     return RP_OK;
