@@ -19,6 +19,7 @@
 // step's normals, the tiles' edge beads and sums, and the potential's parameters.
 #pragma once
 #include "rp_dispatch.h"
+#include "rp_evb_mfma.h"
 #include "rp_nm.h"
 #include "rp_philox.h"
 
@@ -92,16 +93,6 @@ inline int batch_dtiles(const rp_pes* pes) {
   if (pes->kind == PES_WATER) return pes->natom == 3 ? 1 : pes->natom == 6 ? 2 : 4;
   if (pes->kind == PES_COUPLED2D || D <= 16) return 1;
   return 2;
-}
-
-// The EVB block as the fused kernel's MFMA kick reads it from LDS, for DC = 16 DT padded
-// dofs: [kappa, 0 | cA | cB | lam | cub (DC each) | WA (DC rows of stride DC + 1) | WB - WA],
-// zero beyond the potential's own stride, so no operand load needs a clamp or a select.  The
-// difference has columns up to the last dof tile in which the wells' permutation moves a dof
-// (`moved`, BatchArgs), in rows of stride evb_diff_stride.
-__host__ __device__ inline int evb_diff_stride(uint32_t moved) { return moved >> 4 ? 33 : 17; }
-__host__ __device__ inline int evb_kick_lds_size(int DC, uint32_t moved) {
-  return 2 + 4 * DC + DC * (DC + 1) + (moved ? DC * evb_diff_stride(moved) : 0);
 }
 
 // Doubles per bead of the water cluster's positions in LDS

@@ -150,9 +150,7 @@ static BatchArgs base_args(rp_batch* b, const Family& f, double h) {
   a.ndim = b->ndim;
   a.natom = b->natom;
   a.ncu = b->ncu;
-  if (b->pes->kind == PES_EVB)
-    for (int d = 0; d < b->D; ++d)
-      if (b->pes->ip[d / b->ndim] != d / b->ndim) a.moved |= 1u << (d / 4);
+  if (b->pes->kind == PES_EVB) a.moved = evb_moved(b->pes);
   a.first = f.first;
   a.dt = b->dt;
   a.limit = b->limit;

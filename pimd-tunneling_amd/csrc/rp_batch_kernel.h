@@ -2,35 +2,9 @@
 // Included by the per-potential instantiation units (rp_batch_k_*.hip).
 #pragma once
 #include "rp_batch.h"
+#include "rp_evb_mfma.h"
 
 namespace rp {
-
-// f(integral_constant<int, 0..N-1>) expanded at compile time: the state's register indices
-// stay constants even where a loop body is too large for the unroller, so the state never
-// falls back to scratch memory.
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
-__device__ __forceinline__ d4 mfma_f64(double a, double b, d4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
-// DPP moves inside each row of 16 lanes; a lane without a source keeps `old`, or gets zero
-template <int CTRL>
-__device__ __forceinline__ double row_mov(double old, double v) {
-  return __builtin_amdgcn_update_dpp(old, v, CTRL, 0xF, 0xF, false);
-}
-template <int CTRL>
-__device__ __forceinline__ double row_mov0(double v) {
-  return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, true);
-}
-constexpr int kShr = 0x110, kShl = 0x100;  // row_shr:n, row_shl:n
 
 // inclusive sums over each row of 16 lanes, toward higher / lower lanes
 __device__ __forceinline__ double row_prefix(double v) {
@@ -312,137 +286,12 @@ __device__ __forceinline__ void linear_carry(KernArgs& A, const Lane& L,
 // ---------------------------------------------------------------- the kick, p -= dt grad V
 // (verletmodule.f90:565-585)
 
-// The EVB parameter block (evb_eval_at's layout, stride M) -> the kick's LDS layout
-// (evb_kick_lds_size): vectors and matrices zero-padded to DC = 16 DT, matrix rows of
-// stride DC + 1 (the y GEMM reads a column of 16 rows per lane group: an odd stride puts
-// them in distinct banks).  The second matrix is the difference WtB - WtA: the wells differ by
-// a permutation of atoms, so its columns are zero at every atom the permutation leaves.
-template <int M, int DT>
-__device__ __forceinline__ void stage_evb_kick(const double* __restrict__ dp, double* PL, uint32_t moved,
-                                               int tid, int nthreads) {
-  constexpr int DC = DT * 16, LW = DC + 1, NV = 2 + 4 * DC;
-  const double* WA = dp + 1;
-  const double* cA = WA + M * M;
-  const double* WB = cA + M;
-  const double* cB = WB + M * M;
-  const double* lam = cB + M;
-  const double* cub = lam + M;
-  const int ld = evb_diff_stride(moved);
-  for (int e = tid; e < evb_kick_lds_size(DC, moved); e += nthreads) {
-    double v = 0.0;
-    if (e == 0) {
-      v = dp[0];
-    } else if (e >= 2 && e < NV) {
-      const int k = (e - 2) / DC, i = (e - 2) - k * DC;
-      const double* vec = k == 0 ? cA : k == 1 ? cB : k == 2 ? lam : cub;
-      if (i < M) v = vec[i];
-    } else if (e >= NV) {
-      const int f = e - NV, w = f >= DC * LW, r = f - w * (DC * LW);
-      const int i = r / (w ? ld : LW), j = r - i * (w ? ld : LW);
-      if (i < M && j < M) v = w ? WB[i * M + j] - WA[i * M + j] : WA[i * M + j];
-    }
-    PL[e] = v;
-  }
-}
-
-// The EVB on the matrix cores, 16 beads of a wave, from registers to registers.  Both wells'
-// coordinates are y_A = WtA x - cA (one GEMM whose B operand is x as the state holds it: item
-// j of dof tile d is dof 16 d + g + 4 j of bead m, the operand of K-chunk 4 d + j) and
-// y_B = y_A + cA - cB + (WtB - WtA) x, over the K-chunks in `moved` only: those with a dof that
-// the wells' permutation moves.  The mixed gradient is likewise
-// WtA^T (wa hA + wb hB) + (WtB - WtA)^T wb hB, the second product for the dof tiles with a
-// moved dof; its B operand is the first GEMMs' accumulators, scaled in place, and its result
-// has the layout of p.  With two hydrogens exchanged (dofs 0-5 of 27) that is 39 MFMAs per 16
-// beads; both wells in full take 56.  K-chunks beyond M are left out.  The per-bead well
-// energies are reduced over the four lane groups with two xor shuffles.
+// The EVB (evb_gradient), 16 beads of a wave, from registers to registers.
 template <int M, int DT>
 __device__ __forceinline__ void evb_kick(const double* PL, const Lane& L, double dt, uint32_t moved,
                                          const double (&x)[DT][4], double (&p)[DT][4]) {
-  constexpr int DC = DT * 16, LW = DC + 1;
-  const int m = L.m, g = L.g;
-  const double kappa = PL[0];
-  const double* cA = PL + 2 + g;
-  const double* cB = cA + DC;
-  const double* lam = cB + DC;
-  const double* cub = lam + DC;
-  const double* WA = PL + 2 + 4 * DC;
-  const double* WD = WA + DC * LW;
-  const int ld = evb_diff_stride(moved);
-  d4 ya[DT], yb[DT];
-#pragma unroll
-  for (int r = 0; r < DT; ++r) ya[r] = d4{0.0, 0.0, 0.0, 0.0};
-  static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
-    constexpr int kc = decltype(K)::value;
-    if constexpr (4 * kc < M) {
-#pragma unroll
-      for (int r = 0; r < DT; ++r)
-        ya[r] = mfma_f64(WA[(r * 16 + m) * LW + 4 * kc + g], x[kc / 4][kc % 4], ya[r]);
-    }
-  });
-#pragma unroll
-  for (int r = 0; r < DT; ++r) yb[r] = ya[r];
-  static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
-    constexpr int kc = decltype(K)::value;
-    if constexpr (4 * kc < M) {
-      if ((moved >> kc) & 1) {  // wave-uniform
-#pragma unroll
-        for (int r = 0; r < DT; ++r)
-          yb[r] = mfma_f64(WD[(r * 16 + m) * ld + 4 * kc + g], x[kc / 4][kc % 4], yb[r]);
-      }
-    }
-  });
-  // h = lam y + 3 c y^2 and the well energies, per bead m
-  double va = 0.0, vb = 0.0;
-#pragma unroll
-  for (int r = 0; r < DT; ++r)
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      if (r * 16 + 4 * jj >= M) continue;  // padded rows
-      const int i = r * 16 + 4 * jj;
-      const double li = lam[i], ci = cub[i];
-      auto well = [&](double y, double& v, double& h) __attribute__((always_inline)) {
-        const double t = ci * y;
-        v += (y * y) * fma(0.5, li, t);
-        h = y * fma(3.0, t, li);
-      };
-      double ha, hb;
-      well(ya[r][jj] - cA[i], va, ha);
-      well(yb[r][jj] - cB[i], vb, hb);
-      ya[r][jj] = ha;
-      yb[r][jj] = hb;
-    }
-  va += __shfl_xor(va, 16);
-  va += __shfl_xor(va, 32);
-  vb += __shfl_xor(vb, 16);
-  vb += __shfl_xor(vb, 32);
-  const double dl = va - vb, R = sqrt(0.25 * dl * dl + kappa * kappa), f = dl / (4.0 * R);
-  const double wa = -dt * (0.5 - f), wb = -dt * (0.5 + f);
-#pragma unroll
-  for (int r = 0; r < DT; ++r) {
-    yb[r] *= wb;
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) ya[r][jj] = fma(wa, ya[r][jj], yb[r][jj]);
-  }
   d4 ag[DT];
-#pragma unroll
-  for (int d = 0; d < DT; ++d) ag[d] = d4{0.0, 0.0, 0.0, 0.0};
-  static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
-    constexpr int kc = decltype(K)::value;
-    if constexpr (4 * kc < M) {
-#pragma unroll
-      for (int d = 0; d < DT; ++d)
-        ag[d] = mfma_f64(WA[(4 * kc + g) * LW + d * 16 + m], ya[kc / 4][kc % 4], ag[d]);
-    }
-  });
-#pragma unroll
-  for (int d = 0; d < DT; ++d)
-    if ((moved >> (4 * d)) & 15u) {  // wave-uniform
-      static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
-        constexpr int kc = decltype(K)::value;
-        if constexpr (4 * kc < M)
-          ag[d] = mfma_f64(WD[(4 * kc + g) * ld + d * 16 + m], yb[kc / 4][kc % 4], ag[d]);
-      });
-    }
+  evb_gradient<M, DT>(PL, L.m, L.g, moved, -dt, x, ag);
 #pragma unroll
   for (int d = 0; d < DT; ++d)
 #pragma unroll

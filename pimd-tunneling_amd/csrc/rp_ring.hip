@@ -7,7 +7,7 @@
 #include <cmath>
 #include <cstring>
 
-#include "rp_dispatch.h"
+#include "rp_evb_mfma.h"
 #include "rp_ring.h"
 #include <algorithm>
 
@@ -125,215 +125,99 @@ __global__ void __launch_bounds__(kRingTile) ring_um_kernel(RingArgs A, const do
   }
 }
 
-// U_M and its adjoint gradient for the EVB on the matrix cores.  A wave takes a tile of 16
-// beads: both wells' coordinates y = Wt x - cw are one GEMM (rows: 2 x 16 RT well rows; K:
-// the dofs) and the mixed gradient wa WtA^T hA + wb WtB^T hB a second GEMM whose B operand
-// is the first one's accumulators, scaled in place (item j of row tile rt holds row
-// 16 rt + g + 4 j of bead m, the operand of K-chunk 4 rt + j).  The spring terms are then
-// added per (bead, dof) as in ring_um_kernel.  The sums run in another order than that
-// kernel's per-bead loop, so the two agree to rounding, not bit for bit.
-typedef double rd4 __attribute__((ext_vector_type(4)));
-constexpr int kUmWaves = 4;
+// U_M and its adjoint gradient for the EVB on the matrix cores: a wave takes 16 beads of a
+// chain through evb_gradient in registers (x as loaded is the layout of its GEMMs' operand
+// and of its result), adds the springs from the neighbouring lanes' beads, and stores.  Every
+// load and store is 16 consecutive beads of a dof.  Persistent: as many workgroups as the GPU
+// runs at once stage the EVB block in LDS, then a wave takes every waves-th tile of the list
+// (tiles[2t] = chain, tiles[2t + 1] = first bead).
+// 143k beads of 256 chains: 33 us; with the tile's x, potential gradients and neighbours
+// through LDS, four waves and three barriers per 64 beads, 58 us.
+constexpr int kUmWaves = 8;
 
-// Persistent: the grid is a few workgroups per CU, each staging the EVB block once and then
-// taking bead tiles from the task list (tasks[2t] = chain, tasks[2t + 1] = first bead).
 template <int M>
-__global__ void __launch_bounds__(kUmWaves * 64) ring_um_evb_kernel(RingArgs A,
-                                                                    const double* __restrict__ x,
-                                                                    double* __restrict__ grad,
-                                                                    double* __restrict__ energy,
-                                                                    const int* __restrict__ tasks,
-                                                                    int ntask) {
-  constexpr int RT = (M + 15) / 16;  // row tiles per well, and dof tiles
-  constexpr int DC = 16 * RT;        // padded dofs
-  constexpr int LX = DC + 1;         // LDS stride of one bead
-  constexpr int KY = 4 * RT;         // K-chunks of the y GEMM
-  constexpr int KG = 8 * RT;         // K-chunks of the gradient GEMM
-  constexpr int NT = kUmWaves * 64;
-  constexpr int TB = kUmWaves * 16;  // beads per workgroup
-  __shared__ double pl[evb_dev_size<M>()];
-  __shared__ double xs[(TB + 2) * LX];  // x of beads b0-1 .. b0+TB (row 0 is bead b0-1)
-  __shared__ double gp[TB * LX];        // the potential gradient of beads b0 .. b0+TB-1
-  __shared__ double vpot[TB];
-  __shared__ double red[NT];
-  __shared__ double sm[3 * M];  // per dof: mass, end bead a, end bead b
-  const int D = A.D;
-  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
+__global__ void __launch_bounds__(kUmWaves * 64, 4) ring_um_evb_kernel(
+    RingArgs A, uint32_t moved, const double* __restrict__ x, double* __restrict__ grad,
+    double* __restrict__ part, const int* __restrict__ tiles, int ntile) {
+  constexpr int DT = (M + 15) / 16, DC = 16 * DT;
+  extern __shared__ double PL[];
+  const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  {
-    const double* __restrict__ dp = A.pes.dp;
-    constexpr int NPL = (evb_dev_size<M>() + NT - 1) / NT;
-    double vpl[NPL];
-#pragma unroll
-    for (int q = 0; q < NPL; ++q) {
-      const int e = tid + q * NT;
-      vpl[q] = e < evb_dev_size<M>() ? dp[e] : 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q < NPL; ++q)
-      if (tid + q * NT < evb_dev_size<M>()) pl[tid + q * NT] = vpl[q];
-  }
-  for (int task = blockIdx.x; task < ntask; task += gridDim.x) {
-    const int c = tasks[2 * task], b0 = tasks[2 * task + 1];
-    const int n = A.n[c];
+  const int D = A.D, fixedends = A.fixedends;
+  double* mass = PL + ((evb_kick_lds_size(DC, moved) + 1) & ~1);
+  stage_evb_kick<M, DT>(A.pes.dp, PL, moved, tid, kUmWaves * 64);
+  if (tid < DC) mass[tid] = tid < D ? A.massd[tid] : 0.0;
+  __syncthreads();
+  for (int t = blockIdx.x * kUmWaves + wave; t < ntile; t += gridDim.x * kUmWaves) {
+    // an opaque lane per tile: the block's LDS fragments are read where they are used instead
+    // of being kept in (and spilled from) registers across the tiles
+    int lane = tid & 63;
+    asm volatile("" : "+v"(lane));
+    const int m = lane & 15, g = lane >> 4;
+    const int c = tiles[2 * t], b0 = tiles[2 * t + 1], n = A.n[c];
+    const int i = b0 + m;
+    // the bead a lane's row move has no source for: before the tile (m = 0) or after it
+    const int ie = m == 0 ? max(i - 1, 0) : min(i + 1, n - 1);
+    const double ibn2 = 1.0 / (A.betan[c] * A.betan[c]);
     const double* __restrict__ xc = x + A.off[c];
-    {
-      // every staging load of a thread is issued before the first one is used (compile-time
-      // trip counts, registers in between): one memory latency for the whole staging, and it
-      // overlaps the previous tile's last barrier
-      const double* __restrict__ abc = A.ab + (size_t)c * 2 * D;
-      constexpr int NXS = ((TB + 2) * DC + NT - 1) / NT;
-      double vxs[NXS], vsm = 0.0;
+    const double* __restrict__ ab = A.ab + (size_t)c * 2 * D;
+    double xs[DT][4], xe[DT][4];
 #pragma unroll
-      for (int q = 0; q < NXS; ++q) {
-        const int e = tid + q * NT;
-        // consecutive threads, consecutive beads
-        const int d = e / (TB + 2), bl = e - d * (TB + 2);
-        const int i = b0 - 1 + bl;
-        vxs[q] = (d < D && i >= 0 && i < n) ? xc[(size_t)d * n + i] : 0.0;
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int row = 16 * d + 4 * j + g;
+        const double* xd = xc + (size_t)min(row, D - 1) * n;
+        // the fixed ends stand in for beads -1 and n
+        xs[d][j] = row >= D ? 0.0 : i < n ? xd[i] : ab[D + row];
+        xe[d][j] = row >= D ? 0.0
+                   : (m == 0 && i == 0) ? ab[row]
+                   : (m == 15 && i >= n - 1) ? ab[D + row]
+                                             : xd[ie];
       }
-      if (tid < 3 * D) vsm = tid < D ? A.massd[tid] : abc[tid - D];
-      lds_sync<NT>();  // the previous tile is done with xs, gp, vpot and sm
+    d4 ag[DT];
+    const double v = evb_gradient<M, DT>(PL, m, g, moved, 1.0, xs, ag);
+    const bool on = i < n, first = i == 0, last = i == n - 1;
+    double e = on && g == 0 ? v - A.pes.v0 : 0.0;  // as eval_kind
 #pragma unroll
-      for (int q = 0; q < NXS; ++q) {
-        const int e = tid + q * NT;
-        const int d = e / (TB + 2), bl = e - d * (TB + 2);
-        if (e < (TB + 2) * DC) xs[bl * LX + d] = vxs[q];
-      }
-      if (tid < 3 * D) sm[tid] = vsm;
-    }
-    lds_sync<NT>();
-    {
-      const double kappa = pl[0];
-      const double* WA = pl + 1;
-      const double* cA = WA + M * M;
-      const double* WB = cA + M;
-      const double* cB = WB + M * M;
-      const double* lam = cB + M;
-      const double* cub = lam + M;
-      const int tb = wave * 16;
-      rd4 ay[2 * RT];
+    for (int d = 0; d < DT; ++d)
 #pragma unroll
-      for (int r = 0; r < 2 * RT; ++r) ay[r] = rd4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int kc = 0; kc < KY; ++kc) {
-        const int j = 4 * kc + g;
-        const double bx = xs[(tb + m + 1) * LX + j];
-#pragma unroll
-        for (int r = 0; r < 2 * RT; ++r) {
-          const int i = (r % RT) * 16 + m;
-          const double* Wt = r < RT ? WA : WB;
-          const double w = Wt[min(i, M - 1) * M + min(j, M - 1)];
-          ay[r] = __builtin_amdgcn_mfma_f64_16x16x4f64((i < M && j < M) ? w : 0.0, bx, ay[r], 0,
-                                                       0, 0);
+      for (int j = 0; j < 4; ++j) {
+        const int row = 16 * d + 4 * j + g;
+        const double k = mass[row] * ibn2, xi = xs[d][j];
+        const double xl = row_mov<kShr + 1>(xe[d][j], xi);
+        const double xr = row_mov<kShl + 1>(xe[d][j], xi);
+        const double dl = first && !fixedends ? 0.0 : xi - xl;
+        const double dr = last && !fixedends ? 0.0 : xr - xi;
+        if (on) {
+          // the spring to the right, and the one to the fixed start
+          e += (0.5 * k) * (dr * dr + (first ? dl * dl : 0.0));
+          if (grad && row < D) grad[A.off[c] + (size_t)row * n + i] = k * (dl - dr) + ag[d][j];
         }
       }
-      double va = 0.0, vb = 0.0;
-#pragma unroll
-      for (int r = 0; r < 2 * RT; ++r)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int i = (r % RT) * 16 + g + 4 * jj;
-          const bool ok = i < M;
-          const int ic = min(i, M - 1);
-          const double cw = ok ? (r < RT ? cA[ic] : cB[ic]) : 0.0;
-          const double li = ok ? lam[ic] : 0.0, ci = ok ? cub[ic] : 0.0;
-          const double y = ay[r][jj] - cw, y2 = y * y;
-          const double v = (0.5 * li) * y2 + ci * y2 * y;
-          if (r < RT)
-            va += v;
-          else
-            vb += v;
-          ay[r][jj] = li * y + (3.0 * ci) * y2;
-        }
-      va += __shfl_xor(va, 16);
-      va += __shfl_xor(va, 32);
-      vb += __shfl_xor(vb, 16);
-      vb += __shfl_xor(vb, 32);
-      const double dl = va - vb, R = sqrt(0.25 * dl * dl + kappa * kappa), f = dl / (4.0 * R);
-      const double wa = 0.5 - f, wb = 0.5 + f;
-#pragma unroll
-      for (int r = 0; r < 2 * RT; ++r) ay[r] *= (r < RT ? wa : wb);
-      rd4 ag[RT];
-#pragma unroll
-      for (int d = 0; d < RT; ++d) ag[d] = rd4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int kc = 0; kc < KG; ++kc) {
-        const int r = kc / 4, jj = kc % 4;
-        const int i = (r % RT) * 16 + 4 * jj + g;
-        const double* Wt = r < RT ? WA : WB;
-        const double bh = ay[r][jj];
-#pragma unroll
-        for (int d = 0; d < RT; ++d) {
-          const int dof = d * 16 + m;
-          const double w = Wt[min(i, M - 1) * M + min(dof, M - 1)];
-          ag[d] = __builtin_amdgcn_mfma_f64_16x16x4f64((i < M && dof < M) ? w : 0.0, bh, ag[d],
-                                                       0, 0, 0);
-        }
-      }
-      if (g == 0) vpot[tb + m] = (0.5 * (va + vb) - R) - A.pes.v0;  // as eval_kind
-#pragma unroll
-      for (int d = 0; d < RT; ++d)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) gp[(tb + m) * LX + d * 16 + g + 4 * jj] = ag[d][jj];
-    }
-    lds_sync<NT>();
-    // springs per (bead, dof), as in ring_um_kernel; the neighbours, masses and end beads come
-    // from LDS
-    const double bn2 = A.betan[c] * A.betan[c];
-    const double* a = sm + D;
-    const double* b = sm + 2 * D;
-    double e = 0.0;
-    double* __restrict__ gout = grad ? grad + A.off[c] : nullptr;  // loaded once, not per store
-    const bool fixedends = A.fixedends;
-    constexpr int NSP = (TB * M + NT - 1) / NT;
-#pragma unroll
-    for (int q = 0; q < NSP; ++q) {
-      const int t = tid + q * NT;
-      const int d = t / TB, bl = t - d * TB;
-      const int i = b0 + bl;
-      if (t >= TB * D || i >= n) continue;
-      const double m_ = sm[d];
-      const double xi = xs[(bl + 1) * LX + d];
-      const double xl = xs[bl * LX + d];        // bead i - 1 (0 before the first bead)
-      const double xr = xs[(bl + 2) * LX + d];  // bead i + 1 (0 after the last bead)
-      if (d == 0) e += vpot[bl];
-      if (i < n - 1) {
-        const double dx = xr - xi;
-        e += (0.5 * m_ / bn2) * dx * dx;
-      }
-      double sg;
-      if (n == 1)
-        sg = fixedends ? m_ * (2.0 * xi - a[d] - b[d]) / bn2 : 0.0;
-      else if (i == 0)
-        sg = fixedends ? m_ * (2.0 * xi - a[d] - xr) / bn2 : m_ * (xi - xr) / bn2;
-      else if (i == n - 1)
-        sg = fixedends ? m_ * (2.0 * xi - xl - b[d]) / bn2 : m_ * (xi - xl) / bn2;
-      else
-        sg = m_ * (2.0 * xi - xl - xr) / bn2;
-      if (fixedends && i == 0) e += (0.5 * m_ / bn2) * (xi - a[d]) * (xi - a[d]);
-      if (fixedends && i == n - 1) e += (0.5 * m_ / bn2) * (b[d] - xi) * (b[d] - xi);
-      if (gout) gout[(size_t)d * n + i] = sg + gp[bl * LX + d];
-    }
-    // the energy: a wave sum, then the waves' sums through LDS behind an LDS-only barrier (a
-    // full barrier would first wait for every gradient store above to be acknowledged)
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o);
-    if (lane == 0) red[wave] = e;
-    lds_sync<NT>();
-    if (tid == 0) {
-      double t = 0.0;
+    if (lane == 0) part[t] = e;
+  }
+}
+
+// energy[c] = the sum of chain c's tiles, in an order of its own (the same for every batch)
+__global__ void __launch_bounds__(64) ring_um_sum_kernel(const double* __restrict__ part,
+                                                         const int* __restrict__ first,
+                                                         double* __restrict__ energy) {
+  const int c = blockIdx.x, t1 = first[c + 1];
+  double e = 0.0;
+  for (int t = first[c] + threadIdx.x; t < t1; t += 64) e += part[t];
 #pragma unroll
-      for (int w = 0; w < kUmWaves; ++w) t += red[w];
-      atomicAdd(&energy[c], t);
-    }
-  }  // tasks
+  for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o);
+  if (threadIdx.x == 0) energy[c] = e;
 }
 
 // Hessian-vector product of U_M: springs exactly, potential by forward-over-reverse.
 template <int KIND, int MAXD>
 __global__ void __launch_bounds__(kRingTile) ring_hvp_kernel(RingArgs A, const double* __restrict__ x,
                                                              const double* __restrict__ v,
+                                                             const double* __restrict__ w,
                                                              double* __restrict__ hv) {
   const int c = blockIdx.y;
   const int n = A.n[c], D = A.D;
@@ -360,7 +244,8 @@ __global__ void __launch_bounds__(kRingTile) ring_hvp_kernel(RingArgs A, const d
       s = A.fixedends ? 2.0 * vd[i] - vd[i - 1] : vd[i] - vd[i - 1];
     else
       s = 2.0 * vd[i] - vd[i - 1] - vd[i + 1];
-    hv[o + (size_t)d * n + i] = m * s / bn2 + gs[d].d;
+    const double h = m * s / bn2 + gs[d].d;
+    hv[o + (size_t)d * n + i] = w ? w[c] * h : h;  // w: the chains' weights, or null
   }
 }
 
@@ -388,6 +273,57 @@ __global__ void __launch_bounds__(128) ring_hblock_kernel(RingArgs A, const doub
 #pragma unroll
   for (int k = 0; k < MAXD; ++k)
     if (k < D) blk[k] = gs[k].d;
+}
+
+// The weight kernels of a scalar built from the chains' actions (sum_c w_c U_c): grid (tiles of
+// kVecTile elements, chains).
+constexpr int kVecThreads = 256, kVecTile = 4 * kVecThreads;
+
+// x -> the ring's coordinates, and the energies cleared for ring_eval's sums
+__global__ void __launch_bounds__(kVecThreads) ring_load_kernel(const int64_t* __restrict__ off,
+                                                                const int* __restrict__ n, int D,
+                                                                const double* __restrict__ x,
+                                                                double* __restrict__ xr,
+                                                                double* __restrict__ energy) {
+  const int c = blockIdx.y, L = n[c] * D;
+  const int64_t o = off[c];
+  if (energy && blockIdx.x == 0 && threadIdx.x == 0) energy[c] = 0.0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int j = blockIdx.x * kVecTile + k * kVecThreads + threadIdx.x;
+    if (j < L) xr[o + j] = x[o + j];
+  }
+}
+
+// out = w_c g of every chain
+__global__ void __launch_bounds__(kVecThreads) ring_weight_kernel(const int64_t* __restrict__ off,
+                                                                  const int* __restrict__ n, int D,
+                                                                  const double* __restrict__ w,
+                                                                  const double* __restrict__ g,
+                                                                  double* __restrict__ out) {
+  const int c = blockIdx.y, L = n[c] * D;
+  const int64_t o = off[c];
+  const double wc = w[c];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int j = blockIdx.x * kVecTile + k * kVecThreads + threadIdx.x;
+    if (j < L) out[o + j] = wc * g[o + j];
+  }
+}
+
+// out[c] = a . b of chain c, one workgroup per chain, in a fixed order
+__global__ void __launch_bounds__(kRingThreads) ring_dot_kernel(const int64_t* __restrict__ off,
+                                                                const int* __restrict__ n, int D,
+                                                                const double* __restrict__ a,
+                                                                const double* __restrict__ b,
+                                                                double* __restrict__ out) {
+  __shared__ double red[kRingThreads];
+  const int c = blockIdx.x, L = n[c] * D;
+  const int64_t o = off[c];
+  double s = 0.0;
+  for (int j = threadIdx.x; j < L; j += kRingThreads) s += a[o + j] * b[o + j];
+  s = block_sum(s, red);
+  if (threadIdx.x == 0) out[c] = s;
 }
 
 // U_M and its gradient for a potential that lives on the host: the bead energies pe[gbead]
@@ -534,17 +470,6 @@ __device__ __forceinline__ double pivot_recip(double x) {
   double r = __builtin_amdgcn_rcp(x);
   r = fma(r, fma(-x, r, 1.0), r);
   return fma(r, fma(-x, r, 1.0), r);
-}
-
-// f(integral_constant<int, 0..N-1>) expanded at compile time (tile and item indices stay
-// constants, so the tiles stay in registers)
-template <typename F, int... I>
-__device__ __forceinline__ void static_unroll_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_unroll(F&& f) {
-  static_unroll_impl(f, std::make_integer_sequence<int, N>{});
 }
 
 __device__ __forceinline__ double read_lane(double v, int lane) {
@@ -1025,6 +950,7 @@ struct rp_ring {
   int64_t tot = 0, nbeads = 0;
   int nmax = 0;  // the longest chain
   hipStream_t s = nullptr;
+  hipEvent_t ev = nullptr;  // the last stream-ordered call's work (rp_ring_*_stream)
   DevBuf<double> d_x, d_g, d_v, d_hv, d_e, d_ab, d_betan, d_massd, d_blocks, d_sinv, d_work, d_ld,
       d_eta;
   DevBuf<int> d_n, d_nneg;
@@ -1038,7 +964,8 @@ struct rp_ring {
   DevBuf<double> d_pctab;
   DevBuf<int64_t> d_pcoff;
   // the EVB U_M kernel's bead tiles (chain, first bead) and its persistent grid
-  DevBuf<int> d_umtask;
+  DevBuf<int> d_umtask, d_umfirst;
+  DevBuf<double> d_umpart;
   int n_umtask = 0, um_grid = 0;
 };
 
@@ -1082,49 +1009,61 @@ static int ring_host_potential(rp_ring* r, bool want_grad) {
   return RP_OK;
 }
 
-int ring_eval(rp_ring* r, bool want_grad) {
+// U_M of the ring's coordinates into energy (cleared by the caller, for potentials whose
+// kernel adds to it) and, unless null, its gradient into grad, queued on stream
+static int ring_eval_to(rp_ring* r, double* energy, double* grad, hipStream_t stream) {
   RingArgs a = ring_args(r);
-  RP_HIP(hipMemsetAsync(r->d_e.p, 0, sizeof(double) * r->nchain, r->s));
   const dim3 grid((unsigned)((r->nmax + kRingTile - 1) / kRingTile), (unsigned)r->nchain);
   if (r->pes->kind == PES_HOST) {
-    int rc = ring_host_potential(r, want_grad);
+    int rc = ring_host_potential(r, grad != nullptr);  // its gradient goes to d_g
     if (rc) return rc;
-    ring_spring_kernel<<<grid, kRingTile, 0, r->s>>>(a, r->d_x.p, r->d_pe.p,
-                                                     want_grad ? r->d_g.p : nullptr, r->d_e.p);
+    ring_spring_kernel<<<grid, kRingTile, 0, stream>>>(a, r->d_x.p, r->d_pe.p, grad, energy);
     RP_HIP(hipGetLastError());
     return RP_OK;
   }
   return dispatch_pes(r->pes, [&]<int K, int M>() -> int {
-    if constexpr (K == PES_EVB) {  // the EVB's two GEMMs per bead tile on the matrix cores
-      constexpr int TB = kUmWaves * 16;
+    if constexpr (K == PES_EVB) {
+      const uint32_t moved = evb_moved(r->pes);
+      constexpr int DC = 16 * ((M + 15) / 16);
+      const size_t lds = (((evb_kick_lds_size(DC, moved) + 1) & ~1) + DC) * sizeof(double);
       if (!r->d_umtask.p) {  // the bead tiles of every chain, once per ring
-        std::vector<int> t;
-        for (int c = 0; c < r->nchain; ++c)
-          for (int b0 = 0; b0 < r->n[c]; b0 += TB) {
+        std::vector<int> t, first;
+        for (int c = 0; c < r->nchain; ++c) {
+          first.push_back((int)t.size() / 2);
+          for (int b0 = 0; b0 < r->n[c]; b0 += 16) {
             t.push_back(c);
             t.push_back(b0);
           }
+        }
+        first.push_back((int)t.size() / 2);
         int rc;
-        if ((rc = r->d_umtask.alloc(t.size())) || (rc = r->d_umtask.upload(t.data(), t.size(), r->s)))
+        if ((rc = r->d_umpart.alloc(t.size() / 2)) || (rc = r->d_umfirst.alloc(first.size())) ||
+            (rc = r->d_umfirst.upload(first.data(), first.size(), r->s)) ||
+            (rc = r->d_umtask.alloc(t.size())) || (rc = r->d_umtask.upload(t.data(), t.size(), r->s)))
           return rc;
-        RP_HIP(hipStreamSynchronize(r->s));  // t is released at the end of this block
+        RP_HIP(hipStreamSynchronize(r->s));  // t and first are released at the end of this block
         r->n_umtask = (int)(t.size() / 2);
         int ncu = 0, dev = 0, per_cu = 0;
         RP_HIP(hipGetDevice(&dev));
         RP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
         RP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ring_um_evb_kernel<M>,
-                                                            kUmWaves * 64, 0));
-        r->um_grid = std::min(r->n_umtask, std::max(per_cu, 1) * std::max(ncu, 1));
+                                                            kUmWaves * 64, lds));
+        r->um_grid = std::min((r->n_umtask + kUmWaves - 1) / kUmWaves, std::max(per_cu, 1) * std::max(ncu, 1));
       }
-      ring_um_evb_kernel<M><<<r->um_grid, kUmWaves * 64, 0, r->s>>>(
-          a, r->d_x.p, want_grad ? r->d_g.p : nullptr, r->d_e.p, r->d_umtask.p, r->n_umtask);
+      ring_um_evb_kernel<M><<<r->um_grid, kUmWaves * 64, lds, stream>>>(
+          a, moved, r->d_x.p, grad, r->d_umpart.p, r->d_umtask.p, r->n_umtask);
+      ring_um_sum_kernel<<<r->nchain, 64, 0, stream>>>(r->d_umpart.p, r->d_umfirst.p, energy);
     } else {
-      ring_um_kernel<K, M><<<grid, kRingTile, 0, r->s>>>(a, r->d_x.p,
-                                                                want_grad ? r->d_g.p : nullptr, r->d_e.p);
+      ring_um_kernel<K, M><<<grid, kRingTile, 0, stream>>>(a, r->d_x.p, grad, energy);
     }
     RP_HIP(hipGetLastError());
     return RP_OK;
   });
+}
+
+int ring_eval(rp_ring* r, bool want_grad) {
+  if (r->pes->kind != PES_EVB) RP_HIP(hipMemsetAsync(r->d_e.p, 0, sizeof(double) * r->nchain, r->s));
+  return ring_eval_to(r, r->d_e.p, want_grad ? r->d_g.p : nullptr, r->s);
 }
 int ring_tot(const rp_ring* r) { return (int)r->tot; }
 int ring_nchain(const rp_ring* r) { return r->nchain; }
@@ -1249,6 +1188,7 @@ extern "C" int rp_ring_set_preconditioner(rp_ring* r, double sigma) {
 extern "C" int rp_ring_destroy(rp_ring* r) {
   if (!r) return RP_OK;
   if (r->s) (void)hipStreamSynchronize(r->s);
+  if (r->ev) (void)hipEventDestroy(r->ev);
   for (DevBuf<double>* b : {&r->d_x, &r->d_g, &r->d_v, &r->d_hv, &r->d_e, &r->d_ab, &r->d_betan,
                             &r->d_massd, &r->d_blocks, &r->d_sinv, &r->d_work, &r->d_ld, &r->d_eta,
                             &r->d_pe, &r->d_pctab})
@@ -1256,6 +1196,8 @@ extern "C" int rp_ring_destroy(rp_ring* r) {
   r->d_n.free();
   r->d_nneg.free();
   r->d_umtask.free();
+  r->d_umfirst.free();
+  r->d_umpart.free();
   r->d_off.free();
   r->d_boff.free();
   r->d_pcoff.free();
@@ -1289,22 +1231,28 @@ extern "C" int rp_ring_um(rp_ring* r, double* energy, double* grad) {
 
 static int ring_blocks(rp_ring* r, int singlewell);
 
-// d_hv = H d_v at d_x (queued on the ring's stream)
-static int ring_hvp(rp_ring* r) {
-  int rc;
+// hv = H v at d_x, times the chains' weights w unless null (queued on stream)
+static int ring_hvp_to(rp_ring* r, const double* v, const double* w, double* hv, hipStream_t stream) {
   RingArgs a = ring_args(r);
   const dim3 grid((unsigned)((r->nmax + kRingTile - 1) / kRingTile), (unsigned)r->nchain);
-  if (r->pes->kind == PES_HOST) {  // the plugin's Hessian blocks, then the block product
-    if ((rc = ring_blocks(r, 0))) return rc;
-    ring_hvp_blocks_kernel<<<grid, kRingTile, 0, r->s>>>(a, r->d_blocks.p, r->d_v.p, r->d_hv.p);
-    RP_HIP(hipGetLastError());
-    return RP_OK;
-  }
   return dispatch_pes(r->pes, [&]<int K, int M>() -> int {
-    ring_hvp_kernel<K, M><<<grid, kRingTile, 0, r->s>>>(a, r->d_x.p, r->d_v.p, r->d_hv.p);
+    ring_hvp_kernel<K, M><<<grid, kRingTile, 0, stream>>>(a, r->d_x.p, v, w, hv);
     RP_HIP(hipGetLastError());
     return RP_OK;
   });
+}
+
+// d_hv = H d_v at d_x (queued on the ring's stream)
+static int ring_hvp(rp_ring* r) {
+  int rc;
+  if (r->pes->kind == PES_HOST) {  // the plugin's Hessian blocks, then the block product
+    if ((rc = ring_blocks(r, 0))) return rc;
+    const dim3 grid((unsigned)((r->nmax + kRingTile - 1) / kRingTile), (unsigned)r->nchain);
+    ring_hvp_blocks_kernel<<<grid, kRingTile, 0, r->s>>>(ring_args(r), r->d_blocks.p, r->d_v.p, r->d_hv.p);
+    RP_HIP(hipGetLastError());
+    return RP_OK;
+  }
+  return ring_hvp_to(r, r->d_v.p, nullptr, r->d_hv.p, r->s);
 }
 
 extern "C" int rp_ring_hvp(rp_ring* r, const double* v, double* hv) {
@@ -1342,6 +1290,63 @@ extern "C" int rp_ring_hvp_device(rp_ring* r, const double* v, double* hv) {
   if ((rc = ring_hvp(r))) return rc;
   RP_HIP(hipMemcpyAsync(hv, r->d_hv.p, sizeof(double) * r->tot, hipMemcpyDeviceToDevice, r->s));
   RP_HIP(hipStreamSynchronize(r->s));
+  return RP_OK;
+}
+
+// Stream-ordered entry points: the work is queued on the caller's stream, ordered with every
+// other call on the ring by one event (the caller's stream waits for what the ring last
+// queued, the ring's own stream for this).
+static int stream_begin(rp_ring* r, hipStream_t s) {
+  if (!r->ev) RP_HIP(hipEventCreateWithFlags(&r->ev, hipEventDisableTiming));
+  else RP_HIP(hipStreamWaitEvent(s, r->ev, 0));
+  return RP_OK;
+}
+static int stream_end(rp_ring* r, hipStream_t s) {
+  RP_HIP(hipGetLastError());
+  RP_HIP(hipEventRecord(r->ev, s));
+  RP_HIP(hipStreamWaitEvent(r->s, r->ev, 0));
+  return RP_OK;
+}
+static dim3 vec_grid(const rp_ring* r) {
+  return dim3((unsigned)((r->nmax * r->D + kVecTile - 1) / kVecTile), (unsigned)r->nchain);
+}
+
+extern "C" int rp_ring_action_stream(rp_ring* r, const double* x, double* energy, double* grad,
+                                     void* stream) {
+  RP_REQUIRE(r && x && energy, "rp_ring_action_stream: bad arguments");
+  RP_REQUIRE(r->pes->kind != PES_HOST, "rp_ring_action_stream: the potential lives on the host");
+  hipStream_t s = (hipStream_t)stream;
+  int rc = stream_begin(r, s);
+  if (rc) return rc;
+  ring_load_kernel<<<vec_grid(r), kVecThreads, 0, s>>>(r->d_off.p, r->d_n.p, r->D, x, r->d_x.p, energy);
+  if ((rc = ring_eval_to(r, energy, grad, s))) return rc;
+  return stream_end(r, s);
+}
+
+extern "C" int rp_ring_hvp_stream(rp_ring* r, const double* x, const double* v, const double* w,
+                                  double* hv, void* stream) {
+  RP_REQUIRE(r && x && v && hv, "rp_ring_hvp_stream: bad arguments");
+  RP_REQUIRE(r->pes->kind != PES_HOST, "rp_ring_hvp_stream: the potential lives on the host");
+  hipStream_t s = (hipStream_t)stream;
+  int rc = stream_begin(r, s);
+  if (rc) return rc;
+  ring_load_kernel<<<vec_grid(r), kVecThreads, 0, s>>>(r->d_off.p, r->d_n.p, r->D, x, r->d_x.p, nullptr);
+  if ((rc = ring_hvp_to(r, v, w, hv, s))) return rc;
+  return stream_end(r, s);
+}
+
+extern "C" int rp_ring_weight_stream(rp_ring* r, const double* w, const double* g, double* out,
+                                     void* stream) {
+  RP_REQUIRE(r && w && g && out, "rp_ring_weight_stream: bad arguments");
+  ring_weight_kernel<<<vec_grid(r), kVecThreads, 0, (hipStream_t)stream>>>(r->d_off.p, r->d_n.p, r->D, w, g, out);
+  RP_HIP(hipGetLastError());
+  return RP_OK;
+}
+
+extern "C" int rp_ring_dot_stream(rp_ring* r, const double* a, const double* b, double* out, void* stream) {
+  RP_REQUIRE(r && a && b && out, "rp_ring_dot_stream: bad arguments");
+  ring_dot_kernel<<<r->nchain, kRingThreads, 0, (hipStream_t)stream>>>(r->d_off.p, r->d_n.p, r->D, a, b, out);
+  RP_HIP(hipGetLastError());
   return RP_OK;
 }
 

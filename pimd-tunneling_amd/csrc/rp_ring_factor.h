@@ -59,7 +59,7 @@ __global__ void __launch_bounds__(128, 2) ring_factor_kernel(
 #pragma unroll
     for (int j = 0; j < 4; ++j) vo[t][j] = min(16 * t + 4 * j + g, D - 1) * D * 8;
   }
-  rd4 acc[RT][RT], nxt[RT][RT];
+  d4 acc[RT][RT], nxt[RT][RT];
   auto load = [&](int bead) __attribute__((always_inline)) {
     const int so = bead * DD8;
 #pragma unroll
@@ -102,7 +102,7 @@ __global__ void __launch_bounds__(128, 2) ring_factor_kernel(
     return (int)(sd + ((sa & ~sd) << 1));
   };
   auto sweep = [&]() __attribute__((always_inline)) {
-    static_unroll<4 * RT>([&](auto Sx) __attribute__((always_inline)) {
+    static_for<4 * RT>([&](auto Sx) __attribute__((always_inline)) {
       constexpr int s = decltype(Sx)::value, t = s / 4, j = s % 4;
       if (4 * s >= D) return;  // uniform
       double W[RT];
@@ -134,7 +134,7 @@ __global__ void __launch_bounds__(128, 2) ring_factor_kernel(
       double pw[RT];                  // -P M[K][c], and +P in the pivot columns
 #pragma unroll
       for (int ct = 0; ct < RT; ++ct) {
-        const rd4 zero = {0.0, 0.0, 0.0, 0.0};
+        const d4 zero = {0.0, 0.0, 0.0, 0.0};
         pw[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(-P, W[ct], zero, 0, 0, 0)[0];
       }
       pw[t] = pc ? P : pw[t];
@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(128, 2) ring_factor_kernel(
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int ct = 0; ct < RT; ++ct) acc[rt][ct] = rd4{0.0, 0.0, 0.0, 0.0};
+    for (int ct = 0; ct < RT; ++ct) acc[rt][ct] = d4{0.0, 0.0, 0.0, 0.0};
   const int count = side ? n - 1 - h : h;  // beads of this side, without the middle one
   load(side ? n - 1 : 0);
   for (int k = 0; k < count; ++k) {

@@ -6,10 +6,10 @@ layout (n, ndim, natom) column-major, one after another).  Its backward pass is 
 device adjoint (rp_ring_um), and the backward of that backward is the device
 forward-over-reverse Hessian-vector product (rp_ring_hvp), so first and second
 derivatives of any scalar built from the actions come from the hand-written kernels.
-A tensor on the GPU stays there: the library's device-memory entry points
-(rp_ring_set_x_device, rp_ring_um_device, rp_ring_hvp_device) copy it device to device, and
-the per-chain weighting is done by torch on the same device.  CPU tensors go through the
-host entry points.
+A tensor on the GPU stays there: the library's stream-ordered entry points
+(rp_ring_action_stream, rp_ring_hvp_stream and the per-chain weights and dot products) queue
+their kernels on torch's current stream, so nothing waits for the host.  CPU tensors, and
+potentials that live on the host, go through the host entry points.
 
 The Ring is the function's workspace: every evaluation loads x into its device coordinates
 and leaves them there (keep an optimised instanton in a Ring of its own).  The gradient made
@@ -18,9 +18,12 @@ evaluation in all.
 """
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import torch
 
+from . import _lib as L
 from .instanton import Ring
 
 
@@ -28,49 +31,78 @@ def _host(t: torch.Tensor) -> np.ndarray:
     return np.ascontiguousarray(t.detach().to("cpu", torch.float64).numpy())
 
 
-def _device(t: torch.Tensor) -> torch.Tensor:
-    """t as a contiguous float64 tensor on its GPU, every write to it complete."""
-    d = t.detach().to(torch.float64).contiguous()
-    torch.cuda.current_stream(d.device).synchronize()
-    return d
-
-
 def _flat(chains) -> torch.Tensor:
     return torch.from_numpy(np.concatenate([c.reshape(-1) for c in chains]))
 
 
-def _load_x(ring: Ring, x: torch.Tensor) -> None:
-    if x.is_cuda:
-        ring.set_x_device(_device(x).data_ptr())
-    else:
-        ring.set_x(ring.unpack(_host(x)))
+def _on_device(ring: Ring, x: torch.Tensor) -> bool:
+    return x.is_cuda and ring.pes.spec is not None  # a host potential has no spec
+
+
+def _f64(t: torch.Tensor) -> torch.Tensor:
+    return t.detach().to(torch.float64).contiguous()
+
+
+def _call(name: str, ring: Ring, like: torch.Tensor, *tensors) -> None:
+    """One stream-ordered library call on torch's current stream of the tensors' GPU."""
+    stream = torch.cuda.current_stream(like.device).cuda_stream
+    ptrs = [None if t is None else C.c_void_p(t.data_ptr()) for t in tensors]
+    L.check(getattr(L.lib(), name)(ring.h, *ptrs, C.c_void_p(stream)))
+
+
+def _vector(ring: Ring, t: torch.Tensor, what: str) -> torch.Tensor:
+    if t.numel() != int(ring.off[-1]):  # the kernels read the ring's chains, whatever the tensor holds
+        raise ValueError(f"ring_action: {what} has {t.numel()} values, the ring's chains {int(ring.off[-1])}")
+    return _f64(t)
 
 
 def _um(ring: Ring, x: torch.Tensor):
-    """(U_M per chain as a host array, the flat adjoint gradient on x's device, float64)"""
-    _load_x(ring, x)
-    if x.is_cuda:
-        g = torch.empty(x.numel(), dtype=torch.float64, device=x.device)
-        return ring.um_device(g.data_ptr()), g
+    """(U_M per chain, the flat adjoint gradient), float64 on x's device"""
+    if _on_device(ring, x):
+        xd = _vector(ring, x, "x")
+        e = torch.empty(ring.nchain, dtype=torch.float64, device=x.device)
+        g = torch.empty_like(xd)
+        _call("rp_ring_action_stream", ring, x, xd, e, g)
+        return e, g
+    ring.set_x(ring.unpack(_host(x)))
     g, e = ring.UMforceenergy()
-    return e, _flat(g)
+    return torch.as_tensor(e, device=x.device), _flat(g).to(x.device)
 
 
-def _hvp(ring: Ring, x: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
-    """H(x) v, flat, on x's device (float64)"""
-    _load_x(ring, x)
-    if x.is_cuda:
-        vd = _device(v)
-        hv = torch.empty_like(vd)
-        ring.hvp_device(vd.data_ptr(), hv.data_ptr())
+def _hvp(ring: Ring, x: torch.Tensor, v: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """w_c H_c(x) v of every chain, flat, on x's device (float64)"""
+    if _on_device(ring, x):
+        hv = torch.empty(v.numel(), dtype=torch.float64, device=x.device)
+        _call("rp_ring_hvp_stream", ring, x, _vector(ring, x, "x"), _vector(ring, v, "the vector"), _f64(w), hv)
         return hv
-    return _flat(ring.hvp(ring.unpack(_host(v))))
+    ring.set_x(ring.unpack(_host(x)))
+    hv = _flat(ring.hvp(ring.unpack(_host(v)))).to(x.device)
+    return _weighted(ring, x, w, hv)
 
 
 def _chain_index(ring: Ring, device) -> torch.Tensor:
     """the chain of every element of a flat coordinate vector"""
     sizes = torch.as_tensor(np.diff(ring.off), dtype=torch.int64)
     return torch.repeat_interleave(torch.arange(ring.nchain), sizes).to(device)
+
+
+def _weighted(ring: Ring, x: torch.Tensor, w: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
+    """w_c g over every chain (float64)"""
+    if _on_device(ring, x):
+        out = torch.empty_like(g)
+        _call("rp_ring_weight_stream", ring, x, _f64(w), g, out)
+        return out
+    return w.to(torch.float64)[_chain_index(ring, x.device)] * g
+
+
+def _dots(ring: Ring, x: torch.Tensor, a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """a . b of every chain (float64)"""
+    if _on_device(ring, x):
+        out = torch.empty(ring.nchain, dtype=torch.float64, device=x.device)
+        _call("rp_ring_dot_stream", ring, x, a, _vector(ring, b, "the vector"), out)
+        return out
+    out = torch.zeros(ring.nchain, dtype=torch.float64, device=x.device)
+    return out.index_add_(0, _chain_index(ring, x.device), a * b.to(torch.float64))
 
 
 class _Action(torch.autograd.Function):
@@ -80,7 +112,7 @@ class _Action(torch.autograd.Function):
         ctx.ring = ring
         ctx.g = g
         ctx.save_for_backward(x)
-        return torch.as_tensor(e, dtype=x.dtype, device=x.device)
+        return e.to(x.dtype)
 
     @staticmethod
     def backward(ctx, gout):
@@ -96,24 +128,19 @@ class _ActionGrad(torch.autograd.Function):
     def forward(ctx, x, w, ring, g=None):
         if g is None:
             _, g = _um(ring, x)
-        cix = _chain_index(ring, x.device)
         ctx.ring = ring
         ctx.save_for_backward(x, w)
         ctx.g = g
-        ctx.cix = cix
-        return (w.to(torch.float64)[cix] * g).to(x.dtype)
+        return _weighted(ring, x, w, g).to(x.dtype)
 
     @staticmethod
     def backward(ctx, gg):
         x, w = ctx.saved_tensors
-        ring, cix = ctx.ring, ctx.cix
-        # d/dx: sum_c w_c H_c gg_c (the HVP runs at the x of the forward pass)
-        hv = _hvp(ring, x, gg)
-        dx = w.to(torch.float64)[cix] * hv
-        # d/dw_c: grad U_c . gg_c
-        dw = torch.zeros(ring.nchain, dtype=torch.float64, device=x.device)
-        dw.index_add_(0, cix, ctx.g * gg.to(torch.float64))
-        return dx.to(x.dtype), dw.to(w.dtype), None, None
+        ring = ctx.ring
+        # d/dx: sum_c w_c H_c gg_c (the HVP runs at the x of the forward pass); d/dw_c: grad U_c . gg_c
+        dx = _hvp(ring, x, gg, w).to(x.dtype) if ctx.needs_input_grad[0] else None
+        dw = _dots(ring, x, ctx.g, gg).to(w.dtype) if ctx.needs_input_grad[1] else None
+        return dx, dw, None, None
 
 
 def ring_action(x: torch.Tensor, ring: Ring) -> torch.Tensor:
