@@ -53,6 +53,7 @@ struct BatchArgs {
   int first, count;   // polymers (batch order) of this launch's family
   int groups, pack;   // polymer groups per workgroup, polymers per group (launch_batch_kind)
   int ncu;            // compute units of the device
+  int helpers;        // kWide: helper waves
   uint32_t moved;     // EVB: K-chunks of 4 dofs with a dof that the wells' permutation moves
   int nsteps;
   int64_t step0, imin;
@@ -114,6 +115,8 @@ __host__ __device__ constexpr int wave_lds(int dt_tiles, int water_d) {
 // barriers, and the carries.
 struct BatchLds {
   int shared, group, e, tot, ex, row;
+  // kWide: the next step's source, after one group: 2 nt tiles x DC rows x 16 beads
+  __host__ __device__ int wide() const { return shared + group; }
 };
 __host__ __device__ inline BatchLds batch_lds(int n, int dt_tiles, int pes_lds, int water_d) {
   const int DC = 16 * dt_tiles, nt = batch_tiles(n), HP = 16 * nt;

@@ -172,6 +172,39 @@ __device__ __forceinline__ void noise_gemm(KernArgs& A, const Lane& L, double (&
     }
 }
 
+// The same for one tile and dof tile, both halves, into the step's source R[half][row][bead]
+// (kWide: helper waves)
+template <int DT>
+__device__ __forceinline__ void noise_gemm_to(KernArgs& A, const Lane& L, int tile, int dt, double* R) {
+  constexpr int DC = 16 * DT;
+  const int HP = 16 * L.nt;
+  const double* __restrict__ T0 = A.Tf;
+  const double* __restrict__ T1 = A.Tf + (size_t)HP * HP;
+  const int toff = L.g * HP + tile * 16 + L.m;
+  const double* z0 = L.Z + z_at<DC>(HP, 0, L.g, 16 * dt + L.m);
+  const double* z1 = z0 + HP * DC;
+  d4 P = {0.0, 0.0, 0.0, 0.0}, Q = P;
+  for (int kc = 0; kc < HP >> 2; kc += 4) {  // HP/4 is a multiple of 4: four chunks' loads at once
+    double b0[4], b1[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      b0[u] = (T0 + (size_t)(4 * (kc + u)) * HP)[toff];
+      b1[u] = (T1 + (size_t)(4 * (kc + u)) * HP)[toff];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      P = mfma_f64(z0[4 * (kc + u) * DC], b0[u], P);
+      Q = mfma_f64(z1[4 * (kc + u) * DC], b1[u], Q);
+    }
+  }
+  double* r = R + (tile * 2 * DC + 16 * dt + L.g) * 16 + L.m;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    r[4 * j * 16] = P[j] + Q[j];
+    r[(DC + 4 * j) * 16] = P[j] - Q[j];
+  }
+}
+
 // The wave's edge beads, for the neighbours of the adjacent tiles: slot tile + 1 holds
 // [lower m = 0 | lower m = 15 | upper m = 0 | upper m = 15]; slot 0 holds the fixed ends at
 // the places of m = 15, slot nt + 1 each half's last bead, where the halves meet.
@@ -465,7 +498,7 @@ __device__ __forceinline__ void water_kick(KernArgs& A, const Lane& L, double* X
 }
 
 // ---------------------------------------------------------------- the step kernel
-enum : int { kPile = 0, kLimit, kPack, kAndersen };
+enum : int { kPile = 0, kLimit, kPack, kAndersen, kWide };
 
 // One workgroup holds a.groups polymer groups of 2 nt waves each; a group is one polymer, or
 // (PACK, at most 8 dofs) a.pack polymers side by side in the 16 rows of an MFMA tile.  The
@@ -476,7 +509,12 @@ enum : int { kPile = 0, kLimit, kPack, kAndersen };
 // Langevin (time_step_pile): kick, normals -> LDS | T (lambda z) | linear step | carries.
 // Andersen (time_step_nm): [resample] A(dt/2), kick, A(dt/2).  Bars are barriers.
 //
-// MODE: kPile, kLimit (with dHdrlimit re-initialisations), kPack or kAndersen.
+// MODE: kPile, kLimit (with dHdrlimit re-initialisations), kPack, kAndersen, or kWide: kPile for
+// batches that leave most of the GPU idle, where a step's latency is what counts.  A.helpers
+// more waves make the next step's normals while the polymer's own waves take the kick, and the
+// next step's T (lambda z), into LDS, while those take the linear step.  us per 8-step launch of
+// 44 polymers of the 27-dof EVB, without and with: N = 32 89 and 64, 64 94 and 70, 128 128 and
+// 109; where it stops paying stands at launch_batch_kind.
 //
 // FP64 MFMAs and FP64 vector instructions share one pipe (256 workgroups of 8 waves: MFMA
 // alone 2.29 ms, as many FMAs alone 2.90 ms, both on different waves 5.29 ms), so the step's
@@ -486,13 +524,13 @@ template <int KIND, int MAXD, int DT, int MODE>
 __global__ void __launch_bounds__(DT > 2 ? 512 : 1024, DT > 2 ? 2 : 4) batch_kernel(BatchArgs) {
   extern __shared__ double S[];
   constexpr int DC = DT * 16;
-  constexpr bool LANGEVIN = MODE != kAndersen, PACK = MODE == kPack;
+  constexpr bool LANGEVIN = MODE != kAndersen, PACK = MODE == kPack, WIDE = MODE == kWide;
   KernArgs* const args = (KernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
   const int tid = threadIdx.x;
   // wave-uniform values, in SGPRs
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nwave = 2 * batch_tiles(args->N);
-  const int grp0 = wave / nwave, wave0 = wave - grp0 * nwave;
+  const int grp0 = WIDE ? 0 : wave / nwave, wave0 = wave - grp0 * nwave;  // kWide: helpers from nwave up
   const double* PL = S;  // EVB block (stage_evb_kick's layout), KIND == PES_EVB only
   // the lane's place, derived afresh from opaque copies in each phase of a step
   auto place = [&](KernArgs& A) __attribute__((always_inline)) -> Lane {
@@ -522,6 +560,11 @@ __global__ void __launch_bounds__(DT > 2 ? 512 : 1024, DT > 2 ? 2 : 4) batch_ker
     L.Row = base + B.row;
     L.own = wave_lds(DT, KIND == PES_WATER ? MAXD : 0);
     L.Own = base + B.ex + wv * L.own;
+    if (WIDE && wv >= 2 * L.nt) {  // a helper: no beads of its own
+      L.wtid -= L.wthreads;
+      L.wthreads = A.helpers * 64;
+      L.on = L.last = false;
+    }
     return L;
   };
   auto refresh = [&]() __attribute__((always_inline)) -> KernArgs& {
@@ -563,9 +606,10 @@ __global__ void __launch_bounds__(DT > 2 ? 512 : 1024, DT > 2 ? 2 : 4) batch_ker
     const Lane L = place(A);
     const int N = A.N, D = A.D;
     if constexpr (KIND == PES_EVB) stage_evb_kick<MAXD, DT>(A.pes.dp, S, A.moved, tid, blockDim.x);
-    for (int e = L.wtid; e < (int)(L.Tot - L.Z); e += L.wthreads) L.Z[e] = 0.0;  // Z and E
+    const int ngrp = WIDE ? blockDim.x : L.wthreads;
+    for (int e = WIDE ? tid : L.wtid; e < (int)(L.Tot - L.Z); e += ngrp) L.Z[e] = 0.0;  // Z and E
     __syncthreads();
-    for (int row = L.wtid; row < DC; row += L.wthreads) {
+    for (int row = WIDE ? tid : L.wtid; row < DC; row += ngrp) {
       const int pol = PACK ? row / D : 0, d = row - pol * D;
       const bool real = row < R;
       const double* pa = A.pdata + (size_t)(poly + (real ? pol : 0)) * 3 * DC;
@@ -669,13 +713,56 @@ __global__ void __launch_bounds__(DT > 2 ? 512 : 1024, DT > 2 ? 2 : 4) batch_ker
     linear_carry<DT>(A, place(A), aoa ? A.aoa : A.rot, x);
   };
 
+  // kWide: R, after the row tables; the step after the current one's source
+  double* const Rn = S + batch_lds(args->N, DT, KIND == PES_EVB ? evb_kick_lds_size(DC, args->moved) : 0,
+                                   KIND == PES_WATER ? args->D : 0).wide();
+  const int hw = WIDE ? wave - nwave : 0;  // helper number, negative in the polymer's own waves
+  auto helper_gemm = [&]() __attribute__((always_inline)) {
+    KernArgs& A = refresh();
+    const Lane L = place(A);
+    for (int u = hw; u < L.nt * DT; u += A.helpers) noise_gemm_to<DT>(A, L, u / DT, u % DT, Rn);
+  };
   __syncthreads();
+  if constexpr (WIDE) {  // the first step's source
+    if (hw >= 0) noise(false);
+    __syncthreads();
+    if (hw >= 0) helper_gemm();
+    __syncthreads();
+  }
   bool stop = false;
   const int64_t step0 = args->step0p ? *args->step0p : args->step0;
 #pragma unroll 1
   for (int s = 0; s < args->nsteps; ++s) {
     const int64_t ii = step0 + s + 1;  // the reference's step counter
-    if constexpr (LANGEVIN) {
+    if constexpr (WIDE) {
+      cur += need;
+      double r[DT][4];
+      if (hw >= 0) {
+        if (s + 1 < args->nsteps) noise(false);
+        __syncthreads();
+        if (s + 1 < args->nsteps) helper_gemm();
+        __syncthreads();
+        continue;
+      }
+      kick();
+      {
+        const Lane L = place(refresh());
+        const double* q = Rn + ((L.tile * 2 + L.h) * DC + L.g) * 16 + L.m;
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) r[d][j] = q[(16 * d + 4 * j) * 16];
+        publish_edges<DT>(L, x);
+        __syncthreads();
+      }
+      {
+        KernArgs& A = refresh();
+        linear_local<DT, true>(A, place(A), A.aoa, x, p, r);
+        __syncthreads();
+      }
+      KernArgs& A = refresh();
+      linear_carry<DT>(A, place(A), A.aoa, x);
+    } else if constexpr (LANGEVIN) {
       KernArgs& A = refresh();
       if (A.noise && cur + need > A.noise_cap) {
         stop = true;
@@ -779,6 +866,7 @@ __global__ void __launch_bounds__(DT > 2 ? 512 : 1024, DT > 2 ? 2 : 4) batch_ker
       }
     }
   }
+  if (WIDE && hw >= 0) return;
   check();
   if (!live) return;
   KernArgs& A = refresh();
@@ -830,8 +918,9 @@ __global__ void __launch_bounds__(DT > 2 ? 512 : 1024, DT > 2 ? 2 : 4) batch_ker
 //    rows of a tile as fit, but no more than leaves a workgroup for every CU.
 //  * Groups per workgroup, for plain Langevin, where every group of a workgroup runs the same
 //    steps: the fewest that keep a CU busiest by the score below, or a.waves (set_launch) over
-//    the tiles of a half; and no more than leaves a workgroup for every CU.  Otherwise one: resamples and re-initialisations fall
-//    differently.
+//    the tiles of a half; and no more than leaves a workgroup for every CU.  Otherwise one:
+//    resamples and re-initialisations fall differently.
+//  * kWide (plain Langevin, no wave budget set, few polymers): helper waves, one group.
 template <int KIND, int MAXD, int DT>
 int launch_batch_kind(const BatchArgs& a0, int thermostat, int npoly, hipStream_t s) {
   BatchArgs a = a0;
@@ -846,6 +935,17 @@ int launch_batch_kind(const BatchArgs& a0, int thermostat, int npoly, hipStream_
   const BatchLds B = batch_lds(a.N, DT, KIND == PES_EVB ? evb_kick_lds_size(DT * 16, a.moved) : 0,
                                KIND == PES_WATER ? a.D : 0);
   const int units = (npoly + a.pack - 1) / a.pack;
+  // kWide: enough helpers for the transform's tiles and the normals, a wave per 64 blocks of
+  // them, as far as a workgroup has waves left.  Both lines measured, us per 8-step launch
+  // without and with: past one workgroup per CU the helpers only take the kick's time (264
+  // polymers of the 27-dof EVB, N = 32: 91 and 113; 1012: 126 and 217); with fewer than half as
+  // many helpers as tiles they are waited for (44 polymers, N = 160, 6 helpers for 10 tiles: 167
+  // and 141; N = 192, 4 for 12: 176 and 180; 88 quartic, N = 224, 2 for 7: 92 and 120).
+  const int free_waves = (DT > 2 ? 8 : 16) - 2 * nt, tiles = nt * DT;
+  a.helpers = std::min(free_waves, std::max(tiles, (a.D * ((a.N >> 1) + 1) + 63) / 64));
+  const size_t wide_lds = (B.wide() + (size_t)2 * 16 * nt * 16 * DT) * sizeof(double);
+  const bool wide = plain && a.pack == 1 && !a.waves && units <= a.ncu &&
+                    2 * a.helpers >= tiles && wide_lds <= kBatchLds;
   constexpr int kWaves = DT > 2 ? 8 : 16;  // of a workgroup (launch bound)
   auto go = [&](auto kern) -> int {
     auto lds_of = [&](int g) { return (B.shared + (size_t)g * B.group) * sizeof(double); };
@@ -883,6 +983,14 @@ int launch_batch_kind(const BatchArgs& a0, int thermostat, int npoly, hipStream_
     if (a.pack > 1) return go(batch_kernel<KIND, MAXD, DT, kPack>);
   }
   if (a.limit >= 0.0) return go(batch_kernel<KIND, MAXD, DT, kLimit>);
+  if (wide) {
+    auto kern = batch_kernel<KIND, MAXD, DT, kWide>;
+    RP_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)wide_lds));
+    kern<<<units, (2 * nt + a.helpers) * 64, wide_lds, s>>>(a);
+    RP_HIP(hipGetLastError());
+    return RP_OK;
+  }
   return go(batch_kernel<KIND, MAXD, DT, kPile>);
 }
 

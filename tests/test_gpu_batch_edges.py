@@ -115,3 +115,19 @@ def test_polymers_sharing_a_workgroup(name, n, count):
     b.set_path(lampath, path)
     b.init_path()
     _check(sp, b, pols, [0, 1, 15, 16, 17, count // 2, count - 2, count - 1], 8, LANGEVIN, 1, lampath, path)
+
+
+@pytest.mark.parametrize("name,ns", [("evb", [2, 33, 159, 160, 161, 192, 193]), ("quartic", [223, 224, 225]),
+                                     ("water6", [64, 65])])
+@pytest.mark.parametrize("waves", [0, 8])
+def test_helper_waves(name, ns, waves):
+    """Few polymers take helper waves up to a bead count, unless a wave budget is set; several
+    launches of a few steps each hand the stream position over between them."""
+    sp = SPECS[name]()
+    lampath, path = _path(sp)
+    pols = _polymers(sp, path, ns, 2)
+    b = Batch(Pes(sp), sp.mass, pols, TAU, DT, GAMMA, seed=SEED)
+    b.set_path(lampath, path)
+    b.set_launch(3, waves)
+    b.init_path()
+    _check(sp, b, pols, range(len(pols)), 8, LANGEVIN, 1, lampath, path)
