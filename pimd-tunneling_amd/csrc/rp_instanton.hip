@@ -158,6 +158,110 @@ __device__ __forceinline__ void each(F&& f) {
   }
 }
 
+// P the spring tridiagonal of rp_ring_set_preconditioner: v <- P^-1 v, and this lane's part of
+// y.P^-1.y, for one chain's vectors (dof columns of n beads, the ring layout).  A wave solves
+// one dof column: each lane takes a run of at most kPcRun consecutive beads, and both Thomas
+// sweeps -- the forward d'_i = alpha_i d'_{i-1} + inv_i r_i and the backward
+// x_i = alpha_i x_{i+1} + d'_i -- are affine recurrences, so a lane composes its run into one
+// affine map, a wave scan of those maps gives each lane its incoming value, and the lane
+// replays its run.  P = L D L^T with pivots D_i = 1/inv_i, so y.P^-1.y = sum d'_i^2 / inv_i
+// takes the forward sweep of y alone, and no scratch vector.  LDS: v is in LDS, element j at
+// pc_skew(j); else it is the argument.  The callers bracket it with barriers.
+// runs of 8 beads start 9 doubles apart: a lane's run and its neighbours' miss each other's banks
+__host__ __device__ constexpr int pc_skew(int j) { return j + (j >> 3); }
+
+__device__ __forceinline__ double pc_scan_up(double A, double B) {  // value entering this lane
+  const int lane = threadIdx.x & 63;
+  for (int o = 1; o < 64; o <<= 1) {  // inclusive scan: lanes below come first
+    const double A2 = __shfl_up(A, o), B2 = __shfl_up(B, o);
+    if (lane >= o) {
+      B = A * B2 + B;
+      A = A * A2;
+    }
+  }
+  const double x = __shfl_up(B, 1);
+  return lane == 0 ? 0.0 : x;
+}
+
+template <bool LDS>
+__device__ __forceinline__ double& pc_at(double* v, int j) {
+  extern __shared__ double V[];
+  if constexpr (LDS) return V[pc_skew(j)];
+  return v[j];
+}
+
+template <bool LDS>
+__device__ __forceinline__ double pc_solve(double* v, const double* y, int n, int D, int ndim,
+                           const double* __restrict__ tab) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int run = (n + 63) >> 6, n64 = run * 64;
+  const int i0 = lane * run;
+  double ypy = 0.0;
+  for (int col = wave; col < D; col += kLbWaves) {
+    const double* __restrict__ tinv = tab + (size_t)(col / ndim) * n64 * 2 + lane;
+    const double* __restrict__ tal = tinv + n64;
+    const int b0 = col * n + i0;
+    double w[kPcRun];
+    auto compose = [&](const auto& load) __attribute__((always_inline)) {  // w and the run's map
+      double A = 1.0, B = 0.0;
+#pragma unroll
+      for (int q = 0; q < kPcRun; ++q) {
+        w[q] = 0.0;
+        if (q < run) {
+          const double al = tal[q * 64];
+          w[q] = i0 + q < n ? load(b0 + q) : 0.0;
+          B = al * B + tinv[q * 64] * w[q];
+          A = al * A;
+        }
+      }
+      return pc_scan_up(A, B);
+    };
+    if (y) {
+      double x = compose([&](int j) __attribute__((always_inline)) { return y[j]; });
+#pragma unroll
+      for (int q = 0; q < kPcRun; ++q)
+        if (q < run) {
+          const double inv = tinv[q * 64];
+          x = tal[q * 64] * x + inv * w[q];
+          ypy += i0 + q < n ? x * x / inv : 0.0;
+        }
+    }
+    // forward sweep
+    double x = compose([&](int j) __attribute__((always_inline)) { return pc_at<LDS>(v, j); });
+#pragma unroll
+    for (int q = 0; q < kPcRun; ++q)
+      if (q < run) {
+        x = tal[q * 64] * x + tinv[q * 64] * w[q];
+        w[q] = i0 + q < n ? x : 0.0;  // d'_i
+      }
+    // backward sweep
+    double A = 1.0, B = 0.0;
+#pragma unroll
+    for (int q = kPcRun - 1; q >= 0; --q)
+      if (q < run) {
+        const double al = tal[q * 64];
+        B = al * B + w[q];
+        A = al * A;
+      }
+    for (int o = 1; o < 64; o <<= 1) {  // inclusive scan: lanes above come first
+      const double A2 = __shfl_down(A, o), B2 = __shfl_down(B, o);
+      if (lane + o < 64) {
+        B = A * B2 + B;
+        A = A * A2;
+      }
+    }
+    x = __shfl_down(B, 1);
+    if (lane == 63) x = 0.0;
+#pragma unroll
+    for (int q = kPcRun - 1; q >= 0; --q)
+      if (q < run) {
+        x = tal[q * 64] * x + w[q];
+        if (i0 + q < n) pc_at<LDS>(v, b0 + q) = x;
+      }
+  }
+  return ypy;
+}
+
 // d = -H g by the two-loop recursion, the descent check, and the first trial point.  Each
 // pass over the chain fuses one correction's update with the next correction's dot product,
 // so the recursion reads the direction 2k + 1 times for k pairs.
@@ -165,14 +269,18 @@ __device__ __forceinline__ void each(F&& f) {
 // j = threadIdx.x + q kLbThreads in slot q) through the 2k passes of the recursion, which then
 // read only the pairs, with every load of a pass in flight at once; the arithmetic and its
 // order are those of the streaming form (P = 0), which keeps D in HBM for longer chains.
-template <int P>
+// PC: the initial matrix is gamma P^-1 (gamma = s.y / y.P^-1.y of the newest pair; the first
+// and the reset directions are -P^-1 g, tried at unit step); the solves take dof columns, so
+// between the loops the vector goes through LDS (P <= 16) or HBM.
+template <int P, bool PC>
 __global__ void __launch_bounds__(kLbThreads) lb_direction_kernel(LbArgs A) {
+  constexpr bool LDS = PC && P > 0 && P <= 16;
   __shared__ double red[kLbWaves];
   __shared__ double alpha[kMaxM + 1];
   const int c = blockIdx.x;
   if (A.st[c].op != OP_DIRECTION) return;  // uniform over the workgroup
   const int k = A.st[c].count, head = A.st[c].head;
-  const double gam = A.st[c].gam, ginf = A.st[c].ginf;
+  const double gam = PC ? 1.0 : A.st[c].gam, ginf = A.st[c].ginf;
   const double* rho = A.rho + (int64_t)c * (kMaxM + 1);
   const int64_t base = A.off[c], tot = A.tot;
   const int L = A.n[c] * A.D;
@@ -187,14 +295,31 @@ __global__ void __launch_bounds__(kLbThreads) lb_direction_kernel(LbArgs A) {
   auto Sv = [=](int i) { return S0 + (int64_t)slot(i) * tot; };
   auto Yv = [=](int i) { return Y0 + (int64_t)slot(i) * tot; };
   double part = 0.0, a0 = 1.0;
-  if (k == 0) {
-    a0 = fmin(1.0, 1.0 / fmax(ginf, 1e-300));
+  // PC: the vector's place during a solve (LDS: pc_skew(L) doubles of it), and the solve
+  auto W = [&](int j) __attribute__((always_inline)) -> double& { return pc_at<LDS>(D, j); };
+  auto solve = [&](const double* y) __attribute__((always_inline)) {
+    __syncthreads();
+    const double ypy = pc_solve<LDS>(D, y, A.n[c], A.D, A.ndim, A.pctab + A.pcoff[c]);
+    __syncthreads();
+    return ypy;
+  };
+  // d = -g, PC d = -P^-1 g: the first direction and the fallback of a non-descent one
+  auto steepest = [&]() __attribute__((always_inline)) {
+    if constexpr (PC) {
+      for (int j = threadIdx.x; j < L; j += kLbThreads) W(j) = -G[j];
+      solve(nullptr);
+    }
+    a0 = PC ? 1.0 : fmin(1.0, 1.0 / fmax(ginf, 1e-300));
+    part = 0.0;
     for (int j = threadIdx.x; j < L; j += kLbThreads) {
-      const double v = -G[j];
+      const double v = PC ? W(j) : -G[j];
       D[j] = v;
       part += G[j] * v;
       XT[j] = X[j] + a0 * v;
     }
+  };
+  if (k == 0) {
+    steepest();
   } else if constexpr (P > 0) {
     // loads at a clamped index and selects, no branch per element: the loads of a chunk
     // issue back to back.  Slots past the chain end keep d = 0 and add nothing.  The thread
@@ -256,8 +381,23 @@ __global__ void __launch_bounds__(kLbThreads) lb_direction_kernel(LbArgs A) {
           const double w = y * v + part;
           d[q] = in(q) ? v : d[q];
           part = in(q) ? w : part;
+          if constexpr (PC)
+            if (in(q)) W(j) = v;
         });
       }
+    }
+    if constexpr (PC) {
+      const double scale = 1.0 / (rho[slot(k - 1)] * lb_sum(solve(Yv(k - 1)), red));
+      const double* Yp = Yv(0);
+      part = 0.0;
+      fresh();
+      each<0, P>([&](int q) __attribute__((always_inline)) {
+        const int j = at(q);
+        const double v = scale * W(j);
+        const double w = Yp[j] * v + part;
+        d[q] = in(q) ? v : d[q];
+        part = in(q) ? w : part;
+      });
     }
     __syncthreads();  // alpha[] complete before the forward loop reads it
     for (int i = 0; i < k; ++i) {
@@ -317,6 +457,16 @@ __global__ void __launch_bounds__(kLbThreads) lb_direction_kernel(LbArgs A) {
         }
       }
     }
+    if constexpr (PC) {
+      const double scale = 1.0 / (rho[slot(k - 1)] * lb_sum(solve(Yv(k - 1)), red));
+      const double* Yp = Yv(0);
+      part = 0.0;
+      for (int j = threadIdx.x; j < L; j += kLbThreads) {
+        const double d = scale * D[j];
+        D[j] = d;
+        part += Yp[j] * d;
+      }
+    }
     __syncthreads();  // alpha[] complete before the forward loop reads it
     for (int i = 0; i < k; ++i) {
       const double coef = alpha[i] - rho[slot(i)] * lb_sum(part, red);
@@ -343,14 +493,7 @@ __global__ void __launch_bounds__(kLbThreads) lb_direction_kernel(LbArgs A) {
   double dg0 = lb_sum(part, red);
   const bool reset = !(dg0 < 0.0);  // not a descent direction: steepest descent, no history
   if (reset && k > 0) {
-    a0 = fmin(1.0, 1.0 / fmax(ginf, 1e-300));
-    part = 0.0;
-    for (int j = threadIdx.x; j < L; j += kLbThreads) {
-      const double v = -G[j];
-      D[j] = v;
-      part += G[j] * v;
-      XT[j] = X[j] + a0 * v;
-    }
+    steepest();
     dg0 = lb_sum(part, red);
   }
   if (threadIdx.x == 0) {
@@ -368,194 +511,6 @@ __global__ void __launch_bounds__(kLbThreads) lb_direction_kernel(LbArgs A) {
     t.prev_is_g = 1;
     t.nls = 0;
     t.a_cur = a0;
-    t.op = OP_NONE;
-    A.st[c] = t;
-  }
-}
-
-// v <- P^-1 v for one chain's vector in HBM (dof columns of n beads, the ring layout), P the
-// spring tridiagonal of rp_ring_set_preconditioner.  A wave solves one dof column: each lane
-// takes a run of at most kPcRun consecutive beads, and both Thomas sweeps -- the forward
-// d'_i = alpha_i d'_{i-1} + inv_i r_i and the backward x_i = alpha_i x_{i+1} + d'_i -- are
-// affine recurrences, so a lane composes its run into one affine map, a wave scan of those
-// maps (xor-free shuffles up / down) gives each lane its incoming value, and the lane
-// replays its run.  The callers bracket it with barriers.
-constexpr int kPcRun = 16;  // beads per lane: n <= 64 kPcRun = 1024
-__device__ void pc_solve(double* v, int n, int D, int ndim, const double* __restrict__ tab) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int run = (n + 63) >> 6;
-  const int i0 = lane * run;
-  for (int col = wave; col < D; col += kLbWaves) {
-    const double* t = tab + (size_t)(col / ndim) * n * 2;
-    double* vc = v + (size_t)col * n;
-    double w[kPcRun];
-    // forward sweep
-    double A = 1.0, B = 0.0;
-#pragma unroll
-    for (int q = 0; q < kPcRun; ++q) {
-      const int i = i0 + q;
-      w[q] = 0.0;
-      if (q < run && i < n) {
-        const double al = t[2 * i + 1];
-        w[q] = vc[i];
-        B = al * B + t[2 * i] * w[q];
-        A = al * A;
-      }
-    }
-    for (int o = 1; o < 64; o <<= 1) {  // inclusive scan: lanes below come first
-      const double A2 = __shfl_up(A, o), B2 = __shfl_up(B, o);
-      if (lane >= o) {
-        B = A * B2 + B;
-        A = A * A2;
-      }
-    }
-    double x = __shfl_up(B, 1);
-    if (lane == 0) x = 0.0;
-#pragma unroll
-    for (int q = 0; q < kPcRun; ++q) {
-      const int i = i0 + q;
-      if (q < run && i < n) {
-        x = t[2 * i + 1] * x + t[2 * i] * w[q];
-        w[q] = x;  // d'_i
-      }
-    }
-    // backward sweep
-    A = 1.0;
-    B = 0.0;
-#pragma unroll
-    for (int q = kPcRun - 1; q >= 0; --q) {
-      const int i = i0 + q;
-      if (q < run && i < n) {
-        const double al = t[2 * i + 1];
-        B = al * B + w[q];
-        A = al * A;
-      }
-    }
-    for (int o = 1; o < 64; o <<= 1) {  // inclusive scan: lanes above come first
-      const double A2 = __shfl_down(A, o), B2 = __shfl_down(B, o);
-      if (lane + o < 64) {
-        B = A * B2 + B;
-        A = A * A2;
-      }
-    }
-    x = __shfl_down(B, 1);
-    if (lane == 63) x = 0.0;
-#pragma unroll
-    for (int q = kPcRun - 1; q >= 0; --q) {
-      const int i = i0 + q;
-      if (q < run && i < n) {
-        x = t[2 * i + 1] * x + w[q];
-        vc[i] = x;
-      }
-    }
-  }
-}
-
-// The direction of the preconditioned search: d = -H g by the two-loop recursion with the
-// initial matrix gamma P^-1 (gamma = s.y / y.P^-1.y of the newest pair; the first and the
-// reset directions are -P^-1 g, tried at unit step).  Plain passes over HBM: with the
-// preconditioner a search takes tens of iterations where the unpreconditioned one takes
-// thousands, so this kernel is not the one tuned for bandwidth.  XT serves as the scratch
-// vector of the y.P^-1.y solve before it receives the trial point.
-__global__ void __launch_bounds__(kLbThreads) lb_direction_pc_kernel(LbArgs A) {
-  __shared__ double red[kLbWaves];
-  __shared__ double alpha[kMaxM + 1];
-  const int c = blockIdx.x;
-  if (A.st[c].op != OP_DIRECTION) return;  // uniform over the workgroup
-  const int k = A.st[c].count, head = A.st[c].head;
-  const double* rho = A.rho + (int64_t)c * (kMaxM + 1);
-  const int64_t base = A.off[c], tot = A.tot;
-  const int n = A.n[c], L = n * A.D;
-  const int m1 = A.m + 1;
-  const double* tab = A.pctab + A.pcoff[c];
-  double* D = A.Dv + base;
-  const double* G = A.G + base;
-  const double* X = A.X + base;
-  double* XT = A.XT + base;
-  const double* S0 = A.S + base;
-  const double* Y0 = A.Y + base;
-  auto slot = [=](int i) { return (head + i) % m1; };
-  auto Sv = [=](int i) { return S0 + (int64_t)slot(i) * tot; };
-  auto Yv = [=](int i) { return Y0 + (int64_t)slot(i) * tot; };
-  // d = -P^-1 g: the first direction and the fallback of a non-descent one
-  auto steepest = [&]() -> double {
-    for (int j = threadIdx.x; j < L; j += kLbThreads) D[j] = -G[j];
-    __syncthreads();
-    pc_solve(D, n, A.D, A.ndim, tab);
-    __syncthreads();
-    double part = 0.0;
-    for (int j = threadIdx.x; j < L; j += kLbThreads) {
-      part += G[j] * D[j];
-      XT[j] = X[j] + D[j];
-    }
-    return lb_sum(part, red);
-  };
-  double dg0;
-  bool reset = false;
-  if (k == 0) {
-    dg0 = steepest();
-  } else {
-    // backward loop: q = g - sum alpha_i y_i, q in D
-    for (int j = threadIdx.x; j < L; j += kLbThreads) D[j] = G[j];
-    for (int i = k - 1; i >= 0; --i) {
-      const double* Si = Sv(i);
-      const double* Yi = Yv(i);
-      double part = 0.0;
-      for (int j = threadIdx.x; j < L; j += kLbThreads) part += Si[j] * D[j];
-      const double al = rho[slot(i)] * lb_sum(part, red);
-      if (threadIdx.x == 0) alpha[i] = al;
-      for (int j = threadIdx.x; j < L; j += kLbThreads) D[j] -= al * Yi[j];
-    }
-    // gamma = s.y / y.P^-1.y of the newest pair, with XT as the solve's scratch
-    const double* Yk = Yv(k - 1);
-    for (int j = threadIdx.x; j < L; j += kLbThreads) XT[j] = Yk[j];
-    __syncthreads();
-    pc_solve(XT, n, A.D, A.ndim, tab);
-    pc_solve(D, n, A.D, A.ndim, tab);
-    __syncthreads();
-    double part = 0.0;
-    for (int j = threadIdx.x; j < L; j += kLbThreads) part += Yk[j] * XT[j];
-    const double ypy = lb_sum(part, red);
-    const double gam = (1.0 / rho[slot(k - 1)]) / ypy;
-    for (int j = threadIdx.x; j < L; j += kLbThreads) D[j] *= gam;
-    // forward loop: r += s_i (alpha_i - rho_i y_i.r)
-    for (int i = 0; i < k; ++i) {
-      const double* Si = Sv(i);
-      const double* Yi = Yv(i);
-      part = 0.0;
-      for (int j = threadIdx.x; j < L; j += kLbThreads) part += Yi[j] * D[j];
-      const double coef = alpha[i] - rho[slot(i)] * lb_sum(part, red);
-      for (int j = threadIdx.x; j < L; j += kLbThreads) D[j] += coef * Si[j];
-    }
-    part = 0.0;
-    for (int j = threadIdx.x; j < L; j += kLbThreads) {
-      const double d = -D[j];
-      D[j] = d;
-      part += G[j] * d;
-      XT[j] = X[j] + d;
-    }
-    dg0 = lb_sum(part, red);
-    reset = !(dg0 < 0.0);  // not a descent direction: the preconditioned steepest descent
-    if (reset) {
-      __syncthreads();
-      dg0 = steepest();
-    }
-  }
-  if (threadIdx.x == 0) {
-    LbChain t = A.st[c];
-    if (reset) {
-      t.count = 0;
-      t.head = 0;
-    }
-    t.dg0 = dg0;
-    t.f0 = t.f;
-    t.phase = LS_BRACKET;
-    t.a_prev = 0.0;
-    t.f_prev = t.f;
-    t.dg_prev = dg0;
-    t.prev_is_g = 1;
-    t.nls = 0;
-    t.a_cur = 1.0;
     t.op = OP_NONE;
     A.st[c] = t;
   }
@@ -673,7 +628,7 @@ __global__ void __launch_bounds__(kLbThreads) lb_feed_kernel(LbArgs A) {
       pg = fmax(pg, fabs(ga));
       X[j] = xa;
       G[j] = ga;
-      XT[j] = xa;
+      if (!cur) XT[j] = xa;
     }
     const double sy = lb_sum(psy, red);
     const double yy = lb_sum(pyy, red);
@@ -758,12 +713,27 @@ extern "C" int rp_instanton(rp_ring* r, double pgtol, double factr, int m, int m
   // direction kernel by the longest chain's elements per thread
   const int nmax = *std::max_element(ring_n(r).begin(), ring_n(r).end());
   const int per = (nmax * rb.D + kLbThreads - 1) / kLbThreads;
-  auto direction = A.pctab ? lb_direction_pc_kernel
-                 : per <= 8 ? lb_direction_kernel<8> : per <= 16 ? lb_direction_kernel<16>
-                 : per <= 28 ? lb_direction_kernel<28> : lb_direction_kernel<0>;
+  const bool pre = A.pctab != nullptr;
+  // Preconditioned, us per launch of 128 chains of the 27-dof EVB, averaged over a search's
+  // first ten iterations: a vector streamed through HBM in every pass and P^-1 y written out
+  // 117 (n = 256), 242 (512); in registers 43 and 77, where what is left is the pairs' bytes at
+  // what one CU draws from beyond its L2 (10 us a pair for 13824 coordinates; more loads in
+  // flight change nothing).  At 28 elements per thread the registers spill, and streaming is as
+  // good: 197 and 173 (n = 640), 297 and 311 (1024).
+  void (*direction)(LbArgs) =
+      pre ? (per <= 8 ? lb_direction_kernel<8, true> : per <= 16 ? lb_direction_kernel<16, true>
+                                                                 : lb_direction_kernel<0, true>)
+          : (per <= 8    ? lb_direction_kernel<8, false>
+             : per <= 16 ? lb_direction_kernel<16, false>
+             : per <= 28 ? lb_direction_kernel<28, false>
+                         : lb_direction_kernel<0, false>);
+  const size_t lds = pre && per <= 16 ? (pc_skew(nmax * rb.D) + 1) * sizeof(double) : 0;
+  if (lds)
+    RP_HIP(hipFuncSetAttribute((const void*)direction,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   RP_REQUIRE(!A.pctab || nmax <= 64 * kPcRun,
              "rp_instanton: the preconditioner takes chains of at most %d beads", 64 * kPcRun);
-  direction<<<nc, kLbThreads, 0, rb.s>>>(A);
+  direction<<<nc, kLbThreads, lds, rb.s>>>(A);
   RP_HIP(hipGetLastError());
   std::vector<int> hs(nc);
   const long cap = maxiter > 0 ? (long)maxiter * kMaxLS + 1 : kMaxRounds;
@@ -780,7 +750,7 @@ extern "C" int rp_instanton(rp_ring* r, double pgtol, double factr, int m, int m
     if ((rc = ring_eval(r, true))) return rc;
     lb_feed_kernel<<<nc, kLbThreads, 0, rb.s>>>(A);
     RP_HIP(hipGetLastError());
-    direction<<<nc, kLbThreads, 0, rb.s>>>(A);
+    direction<<<nc, kLbThreads, lds, rb.s>>>(A);
     RP_HIP(hipGetLastError());
   }
   if (capped) {

@@ -26,8 +26,12 @@ struct RingBufs {
   hipStream_t s;
 };
 RingBufs ring_bufs(rp_ring* r);
-// the instanton search's preconditioner (rp_ring_set_preconditioner): Thomas coefficients
-// {1/denominator, alpha} per (chain, atom, bead) from tab + off[chain], or tab = nullptr (off)
+// the instanton search's preconditioner (rp_ring_set_preconditioner): Thomas coefficients per
+// (chain, atom) from tab + off[chain], [1/denominator | alpha], or tab = nullptr (off).  A lane
+// of the solve takes `run` consecutive beads; bead lane run + q is entry 64 q + lane, so that
+// a wave's loads are contiguous; the entries past the chain's end are {0, 0}.
+constexpr int kPcRun = 16;  // beads per lane at most: n <= 64 kPcRun = 1024
+inline int pc_run(int n) { return (n + 63) >> 6; }
 struct RingPc {
   const double* tab;
   const int64_t* off;

@@ -1158,22 +1158,23 @@ extern "C" int rp_ring_set_preconditioner(rp_ring* r, double sigma) {
   int64_t tot = 0;
   for (int c = 0; c < r->nchain; ++c) {
     pcoff[c] = tot;
-    tot += (int64_t)r->natom * r->n[c] * 2;
+    tot += (int64_t)r->natom * pc_run(r->n[c]) * 64 * 2;
   }
-  std::vector<double> tab(tot);
+  std::vector<double> tab(tot, 0.0);
   for (int c = 0; c < r->nchain; ++c) {
-    const int n = r->n[c];
+    const int n = r->n[c], run = pc_run(n);
     for (int at = 0; at < r->natom; ++at) {
       const double k = r->hmass[at] / (r->betan[c] * r->betan[c]), off = -k;
-      double* t = tab.data() + pcoff[c] + (int64_t)at * n * 2;
+      double* t = tab.data() + pcoff[c] + (int64_t)at * run * 64 * 2;
       double cp = 0.0;  // c'_{i-1}
       for (int i = 0; i < n; ++i) {
         const bool end = !r->fixedends && (i == 0 || i == n - 1);
         const double diag = (end ? k : 2.0 * k) + r->pc_sigma;
         const double inv = 1.0 / (diag - off * cp);
         cp = off * inv;
-        t[2 * i] = inv;
-        t[2 * i + 1] = -cp;
+        const int e = i % run * 64 + i / run;
+        t[e] = inv;
+        t[run * 64 + e] = -cp;
       }
     }
   }
