@@ -37,6 +37,7 @@ typedef const __attribute__((address_space(4))) BatchArgs KernArgs;
 // the middle bead of an odd chain).
 struct Lane {
   double *Z, *E, *Tot, *Row, *Own;
+  int N;               // beads of the chain
   int h, tile, nt;     // wave-uniform: the wave's half and bead tile, tiles per half
   int own;             // doubles of a wave's own area
   int wtid, wthreads;  // this thread among the group's threads
@@ -235,17 +236,23 @@ __device__ __forceinline__ void linear_local(KernArgs& A, const Lane& L,
                                              const __attribute__((address_space(4))) Linear& C,
                                              double (&x)[DT][4], double (&p)[DT][4], const double (&r)[DT][4]) {
   constexpr int DC = 16 * DT;
-  const double w = (double)(L.l + 1), v = (double)(A.N - L.l), wf = w * A.iG;
+  const double w = (double)(L.l + 1), v = (double)(L.N - L.l), wf = w * A.iG;
   const double* ea = L.E + (2 * L.h + 1) * DC + L.g;  // this half's fixed end
   const double* eb = L.E + (3 - 2 * L.h) * DC + L.g;  // the other one
-  const double* meet = L.E + ((L.nt + 1) * 4 + (L.h ^ 1)) * DC + L.g;
-  // the edge slot a lane's row move has no source for: the tile before (m = 0) or after
-  const double* en = L.E + ((L.m == 0 ? L.tile * 4 + 1 : (L.tile + 2) * 4) + 2 * L.h) * DC + L.g;
+  // Where a lane's row moves have no source: the bead before the tile (m = 0), the one after it
+  // (m = 15), or, for the half's last bead, the other half's, which the lanes past it also hold
+  // and so pass to a last bead with m < 15.  One read for every lane, and the tile's sums go out
+  // once per dof tile: a branch per element leaves each element waiting for its own LDS reads
+  // (8 steps of the 27-dof EVB: 44 polymers, N = 32, 63 us with branches, 57 without; 5632,
+  // N = 128, 2.12 and 2.07 ms).
+  const double* en = L.E + (L.m == 0               ? L.tile * 4 + 1 + 2 * L.h
+                            : L.last || !L.on ? (L.nt + 1) * 4 + (L.h ^ 1)
+                                                   : (L.tile + 2) * 4 + 2 * L.h) * DC + L.g;
   const double* Row = L.Row + L.g;
-  const bool edge = L.m == 0 || L.m == 15;
   double* tot = L.Tot + (L.tile * 2 + L.h) * DC * 2 + 2 * L.g + (L.m ? 0 : 1);
   static_for<DT>([&](auto Dx) __attribute__((always_inline)) {
     constexpr int d = decltype(Dx)::value;
+    double sum[4];
     static_for<4>([&](auto J) __attribute__((always_inline)) {
       constexpr int j = decltype(J)::value, row = 16 * d + 4 * j;
       const double xi = x[d][j], pi = p[d][j];
@@ -254,24 +261,26 @@ __device__ __forceinline__ void linear_local(KernArgs& A, const Lane& L,
       // neighbours l - 1 and l + 1; the halves meet at their last beads
       const double e = en[row];
       const double prev = row_mov<kShr + 1>(e, xi);
-      double next = row_mov<kShl + 1>(e, xi);
-      next = L.last ? meet[row] : next;
+      const double next = row_mov<kShl + 1>(e, L.on ? xi : e);
       // K^-1 of the tile's own beads
       const double u = L.on ? (NOISE ? fma(C.cu, pi, ri) : pi) : 0.0;
       const double f = v * u;
       const double a = row_prefix(w * u), b = row_suffix(f);
-      if (edge) tot[2 * row] = L.m ? a : b;  // prefix total in lane 15, suffix total in lane 0
+      sum[j] = L.m ? a : b;  // prefix total in lane 15, suffix total in lane 0
       const double s = v * a + w * (b - f);
       const double xa = ea[row], xeq = xa + (eb[row] - xa) * wf;
       double xn = xeq + C.cy * (xi - xeq) + (C.gx * Row[RW_IM * DC + row]) * s;
       double pn = C.cp * pi - (C.ck * Row[RW_M * DC + row]) * ((xi - prev) + (xi - next));
       if constexpr (NOISE) pn += C.cr * ri;
-      // computed here: sunk past the next element's branches they would hold its inputs
+      // computed here: sunk past the next element's they would hold its inputs
       asm volatile("" : "+v"(xn), "+v"(pn));
       x[d][j] = xn;
       p[d][j] = pn;
       if constexpr (j & 1) __builtin_amdgcn_sched_barrier(0);  // two elements at a time: bounded registers
     });
+    if (L.m == 0 || L.m == 15)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) tot[2 * (16 * d + 4 * j)] = sum[j];
   });
 }
 
@@ -304,7 +313,7 @@ __device__ __forceinline__ void linear_carry(KernArgs& A, const Lane& L,
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
-  const double w = (double)(L.l + 1), v = (double)(A.N - L.l);
+  const double w = (double)(L.l + 1), v = (double)(L.N - L.l);
   const double* Row = L.Row + L.g;
   const double* k = car + 2 * L.g;
 #pragma unroll
@@ -514,7 +523,7 @@ enum : int { kPile = 0, kLimit, kPack, kAndersen, kWide };
 // more waves make the next step's normals while the polymer's own waves take the kick, and the
 // next step's T (lambda z), into LDS, while those take the linear step.  us per 8-step launch of
 // 44 polymers of the 27-dof EVB, without and with: N = 32 89 and 64, 64 94 and 70, 128 128 and
-// 109; where it stops paying stands at launch_batch_kind.
+// 109 (57, 65 and 105 since linear_local lost its branches); where it stops paying stands at launch_batch_kind.
 //
 // FP64 MFMAs and FP64 vector instructions share one pipe (256 workgroups of 8 waves: MFMA
 // alone 2.29 ms, as many FMAs alone 2.90 ms, both on different waves 5.29 ms), so the step's
@@ -531,16 +540,22 @@ __global__ void __launch_bounds__(DT > 2 ? 512 : 1024, DT > 2 ? 2 : 4) batch_ker
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nwave = 2 * batch_tiles(args->N);
   const int grp0 = WIDE ? 0 : wave / nwave, wave0 = wave - grp0 * nwave;  // kWide: helpers from nwave up
+  // all that a lane's place needs of the arguments, in two SGPRs: no phase waits for a scalar
+  // load before it can address LDS
+  const int nbeads = args->N;
+  const int nshared = batch_lds(nbeads, DT, KIND == PES_EVB ? evb_kick_lds_size(DC, args->moved) : 0,
+                                KIND == PES_WATER ? args->D : 0).shared;
   const double* PL = S;  // EVB block (stage_evb_kick's layout), KIND == PES_EVB only
   // the lane's place, derived afresh from opaque copies in each phase of a step
   auto place = [&](KernArgs& A) __attribute__((always_inline)) -> Lane {
     int lane = tid & 63, grp = grp0, wv = wave0;
     asm volatile("" : "+v"(lane));
     asm volatile("" : "+s"(grp), "+s"(wv));
-    const int N = A.N;
-    const BatchLds B = batch_lds(N, DT, KIND == PES_EVB ? evb_kick_lds_size(DC, A.moved) : 0,
-                                 KIND == PES_WATER ? A.D : 0);
+    int N = nbeads, shared = nshared;
+    asm volatile("" : "+s"(N), "+s"(shared));
+    const BatchLds B = batch_lds(N, DT, shared, KIND == PES_WATER ? MAXD : 0);
     Lane L;
+    L.N = N;
     L.nt = batch_tiles(N);
     L.h = wv & 1;
     L.tile = wv >> 1;
@@ -825,8 +840,7 @@ __global__ void __launch_bounds__(DT > 2 ? 512 : 1024, DT > 2 ? 2 : 4) batch_ker
             constexpr int d = decltype(Dx)::value, j = decltype(J)::value;
             contr -= L.Row[RW_MDB * DC + row] * x[d][j];
           });
-          contr += __shfl_xor(contr, 16);
-          contr += __shfl_xor(contr, 32);
+          contr = sum_groups(contr);
         }
         if constexpr (MODE == kLimit) {
           // dHdrlimit: a step whose term is too large is not counted and the path is

@@ -33,6 +33,23 @@ template <int CTRL>
 __device__ __forceinline__ double row_mov0(double v) {
   return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, true);
 }
+// The sum over the four lane groups of 16, in every lane: swaps of rows and of halves between
+// two registers that hold the same value leave both addends in every lane (vector moves; a
+// shuffle through LDS waits twice)
+__device__ __forceinline__ double sum_groups(double v) {
+  auto join = [](unsigned lo, unsigned hi) __attribute__((always_inline)) {
+    return __hiloint2double((int)hi, (int)lo);
+  };
+  unsigned lo = __double2loint(v), hi = __double2hiint(v);
+  auto l16 = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  auto h16 = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  v = join(l16[0], h16[0]) + join(l16[1], h16[1]);
+  lo = __double2loint(v);
+  hi = __double2hiint(v);
+  auto l32 = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  auto h32 = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  return join(l32[0], h32[0]) + join(l32[1], h32[1]);
+}
 constexpr int kShr = 0x110, kShl = 0x100;  // row_shr:n, row_shl:n
 
 // The EVB block as evb_gradient reads it from LDS, for DC = 16 DT padded
@@ -96,7 +113,7 @@ __device__ __forceinline__ void stage_evb_kick(const double* __restrict__ dp, do
 // moved dof; its B operand is the first GEMMs' accumulators, scaled in place, and its result
 // has the layout of x.  With two hydrogens exchanged (dofs 0-5 of 27) that is 39 MFMAs per 16
 // beads; both wells in full take 56.  K-chunks beyond M are left out.  The per-bead well
-// energies are reduced over the four lane groups with two xor shuffles.
+// energies are reduced over the four lane groups (sum_groups).
 template <int M, int DT>
 __device__ __forceinline__ double evb_gradient(const double* PL, int m, int g, uint32_t moved,
                                                double scale, const double (&x)[DT][4],
@@ -153,10 +170,8 @@ __device__ __forceinline__ double evb_gradient(const double* PL, int m, int g, u
       ya[r][jj] = ha;
       yb[r][jj] = hb;
     }
-  va += __shfl_xor(va, 16);
-  va += __shfl_xor(va, 32);
-  vb += __shfl_xor(vb, 16);
-  vb += __shfl_xor(vb, 32);
+  va = sum_groups(va);
+  vb = sum_groups(vb);
   const double dl = va - vb, R = sqrt(0.25 * dl * dl + kappa * kappa), f = dl / (4.0 * R);
   const double wa = scale * (0.5 - f), wb = scale * (0.5 + f);
 #pragma unroll
