@@ -212,14 +212,17 @@ int rp_batch_family_shape(rp_batch *b, int fam, int *waves, int *units_per_wave,
  * steps-per-launch candidates; it keeps the fastest and reports the steps and the most
  * frequent wave count. */
 int rp_batch_set_launch(rp_batch *b, int steps_per_launch, int waves);
-/* rp_batch_run replays each family's block of steps_per_launch steps as a captured HIP
- * graph, between that family's timing events, when it draws from the Philox streams
- * (enable = 1, the default); enable = 0 launches the kernels directly.  Injected-noise runs
- * always launch directly.  The results are the same either way. */
+/* enable = 1: rp_batch_run replays each family's block of steps_per_launch steps as a captured
+ * HIP graph, between that family's timing events, when it draws from the Philox streams.
+ * enable = 0 (the default) launches the kernels directly, which is faster for blocks of one
+ * kernel per family; where the batch has no more polymers than the GPU has compute units, the
+ * families then run side by side.  Injected-noise runs always launch directly.  The results are
+ * the same either way. */
 int rp_batch_set_graphs(rp_batch *b, int enable);
 int rp_batch_autotune(rp_batch *b, int trial_steps, int *best_steps, int *best_waves);
 /* hipEvent-timed average duration of one fused-kernel launch per family in the last
- * rp_batch_run: avg_ms[nfam]; launches = launches per family */
+ * rp_batch_run: avg_ms[nfam]; launches = launches per family.  Families that ran side by side
+ * (rp_batch_set_graphs) overlap: their durations do not add up to the run's. */
 int rp_batch_last_kernel_ms(rp_batch *b, double *avg_ms, int64_t *launches);
 
 /* ------------------------------------------------------------------ instantons

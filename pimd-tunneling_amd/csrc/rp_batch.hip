@@ -51,10 +51,18 @@ struct rp_batch {
   std::vector<hipEvent_t> fev;  // per family: start, end
   std::vector<double> fam_ms;   // per family: summed launch time of the last run
   int64_t last_launches = 0;
-  // each family's launch of a step block (the last family's followed by the step counter
-  // update) captured as a HIP graph and replayed between its timing events; a graph is
-  // rebuilt when anything it captured changes
-  int use_graph = 1;
+  // Where every family's workgroups fit on the device at once, the families' launches run side
+  // by side: on s and these streams, between the fork event and the families' end events.  The
+  // longest chains take the streams first; family fi runs on lane[fi] (0: s).
+  std::vector<hipStream_t> side;
+  std::vector<int> lane;
+  hipEvent_t fork = nullptr;
+  // rp_batch_set_graphs: each family's launch of a step block (the last family's followed by
+  // the step counter update) captured as a HIP graph and replayed between its timing events; a
+  // graph is rebuilt when anything it captured changes.  Off by default: a block is one kernel
+  // per family, so a replay saves no launch (run of 8 steps, 44 polymers of the 27-dof EVB,
+  // N = 32: 96 us by graph, 81 us launched), and the first one pays for the capture.
+  int use_graph = 0;
   struct GraphKey {
     int fam = -1;
     int steps = -1;
@@ -193,12 +201,39 @@ static BatchArgs base_args(rp_batch* b, const Family& f, double h) {
   return a;
 }
 
-static int launch_family(rp_batch* b, const BatchArgs& a, int npoly) {
+static int launch_family(rp_batch* b, const BatchArgs& a, int npoly, hipStream_t st) {
   switch (b->pes->kind) {
-    case PES_EVB: return launch_batch_evb(b->pes, a, b->thermostat, npoly, b->s);
-    case PES_WATER: return launch_batch_water(b->pes, a, b->thermostat, npoly, b->s);
-    default: return launch_batch_simple(b->pes, a, b->thermostat, npoly, b->s);
+    case PES_EVB: return launch_batch_evb(b->pes, a, b->thermostat, npoly, st);
+    case PES_WATER: return launch_batch_water(b->pes, a, b->thermostat, npoly, st);
+    default: return launch_batch_simple(b->pes, a, b->thermostat, npoly, st);
   }
+}
+
+// Streams for families side by side.  A polymer takes at most one workgroup and a CU holds at
+// least one, so with no more polymers than CUs nothing queues for a CU and each family takes as
+// long as it would alone.  Beyond that the families fill the device one at a time, and their
+// launches stay in order on one stream.  Up to kLanes at once, the hardware queues a process has
+// by default; streams that share one still run in turn.  A run of 24 steps of 11 polymers each
+// of 17, 45, 99, 150 and 251 beads (27-dof EVB): 1.59 ms in turn, 1.07 side by side; the longest
+// family alone takes 0.65.
+constexpr int kLanes = 4;
+static int side_streams(rp_batch* b) {
+  const int nf = (int)b->fam.size();
+  b->lane.assign(nf, 0);
+  if (nf < 2 || b->npoly > b->ncu) return RP_OK;
+  RP_HIP(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
+  b->side.assign(std::min(nf, kLanes) - 1, nullptr);
+  for (auto& st : b->side) RP_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+  std::vector<int> ord(nf);
+  for (int i = 0; i < nf; ++i) ord[i] = i;
+  std::stable_sort(ord.begin(), ord.end(), [&](int u, int v) { return b->fam[u].N > b->fam[v].N; });
+  std::vector<int64_t> load(b->side.size() + 1, 0);
+  for (int fi : ord) {
+    const int l = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    b->lane[fi] = l;
+    load[l] += b->fam[fi].N;
+  }
+  return RP_OK;
 }
 
 extern "C" int rp_batch_create(rp_pes* pes, const double* mass, int npoly,
@@ -295,6 +330,8 @@ extern "C" int rp_batch_create(rp_pes* pes, const double* mass, int npoly,
         RP_HIP(hipDeviceGetAttribute(&b->ncu, hipDeviceAttributeMultiprocessorCount, dev));
         b->fev.assign(2 * b->fam.size(), nullptr);
         for (auto& e : b->fev) RP_HIP(hipEventCreate(&e));
+        int sr;
+        if ((sr = side_streams(b))) return sr;
         int r;
         if ((r = b->d_state.alloc(off))) return r;
         RP_HIP(hipMemsetAsync(b->d_state.p, 0, off * sizeof(double), b->s));
@@ -323,6 +360,8 @@ extern "C" int rp_batch_create(rp_pes* pes, const double* mass, int npoly,
 extern "C" int rp_batch_destroy(rp_batch* b) {
   if (!b) return RP_OK;
   if (b->s) (void)hipStreamSynchronize(b->s);
+  for (auto& st : b->side)
+    if (st) (void)hipStreamSynchronize(st);
   graph_drop(b);
   b->d_step0.free();
   for (Family& f : b->fam) {
@@ -338,6 +377,9 @@ extern "C" int rp_batch_destroy(rp_batch* b) {
   b->d_flags.free();
   for (auto& e : b->fev)
     if (e) (void)hipEventDestroy(e);
+  if (b->fork) (void)hipEventDestroy(b->fork);
+  for (auto& st : b->side)
+    if (st) (void)hipStreamDestroy(st);
   if (b->s) (void)hipStreamDestroy(b->s);
   delete b;
   return RP_OK;
@@ -476,7 +518,7 @@ static int graph_build(rp_batch* b, size_t fi, int steps, int64_t imin, hipGraph
   a.kicks = b->d_kicks.p;
   a.kick_cap = b->kick_cap;
   RP_HIP(hipStreamBeginCapture(b->s, hipStreamCaptureModeRelaxed));
-  rc = launch_family(b, a, f.count);
+  rc = launch_family(b, a, f.count, b->s);
   if (rc == RP_OK && fi + 1 == b->fam.size()) {
     batch_advance_kernel<<<1, 64, 0, b->s>>>(b->d_step0.p, steps);
     if (hipGetLastError() != hipSuccess)
@@ -504,8 +546,9 @@ static int graph_build(rp_batch* b, size_t fi, int steps, int64_t imin, hipGraph
 }
 
 // One launch per family of `steps` steps, each bracketed by its own events; per-family
-// durations are accumulated into fam_ms.  With the engine's own streams (no injected draws)
-// the block is a replay of its captured graph.
+// durations are accumulated into fam_ms.  By graph (use_graph, no injected draws) the block is a
+// replay, in order on one stream; else its launches run side by side where side_streams set that
+// up.
 static int run_block(rp_batch* b, int steps, int64_t imin, const double* dn, int64_t cap,
                      std::vector<double>& fam_ms) {
   int rc;
@@ -524,22 +567,39 @@ static int run_block(rp_batch* b, int steps, int64_t imin, const double* dn, int
       RP_HIP(hipEventRecord(b->fev[2 * fi + 1], b->s));
     }
   } else {
-    for (size_t fi = 0; fi < b->fam.size(); ++fi) {
-    Family& f = b->fam[fi];
-    BatchArgs a = base_args(b, f, 0.5 * b->dt);
-    a.nsteps = steps;
-    a.step0 = b->steps_done;
-    a.imin = imin;
-    a.noise = dn;
-    a.noise_cap = cap;
-    a.kicks = b->d_kicks.p;
-    a.kick_cap = b->kick_cap;
-    RP_HIP(hipEventRecord(b->fev[2 * fi], b->s));
-    if ((rc = launch_family(b, a, f.count))) return rc;
-    RP_HIP(hipEventRecord(b->fev[2 * fi + 1], b->s));
+    auto stream = [&](size_t fi) { return b->lane[fi] ? b->side[b->lane[fi] - 1] : b->s; };
+    if (!b->side.empty()) {
+      RP_HIP(hipEventRecord(b->fork, b->s));
+      for (hipStream_t st : b->side) RP_HIP(hipStreamWaitEvent(st, b->fork, 0));
     }
+    auto launch = [&](size_t fi) -> int {
+      Family& f = b->fam[fi];
+      BatchArgs a = base_args(b, f, 0.5 * b->dt);
+      a.nsteps = steps;
+      a.step0 = b->steps_done;
+      a.imin = imin;
+      a.noise = dn;
+      a.noise_cap = cap;
+      a.kicks = b->d_kicks.p;
+      a.kick_cap = b->kick_cap;
+      int q;
+      RP_HIP(hipEventRecord(b->fev[2 * fi], stream(fi)));
+      if ((q = launch_family(b, a, f.count, stream(fi)))) return q;
+      RP_HIP(hipEventRecord(b->fev[2 * fi + 1], stream(fi)));
+      return RP_OK;
+    };
+    // the longest first; families come in the order of their bead counts
+    rc = RP_OK;
+    size_t fi = b->fam.size();
+    while (fi > 0 && !rc) rc = launch(--fi);
+    // s waits for what the other streams got, once it has its own; after a failure too
+    for (hipStream_t st : b->side) {
+      RP_HIP(hipEventRecord(b->fork, st));
+      RP_HIP(hipStreamWaitEvent(b->s, b->fork, 0));
+    }
+    if (rc) return rc;
   }
-  RP_HIP(hipEventSynchronize(b->fev[2 * b->fam.size() - 1]));
+  RP_HIP(hipStreamSynchronize(b->s));  // which waits for every family
   fam_ms.resize(b->fam.size(), 0.0);
   for (size_t fi = 0; fi < b->fam.size(); ++fi) {
     float ms = 0.f;

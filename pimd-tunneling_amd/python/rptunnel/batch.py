@@ -129,7 +129,7 @@ class Batch:
         L.check(L.lib().rp_batch_set_launch(self.h, steps_per_launch, waves))
 
     def set_graphs(self, enable=True):
-        """Replay step blocks as captured HIP graphs (default) or launch kernels directly."""
+        """Replay step blocks as captured HIP graphs, or launch kernels directly (default)."""
         L.check(L.lib().rp_batch_set_graphs(self.h, int(bool(enable))))
 
     def autotune(self, trial_steps=64):
