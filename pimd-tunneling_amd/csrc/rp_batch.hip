@@ -77,6 +77,9 @@ struct rp_batch {
              pathd == o.pathd && npath == o.npath && waves == o.waves;
     }
   };
+  PinBuf own_pin;
+  PinBuf* pin = &own_pin;      // read-backs (fetch)
+  std::vector<char> unpinned;  // larger ones
   std::vector<std::pair<GraphKey, hipGraphExec_t>> graphs;  // recent family step blocks
   DevBuf<int64_t> d_step0;
 };
@@ -110,10 +113,43 @@ static void family_tables(const Family& f, std::vector<double>& T, std::vector<d
       Tf[((size_t)(i & 1) * HP + (i >> 1)) * HP + l] = T[(size_t)i * NP + l] * lam[i];
 }
 
-static int batch_flags(rp_batch* b) {
-  int f[2] = {0, 0};
-  RP_HIP(hipMemcpyAsync(f, b->d_flags.p, sizeof(f), hipMemcpyDeviceToHost, b->s));
+// Device arrays -> consecutive places in host memory (*out), then the stream is waited for.  The
+// memory is b->pin, allocated with the batch at the size of its largest read-back (allocating
+// 5.8 MB takes 2 ms, more than a run of 65536 small polymers), and beyond kPinMax pageable.
+constexpr size_t kPinMax = (size_t)16 << 20;
+static int fetch(rp_batch* b, std::initializer_list<std::pair<const void*, size_t>> parts, const char** out) {
+  size_t bytes = 0;
+  for (auto& q : parts) bytes += q.second;
+  int rc;
+  char* dst;
+  if (bytes > kPinMax) {
+    b->unpinned.resize(bytes);
+    dst = b->unpinned.data();
+  } else {
+    if ((rc = b->pin->ensure(bytes))) return rc;
+    dst = b->pin->p;
+  }
+  *out = dst;
+  for (auto& q : parts) {
+    RP_HIP(hipMemcpyAsync(dst, q.first, q.second, hipMemcpyDeviceToHost, b->s));
+    dst += q.second;
+  }
   RP_HIP(hipStreamSynchronize(b->s));
+  return RP_OK;
+}
+// every polymer's 64-bit fields
+static int fetch_pi(rp_batch* b, const int64_t** pi) {
+  const char* h = nullptr;
+  const int rc = fetch(b, {{b->d_pi64.p, b->d_pi64.n * sizeof(int64_t)}}, &h);
+  *pi = reinterpret_cast<const int64_t*>(h);
+  return rc;
+}
+
+static int batch_flags(rp_batch* b) {
+  int rc;
+  const char* h;
+  if ((rc = fetch(b, {{b->d_flags.p, 2 * sizeof(int)}}, &h))) return rc;
+  const int f[2] = {reinterpret_cast<const int*>(h)[0], reinterpret_cast<const int*>(h)[1]};
   if (f[0] || f[1]) {
     int z[2] = {0, 0};
     RP_HIP(hipMemcpy(b->d_flags.p, z, sizeof(z), hipMemcpyHostToDevice));
@@ -332,6 +368,10 @@ extern "C" int rp_batch_create(rp_pes* pes, const double* mass, int npoly,
         for (auto& e : b->fev) RP_HIP(hipEventCreate(&e));
         int sr;
         if ((sr = side_streams(b))) return sr;
+        // a one-polymer batch may be a chain's plan, which brings the chain's buffer
+        const size_t nmax = *std::max_element(b->N.begin(), b->N.end());
+        const size_t most = std::max(2 * 8 * nmax * D, (size_t)npoly * 8 * (size_t)(int(kPI64) + int(kPF64)));
+        if (npoly > 1 && (sr = b->own_pin.ensure(std::min(most, kPinMax)))) return sr;
         int r;
         if ((r = b->d_state.alloc(off))) return r;
         RP_HIP(hipMemsetAsync(b->d_state.p, 0, off * sizeof(double), b->s));
@@ -375,6 +415,7 @@ extern "C" int rp_batch_destroy(rp_batch* b) {
   b->d_stream.free();
   b->d_kicks.free();
   b->d_flags.free();
+  b->own_pin.free();
   for (auto& e : b->fev)
     if (e) (void)hipEventDestroy(e);
   if (b->fork) (void)hipEventDestroy(b->fork);
@@ -645,12 +686,57 @@ extern "C" int rp_batch_set_state(rp_batch* b, int poly, const double* x, const 
 extern "C" int rp_batch_get_state(rp_batch* b, int poly, double* x, double* p) {
   RP_REQUIRE(b && poly >= 0 && poly < b->npoly, "rp_batch_get_state: bad arguments");
   const int k = b->pos[poly];
-  const size_t nd = (size_t)b->N[k] * b->D;
-  if (x) RP_HIP(hipMemcpyAsync(x, b->d_state.p + b->soff[k], nd * sizeof(double), hipMemcpyDeviceToHost, b->s));
-  if (p) RP_HIP(hipMemcpyAsync(p, b->d_state.p + b->soff[k] + nd, nd * sizeof(double), hipMemcpyDeviceToHost, b->s));
-  RP_HIP(hipStreamSynchronize(b->s));
+  const size_t nd = (size_t)b->N[k] * b->D, bytes = nd * sizeof(double);
+  if (!x && !p) return RP_OK;
+  int rc;
+  const char* h;
+  if ((rc = fetch(b, {{b->d_state.p + b->soff[k] + (x ? 0 : nd), x && p ? 2 * bytes : bytes}},
+                  &h)))
+    return rc;
+  if (x) memcpy(x, h, bytes);
+  if (p) memcpy(p, h + (x ? bytes : 0), bytes);
   return RP_OK;
 }
+
+namespace rp {
+int batch_restart(rp_batch* b, const double* d_state, int64_t cursor, int64_t kcursor, PinBuf* pin) {
+  RP_REQUIRE(b->npoly == 1, "batch_restart: one polymer");
+  RP_REQUIRE(cursor >= 0 && kcursor >= 0, "rp_batch_set_cursor: negative cursor");
+  b->pin = pin;
+  int rc;
+  if ((rc = pin->ensure(8 * kPI64 + 8 * kPF64))) return rc;
+  int64_t* pi = reinterpret_cast<int64_t*>(pin->p);
+  std::fill(pi, pi + kPI64, 0);  // and the state's offset
+  pi[PI_CURSOR] = cursor;
+  pi[PI_KCURSOR] = kcursor;
+  pi[PI_RKICK] = -1;
+  double* sum = reinterpret_cast<double*>(pi + kPI64);
+  *sum = 0.0;
+  RP_HIP(hipMemcpyAsync(b->d_pi64.p, pi, kPI64 * 8, hipMemcpyHostToDevice, b->s));
+  RP_HIP(hipMemcpyAsync(b->d_pf64.p + PF_TISUM, sum, 8, hipMemcpyHostToDevice, b->s));
+  RP_HIP(hipMemcpyAsync(b->d_state.p, d_state, 2 * (size_t)b->N[0] * b->D * sizeof(double),
+                        hipMemcpyDeviceToDevice, b->s));
+  RP_HIP(hipStreamSynchronize(b->s));  // pin is free again
+  b->steps_done = 0;
+  return RP_OK;
+}
+
+int batch_result(rp_batch* b, double* d_state, double* sum, int64_t* count, int64_t* nreinit,
+                 int64_t* cursor, int64_t* kcursor) {
+  RP_HIP(hipMemcpyAsync(d_state, b->d_state.p, 2 * (size_t)b->N[0] * b->D * sizeof(double),
+                        hipMemcpyDeviceToDevice, b->s));
+  int rc;
+  const char* h;
+  if ((rc = fetch(b, {{b->d_pi64.p, kPI64 * 8}, {b->d_pf64.p, kPF64 * 8}}, &h))) return rc;
+  const int64_t* pi = reinterpret_cast<const int64_t*>(h);
+  *sum = reinterpret_cast<const double*>(pi + kPI64)[PF_TISUM];
+  *count = pi[PI_TICNT];
+  *nreinit = pi[PI_NREINIT];
+  *cursor = pi[PI_CURSOR];
+  *kcursor = pi[PI_KCURSOR];
+  return RP_OK;
+}
+}  // namespace rp
 
 extern "C" int rp_batch_set_kicks(rp_batch* b, const int32_t* kicks, int64_t nkicks_per_poly) {
   RP_REQUIRE(b && (kicks == nullptr || nkicks_per_poly > 0), "rp_batch_set_kicks: bad arguments");
@@ -706,13 +792,11 @@ extern "C" int rp_batch_run(rp_batch* b, int64_t nsteps, int64_t imin, const dou
 extern "C" int rp_batch_ti_readout(rp_batch* b, double* dhdr_sum, int64_t* count,
                                    int64_t* nreinit) {
   RP_REQUIRE(b, "rp_batch_ti_readout: NULL batch");
-  std::vector<int64_t> pi((size_t)b->npoly * kPI64);
-  std::vector<double> pf((size_t)b->npoly * kPF64);
   int rc;
-  if ((rc = b->d_pi64.download(pi.data(), pi.size(), b->s)) ||
-      (rc = b->d_pf64.download(pf.data(), pf.size(), b->s)))
-    return rc;
-  RP_HIP(hipStreamSynchronize(b->s));
+  const char* h;
+  if ((rc = fetch(b, {{b->d_pi64.p, b->d_pi64.n * 8}, {b->d_pf64.p, b->d_pf64.n * 8}}, &h))) return rc;
+  const int64_t* pi = reinterpret_cast<const int64_t*>(h);
+  const double* pf = reinterpret_cast<const double*>(pi + b->d_pi64.n);
   for (int p = 0; p < b->npoly; ++p) {
     const int k = b->pos[p];
     if (dhdr_sum) dhdr_sum[p] = pf[(size_t)k * kPF64 + PF_TISUM];
@@ -724,20 +808,18 @@ extern "C" int rp_batch_ti_readout(rp_batch* b, double* dhdr_sum, int64_t* count
 
 extern "C" int rp_batch_get_cursor(rp_batch* b, int64_t* cursor) {
   RP_REQUIRE(b && cursor, "rp_batch_get_cursor: bad arguments");
-  std::vector<int64_t> pi((size_t)b->npoly * kPI64);
+  const int64_t* pi;
   int rc;
-  if ((rc = b->d_pi64.download(pi.data(), pi.size(), b->s))) return rc;
-  RP_HIP(hipStreamSynchronize(b->s));
+  if ((rc = fetch_pi(b, &pi))) return rc;
   for (int p = 0; p < b->npoly; ++p) cursor[p] = pi[(size_t)b->pos[p] * kPI64 + PI_CURSOR];
   return RP_OK;
 }
 
 extern "C" int rp_batch_get_kick_cursor(rp_batch* b, int64_t* kick_cursor) {
   RP_REQUIRE(b && kick_cursor, "rp_batch_get_kick_cursor: bad arguments");
-  std::vector<int64_t> pi((size_t)b->npoly * kPI64);
+  const int64_t* pi;
   int rc;
-  if ((rc = b->d_pi64.download(pi.data(), pi.size(), b->s))) return rc;
-  RP_HIP(hipStreamSynchronize(b->s));
+  if ((rc = fetch_pi(b, &pi))) return rc;
   for (int p = 0; p < b->npoly; ++p)
     kick_cursor[p] = pi[(size_t)b->pos[p] * kPI64 + PI_KCURSOR];
   return RP_OK;

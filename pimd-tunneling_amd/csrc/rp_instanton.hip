@@ -675,16 +675,16 @@ extern "C" int rp_instanton(rp_ring* r, double pgtol, double factr, int m, int m
   const int nc = ring_nchain(r);
   const int64_t tot = ring_tot(r);
   const RingBufs rb = ring_bufs(r);
-  DevBuf<double> X, G, Dv, Glo, Gp, S, Y;
-  DevBuf<LbChain> st;
-  DevBuf<double> rho;
-  DevBuf<int> stat;
   int rc;
-  if ((rc = X.alloc(tot)) || (rc = G.alloc(tot)) || (rc = Dv.alloc(tot)) || (rc = Glo.alloc(tot)) ||
-      (rc = Gp.alloc(tot)) || (rc = S.alloc((size_t)(m + 1) * tot)) ||
-      (rc = Y.alloc((size_t)(m + 1) * tot)) || (rc = st.alloc(nc)) || (rc = stat.alloc(nc)) ||
-      (rc = rho.alloc((size_t)nc * (kMaxM + 1))))
+  // [X | G | Dv | Glo | Gprev | S | Y | rho | st], and the status words
+  const size_t pairs = (size_t)(m + 1) * tot, nrho = (size_t)nc * (kMaxM + 1);
+  static_assert(sizeof(LbChain) % sizeof(double) == 0, "states in doubles");
+  double* w;
+  int* stat;
+  if ((rc = ring_search_ws(r, 5 * (size_t)tot + 2 * pairs + nrho + nc * sizeof(LbChain) / sizeof(double),
+                           nc, &w, &stat)))
     return rc;
+  LbChain* st = reinterpret_cast<LbChain*>(w + 5 * (size_t)tot + 2 * pairs + nrho);
   LbArgs A;
   A.nchain = nc;
   A.m = m;
@@ -695,13 +695,19 @@ extern "C" int rp_instanton(rp_ring* r, double pgtol, double factr, int m, int m
   A.tot = tot;
   A.off = rb.off;
   A.n = rb.n;
-  A.X = X.p; A.G = G.p; A.Dv = Dv.p; A.Glo = Glo.p; A.Gprev = Gp.p; A.S = S.p; A.Y = Y.p;
+  A.X = w;
+  A.G = w + tot;
+  A.Dv = w + 2 * tot;
+  A.Glo = w + 3 * tot;
+  A.Gprev = w + 4 * tot;
+  A.S = w + 5 * tot;
+  A.Y = A.S + pairs;
+  A.rho = A.Y + pairs;
   A.XT = rb.x;
   A.GT = rb.g;
   A.E = rb.e;
-  A.st = st.p;
-  A.rho = rho.p;
-  A.status = stat.p;
+  A.st = st;
+  A.status = stat;
   const RingPc pc = ring_pc(r);
   A.pctab = pc.tab;
   A.pcoff = pc.off;
@@ -740,7 +746,7 @@ extern "C" int rp_instanton(rp_ring* r, double pgtol, double factr, int m, int m
   bool capped = true;
   for (long round = 0; round < cap; ++round) {
     if (round % kCheckEvery == 0) {
-      if ((rc = stat.download(hs.data(), nc, rb.s))) return rc;
+      RP_HIP(hipMemcpyAsync(hs.data(), stat, nc * sizeof(int), hipMemcpyDeviceToHost, rb.s));
       RP_HIP(hipStreamSynchronize(rb.s));
       if (std::none_of(hs.begin(), hs.end(), [](int v) { return v == ST_RUN; })) {
         capped = false;
@@ -759,8 +765,9 @@ extern "C" int rp_instanton(rp_ring* r, double pgtol, double factr, int m, int m
   }
   // results; the optimum stays on the device for the Hessian / log-determinant calls
   std::vector<LbChain> hst(nc);
-  RP_HIP(hipMemcpyAsync(rb.x, X.p, tot * sizeof(double), hipMemcpyDeviceToDevice, rb.s));
-  if ((rc = X.download(x_inout, tot, rb.s)) || (rc = st.download(hst.data(), nc, rb.s))) return rc;
+  RP_HIP(hipMemcpyAsync(rb.x, A.X, tot * sizeof(double), hipMemcpyDeviceToDevice, rb.s));
+  RP_HIP(hipMemcpyAsync(x_inout, A.X, tot * sizeof(double), hipMemcpyDeviceToHost, rb.s));
+  RP_HIP(hipMemcpyAsync(hst.data(), st, nc * sizeof(LbChain), hipMemcpyDeviceToHost, rb.s));
   RP_HIP(hipStreamSynchronize(rb.s));
   for (int c = 0; c < nc; ++c) {
     action[c] = hst[c].f;

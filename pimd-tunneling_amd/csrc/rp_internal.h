@@ -60,6 +60,27 @@ struct DevBuf {
   }
 };
 
+// Pinned host memory that an object keeps for its read-backs: a copy into it is one transfer,
+// where a pageable destination is staged and waited for copy by copy (reading back 55 polymers of
+// 17 to 251 beads and 27 dofs one by one: 1.87 ms pageable, 1.08 pinned).  Given back with its
+// owner.
+struct PinBuf {
+  char* p = nullptr;
+  size_t n = 0;
+  int ensure(size_t bytes) {
+    if (bytes <= n) return RP_OK;
+    free();
+    RP_HIP(hipHostMalloc((void**)&p, bytes, hipHostMallocDefault));
+    n = bytes;
+    return RP_OK;
+  }
+  void free() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    n = 0;
+  }
+};
+
 }  // namespace rp
 
 struct rp_pes {
@@ -116,6 +137,12 @@ int pes_maxd(const rp_pes* pes);
 // Whether the batched engine runs a polymer of n beads on this potential: a device
 // potential of a supported kind and size, n in 2..256, its workgroup within a CU's LDS.
 bool batch_supports(const rp_pes* pes, int n);
+// One-polymer batches of the plain chain (propagate_fused): start over from the chain's state,
+// a device array [x | p], at the given stream positions with empty sums, as a fresh batch would;
+// and bring the state back, with the sums and positions.  The read-backs go through `pin`.
+int batch_restart(rp_batch* b, const double* d_state, int64_t cursor, int64_t kcursor, PinBuf* pin);
+int batch_result(rp_batch* b, double* d_state, double* sum, int64_t* count, int64_t* nreinit,
+                 int64_t* cursor, int64_t* kcursor);
 // row stride of the device EVB layout (the MAXD bucket dispatch_pes picks)
 inline int evb_stride(int D) { return D <= 16 ? 16 : D == 27 ? 27 : 32; }
 }  // namespace rp

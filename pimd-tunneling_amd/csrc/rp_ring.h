@@ -38,4 +38,7 @@ struct RingPc {
   int ndim;
 };
 RingPc ring_pc(rp_ring* r);
+// the instanton search's vectors, kept by the ring between searches: `words` doubles and `ints`
+// ints of device memory at least
+int ring_search_ws(rp_ring* r, size_t words, size_t ints, double** w, int** iw);
 }  // namespace rp

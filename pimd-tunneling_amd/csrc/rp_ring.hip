@@ -967,6 +967,8 @@ struct rp_ring {
   DevBuf<int> d_umtask, d_umfirst;
   DevBuf<double> d_umpart;
   int n_umtask = 0, um_grid = 0;
+  DevBuf<double> d_search;  // the instanton search's vectors (ring_search_ws)
+  DevBuf<int> d_searchi;
 };
 
 static RingArgs ring_args(rp_ring* r) {
@@ -1073,6 +1075,14 @@ int ring_D(const rp_ring* r) { return r->D; }
 int ring_upload_x(rp_ring* r, const double* x) { return r->d_x.upload(x, r->tot, r->s); }
 RingPc ring_pc(rp_ring* r) {
   return RingPc{r->pc_sigma > 0.0 ? r->d_pctab.p : nullptr, r->d_pcoff.p, r->ndim};
+}
+int ring_search_ws(rp_ring* r, size_t words, size_t ints, double** w, int** iw) {
+  int rc;
+  if (r->d_search.n < words && (rc = r->d_search.alloc(words))) return rc;
+  if (r->d_searchi.n < ints && (rc = r->d_searchi.alloc(ints))) return rc;
+  *w = r->d_search.p;
+  *iw = r->d_searchi.p;
+  return RP_OK;
 }
 RingBufs ring_bufs(rp_ring* r) {
   return RingBufs{r->d_x.p, r->d_g.p, r->d_e.p, r->d_off.p, r->d_n.p, r->D, r->s};
@@ -1192,13 +1202,14 @@ extern "C" int rp_ring_destroy(rp_ring* r) {
   if (r->ev) (void)hipEventDestroy(r->ev);
   for (DevBuf<double>* b : {&r->d_x, &r->d_g, &r->d_v, &r->d_hv, &r->d_e, &r->d_ab, &r->d_betan,
                             &r->d_massd, &r->d_blocks, &r->d_sinv, &r->d_work, &r->d_ld, &r->d_eta,
-                            &r->d_pe, &r->d_pctab})
+                            &r->d_pe, &r->d_pctab, &r->d_search})
     b->free();
   r->d_n.free();
   r->d_nneg.free();
   r->d_umtask.free();
   r->d_umfirst.free();
   r->d_umpart.free();
+  r->d_searchi.free();
   r->d_off.free();
   r->d_boff.free();
   r->d_pcoff.free();
