@@ -202,4 +202,67 @@ __device__ __forceinline__ double evb_gradient(const double* PL, int m, int g, u
   return 0.5 * (va + vb) - R;
 }
 
+// W x of both wells on the matrix cores, 16 beads of a wave: y_A = WtA x is one GEMM whose B
+// operand is x as the state holds it (item j of dof tile d is dof 16 d + g + 4 j of bead m, the
+// operand of K-chunk 4 d + j), and y_B = y_A + (WtB - WtA) x, over the K-chunks in `moved` only:
+// those with a dof that the wells' permutation moves.  K-chunks beyond M are left out.
+// (evb_gradient holds this and evb_back in its own body: by way of these functions the step
+// kernel for small batches spills 12 VGPRs, 49 -> 52 us per 8 steps of 44 polymers, N = 32.)
+template <int M, int DT>
+__device__ __forceinline__ void evb_modes(const double* WA, const double* WD, int ld, int m, int g,
+                                          uint32_t moved, const double (&x)[DT][4], d4 (&ya)[DT],
+                                          d4 (&yb)[DT]) {
+  constexpr int LW = 16 * DT + 1;
+#pragma unroll
+  for (int r = 0; r < DT; ++r) ya[r] = d4{0.0, 0.0, 0.0, 0.0};
+  static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
+    constexpr int kc = decltype(K)::value;
+    if constexpr (4 * kc < M) {
+#pragma unroll
+      for (int r = 0; r < DT; ++r)
+        ya[r] = mfma_f64(WA[(r * 16 + m) * LW + 4 * kc + g], x[kc / 4][kc % 4], ya[r]);
+    }
+  });
+#pragma unroll
+  for (int r = 0; r < DT; ++r) yb[r] = ya[r];
+  static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
+    constexpr int kc = decltype(K)::value;
+    if constexpr (4 * kc < M) {
+      if ((moved >> kc) & 1) {  // wave-uniform
+#pragma unroll
+        for (int r = 0; r < DT; ++r)
+          yb[r] = mfma_f64(WD[(r * 16 + m) * ld + 4 * kc + g], x[kc / 4][kc % 4], yb[r]);
+      }
+    }
+  });
+}
+
+// ag = WtA^T u + (WtB - WtA)^T w, the second product for the dof tiles with a moved dof: B
+// operands in the accumulator layout of evb_modes, the result in the layout of x
+template <int M, int DT>
+__device__ __forceinline__ void evb_back(const double* WA, const double* WD, int ld, int m, int g,
+                                         uint32_t moved, const d4 (&u)[DT], const d4 (&w)[DT],
+                                         d4 (&ag)[DT]) {
+  constexpr int LW = 16 * DT + 1;
+#pragma unroll
+  for (int d = 0; d < DT; ++d) ag[d] = d4{0.0, 0.0, 0.0, 0.0};
+  static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
+    constexpr int kc = decltype(K)::value;
+    if constexpr (4 * kc < M) {
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+        ag[d] = mfma_f64(WA[(4 * kc + g) * LW + d * 16 + m], u[kc / 4][kc % 4], ag[d]);
+    }
+  });
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+    if ((moved >> (4 * d)) & 15u) {  // wave-uniform
+      static_for<4 * DT>([&](auto K) __attribute__((always_inline)) {
+        constexpr int kc = decltype(K)::value;
+        if constexpr (4 * kc < M)
+          ag[d] = mfma_f64(WD[(4 * kc + g) * ld + d * 16 + m], w[kc / 4][kc % 4], ag[d]);
+      });
+    }
+}
+
 }  // namespace rp

@@ -249,6 +249,138 @@ __global__ void __launch_bounds__(kRingTile) ring_hvp_kernel(RingArgs A, const d
   }
 }
 
+// Potential Hessian blocks of the EVB on the matrix cores.  With s = wa (lam + 6 c y_A) and t its
+// counterpart for well B, per mode, R = sqrt((V_A - V_B)^2 / 4 + kappa^2) and the wells'
+// gradients g_A, g_B, a bead's block is
+//   WtA^T diag(s) WtA + WtB^T diag(t) WtB - u u^T,  u = sqrt(kappa^2 / (4 R^3)) (g_A - g_B).
+// A wave takes 16 beads of the ring's tile list: their modes as in evb_gradient, s, t and u
+// through the wave's own LDS, then bead by bead one MFMA per four modes, well and 16 x 16 tile,
+// both operands the same fragments of Wt (held in registers), one of them scaled.
+// single_first: bead 0's block for every bead.
+// Bound by its MFMAs and the store of the blocks.  139k beads of 27 dofs: 0.34 ms, 0.8 GB of
+// blocks; with a forward-over-reverse sweep per row (ring_hblock_kernel) 1.90 ms.
+constexpr int kHbWaves = 4;
+
+template <int M>
+__global__ void __launch_bounds__(kHbWaves * 64, 2) ring_hblock_evb_kernel(
+    RingArgs A, uint32_t moved, const double* __restrict__ x, int single_first,
+    const int* __restrict__ tiles, int ntile, double* __restrict__ blocks) {
+  constexpr int DT = (M + 15) / 16, DC = 16 * DT, LW = DC + 1, NK = (M + 3) / 4;
+  extern __shared__ double PL[];
+  const int tid = threadIdx.x, D = A.D;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, m = lane & 15, g = lane >> 4;
+  double* st = PL + ((evb_kick_lds_size(DC, moved) + 1) & ~1) + wave * 3 * 16 * LW;  // [s | t | u][bead][LW]
+  stage_evb_kick<M, DT>(A.pes.dp, PL, moved, tid, kHbWaves * 64);
+  __syncthreads();
+  const double* WA = PL + 2 + 4 * DC;
+  const double* WD = WA + DC * LW;
+  const int ld = evb_diff_stride(moved);
+  double fa[NK][DT], fb[NK][DT];
+#pragma unroll
+  for (int kc = 0; kc < NK; ++kc)
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      fa[kc][t] = WA[(4 * kc + g) * LW + 16 * t + m];
+      fb[kc][t] = fa[kc][t] + (moved && 16 * t < ld - 1 ? WD[(4 * kc + g) * ld + 16 * t + m] : 0.0);
+    }
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  for (int tile = blockIdx.x * kHbWaves + wave; tile < ntile; tile += gridDim.x * kHbWaves) {
+    const int c = tiles[2 * tile], b0 = tiles[2 * tile + 1], n = A.n[c];
+    const double* __restrict__ xc = x + A.off[c] + (single_first ? 0 : min(b0 + m, n - 1));
+    double xs[DT][4];
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int row = 16 * d + 4 * j + g;
+        xs[d][j] = row < D ? xc[(size_t)row * n] : 0.0;
+      }
+    {
+      const double kappa = PL[0];
+      const double* cA = PL + 2 + g;
+      const double* cB = cA + DC;
+      const double* lam = cB + DC;
+      const double* cub = lam + DC;
+      d4 ya[DT], yb[DT], ag[DT], sa[DT], sb[DT];
+      evb_modes<M, DT>(WA, WD, ld, m, g, moved, xs, ya, yb);
+      double va = 0.0, vb = 0.0;
+#pragma unroll
+      for (int r = 0; r < DT; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = r * 16 + 4 * j;
+          const double li = lam[i], ci = cub[i];
+          auto well = [&](double y, double& v, double& h, double& s) __attribute__((always_inline)) {
+            const double t = ci * y;
+            v += (y * y) * fma(0.5, li, t);
+            h = y * fma(3.0, t, li);
+            s = fma(6.0, t, li);
+          };
+          double ha, hb, da, db;
+          well(ya[r][j] - cA[i], va, ha, da);
+          well(yb[r][j] - cB[i], vb, hb, db);
+          ya[r][j] = ha - hb;
+          yb[r][j] = -hb;
+          sa[r][j] = da;
+          sb[r][j] = db;
+        }
+      va = sum_groups(va);
+      vb = sum_groups(vb);
+      const double dl = va - vb, R2 = 0.25 * dl * dl + kappa * kappa, R = sqrt(R2), f = dl / (4.0 * R);
+      const double q = sqrt(kappa * kappa / (4.0 * R2 * R));
+      evb_back<M, DT>(WA, WD, ld, m, g, moved, ya, yb, ag);  // g_A - g_B
+      wave_sync();  // the previous tile's reads are done
+#pragma unroll
+      for (int r = 0; r < DT; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          double* o = st + m * LW + 16 * r + 4 * j + g;
+          o[0] = (0.5 - f) * sa[r][j];
+          o[16 * LW] = (0.5 + f) * sb[r][j];
+          o[32 * LW] = q * ag[r][j];
+        }
+      wave_sync();
+    }
+    const int nb = min(16, n - b0);
+    for (int b = 0; b < nb; ++b) {
+      const double* sp = st + b * LW;
+      d4 acc[DT][DT];
+      double u[DT];
+#pragma unroll
+      for (int t = 0; t < DT; ++t) u[t] = g == 0 ? sp[32 * LW + 16 * t + m] : 0.0;
+#pragma unroll
+      for (int rt = 0; rt < DT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < DT; ++ct) acc[rt][ct] = mfma_f64(-u[rt], u[ct], d4{0.0, 0.0, 0.0, 0.0});
+#pragma unroll
+      for (int kc = 0; kc < NK; ++kc) {
+        const double s = sp[4 * kc + g], t = sp[16 * LW + 4 * kc + g];
+#pragma unroll
+        for (int rt = 0; rt < DT; ++rt)
+#pragma unroll
+          for (int ct = 0; ct < DT; ++ct) {
+            acc[rt][ct] = mfma_f64(s * fa[kc][rt], fa[kc][ct], acc[rt][ct]);
+            acc[rt][ct] = mfma_f64(t * fb[kc][rt], fb[kc][ct], acc[rt][ct]);
+          }
+      }
+      double* out = blocks + (size_t)(A.boff[c] + b0 + b) * D * D;
+#pragma unroll
+      for (int rt = 0; rt < DT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < DT; ++ct)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int row = 16 * rt + 4 * j + g, col = 16 * ct + m;
+            if (row < D && col < D) out[row * D + col] = acc[rt][ct][j];
+          }
+    }
+  }
+}
+
 // Potential Hessian blocks of every bead from D forward-over-reverse sweeps:
 // blocks[gbead][i][k] = d grad_k / d x_i.  Thread (bead, i).
 template <int KIND, int MAXD>
@@ -1011,6 +1143,28 @@ static int ring_host_potential(rp_ring* r, bool want_grad) {
   return RP_OK;
 }
 
+// the bead tiles of every chain, once per ring
+static int ring_tiles(rp_ring* r) {
+  if (r->d_umtask.p) return RP_OK;
+  std::vector<int> t, first;
+  for (int c = 0; c < r->nchain; ++c) {
+    first.push_back((int)t.size() / 2);
+    for (int b0 = 0; b0 < r->n[c]; b0 += 16) {
+      t.push_back(c);
+      t.push_back(b0);
+    }
+  }
+  first.push_back((int)t.size() / 2);
+  int rc;
+  if ((rc = r->d_umpart.alloc(t.size() / 2)) || (rc = r->d_umfirst.alloc(first.size())) ||
+      (rc = r->d_umfirst.upload(first.data(), first.size(), r->s)) ||
+      (rc = r->d_umtask.alloc(t.size())) || (rc = r->d_umtask.upload(t.data(), t.size(), r->s)))
+    return rc;
+  RP_HIP(hipStreamSynchronize(r->s));  // t and first are released here
+  r->n_umtask = (int)(t.size() / 2);
+  return RP_OK;
+}
+
 // U_M of the ring's coordinates into energy (cleared by the caller, for potentials whose
 // kernel adds to it) and, unless null, its gradient into grad, queued on stream
 static int ring_eval_to(rp_ring* r, double* energy, double* grad, hipStream_t stream) {
@@ -1028,23 +1182,9 @@ static int ring_eval_to(rp_ring* r, double* energy, double* grad, hipStream_t st
       const uint32_t moved = evb_moved(r->pes);
       constexpr int DC = 16 * ((M + 15) / 16);
       const size_t lds = (((evb_kick_lds_size(DC, moved) + 1) & ~1) + DC) * sizeof(double);
-      if (!r->d_umtask.p) {  // the bead tiles of every chain, once per ring
-        std::vector<int> t, first;
-        for (int c = 0; c < r->nchain; ++c) {
-          first.push_back((int)t.size() / 2);
-          for (int b0 = 0; b0 < r->n[c]; b0 += 16) {
-            t.push_back(c);
-            t.push_back(b0);
-          }
-        }
-        first.push_back((int)t.size() / 2);
-        int rc;
-        if ((rc = r->d_umpart.alloc(t.size() / 2)) || (rc = r->d_umfirst.alloc(first.size())) ||
-            (rc = r->d_umfirst.upload(first.data(), first.size(), r->s)) ||
-            (rc = r->d_umtask.alloc(t.size())) || (rc = r->d_umtask.upload(t.data(), t.size(), r->s)))
-          return rc;
-        RP_HIP(hipStreamSynchronize(r->s));  // t and first are released at the end of this block
-        r->n_umtask = (int)(t.size() / 2);
+      int rc;
+      if ((rc = ring_tiles(r))) return rc;
+      if (!r->um_grid) {
         int ncu = 0, dev = 0, per_cu = 0;
         RP_HIP(hipGetDevice(&dev));
         RP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1393,7 +1533,23 @@ static int ring_blocks(rp_ring* r, int singlewell) {
   for (int c = 0; c < r->nchain; ++c) maxn = std::max(maxn, r->n[c]);
   dim3 grid((maxn * r->D + 127) / 128, r->nchain);
   return dispatch_pes(r->pes, [&]<int K, int M>() -> int {
-    ring_hblock_kernel<K, M><<<grid, 128, 0, r->s>>>(a, r->d_x.p, singlewell, r->d_blocks.p);
+    if constexpr (K == PES_EVB) {
+      if ((rc = ring_tiles(r))) return rc;
+      constexpr int DC = 16 * ((M + 15) / 16);
+      const uint32_t moved = evb_moved(r->pes);
+      const size_t lds = (((evb_kick_lds_size(DC, moved) + 1) & ~1) + kHbWaves * 3 * 16 * (DC + 1)) * sizeof(double);
+      auto kern = ring_hblock_evb_kernel<M>;
+      RP_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      int ncu = 0, dev = 0, per_cu = 0;
+      RP_HIP(hipGetDevice(&dev));
+      RP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+      RP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kHbWaves * 64, lds));
+      const int wgs = std::min((r->n_umtask + kHbWaves - 1) / kHbWaves, std::max(per_cu, 1) * std::max(ncu, 1));
+      kern<<<wgs, kHbWaves * 64, lds, r->s>>>(a, moved, r->d_x.p, singlewell, r->d_umtask.p, r->n_umtask,
+                                              r->d_blocks.p);
+    } else {
+      ring_hblock_kernel<K, M><<<grid, 128, 0, r->s>>>(a, r->d_x.p, singlewell, r->d_blocks.p);
+    }
     RP_HIP(hipGetLastError());
     return RP_OK;
   });
