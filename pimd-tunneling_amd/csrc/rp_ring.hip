@@ -889,13 +889,11 @@ __host__ __device__ inline int ring_middle(int D, int n) { return D <= 32 ? (n -
 //   forward:  t_i = S_i^-1 z_i toward h from both ends, z_0 = v_0, z_{n-1} = v_{n-1}, and the
 //             next bead's z = v + c t where the two are coupled; z_h takes both sides' c t;
 //   backward: y_h = t_h, y_i = t_i + c S_i^-1 y_{i +- 1} outward from h, y_0 = t_0.
-// Half of the threads take each side (HALVES = 2); from one end only, h = n-1 and HALVES = 1.
-// The running vector (z or y, D values) sits in LDS, double-buffered; what a step reads from
-// global memory (its block, and v or t) does not depend on it, so it is loaded P steps
-// ahead into registers, and the per-step barrier orders LDS only, which leaves those loads in
-// flight across it.  Lanes: Q per block row (row r = tid / Q, lane q), each holding the KPL
-// columns k = q + Q j of its row; a row's sum is a DPP butterfly inside its Q lanes.  The LDS
-// vector is zero beyond D, so clamped column loads add nothing.
+// Up to 32 dofs (ring_eta1_wave_kernel) a wave takes each side; above, one workgroup goes from
+// bead 0 to h = n - 1 and back (solve_sweep).  The running vector (z or y, D values) sits in LDS;
+// what a step reads from global memory (its block, and v or t) does not depend on it, so it is
+// loaded P steps ahead into registers.  The LDS vector is zero beyond D, so column loads beyond
+// a row add nothing.
 template <int CTRL>
 __device__ __forceinline__ double dpp_mov(double v) {
   return __builtin_amdgcn_update_dpp(0.0, v, CTRL, 0xF, 0xF, false);
@@ -910,14 +908,16 @@ __device__ __forceinline__ double row_sum(double s) {
   return s;
 }
 
-// One sweep of a side (side 0: beads below h, side 1: above), K steps of this side in Kmax of the
-// workgroup; returns the LDS buffer (of the side's two, zb) that holds its last vector.  src: v
-// (forward) or the t the forward sweep left in dst (backward).  Byte offsets within a chain fit
-// 31 bits (the host checks n D^2 8 < 2^31).
+// One sweep of K steps; returns the LDS buffer (of the two in zb) that holds its last vector.
+// src: v (forward) or the t the forward sweep left in dst (backward).  The per-step barrier
+// orders LDS only, which leaves the loads in flight across it.  Lanes: Q per block row (row
+// r = tid / Q, lane q), each holding the KPL columns k = q + Q j of its row; a row's sum is a
+// DPP butterfly inside its Q lanes.  Byte offsets within a chain fit 31 bits (the host checks
+// n D^2 8 < 2^31).
 template <int Q, int KPL, int P, int NT, bool FWD>
-__device__ __forceinline__ int solve_sweep(int D, int n, int h, int side, int K, int Kmax, int ht,
-                                           double c, const double* __restrict__ S,
-                                           const double* src, double* dst, double* zb, int cur) {
+__device__ __forceinline__ int solve_sweep(int D, int n, int h, int K, int ht, double c,
+                                           const double* __restrict__ S, const double* src,
+                                           double* dst, double* zb, int cur) {
   constexpr int QK = Q * KPL;
   const int r = ht / Q, q = ht - r * Q;
   const int rr = min(r, D - 1);
@@ -931,10 +931,10 @@ __device__ __forceinline__ int solve_sweep(int D, int n, int h, int side, int K,
   const int eo = rr * 8;
   // bead of step k, and the bead of the row value it reads (clamped to the chain)
   auto bead = [&](int k) {
-    const int i = FWD ? (side ? n - 1 - k : k) : (side ? h + 1 + k : h - 1 - k);
+    const int i = FWD ? k : h - 1 - k;
     return min(max(i, 0), n - 1);
   };
-  auto ebead = [&](int k) { return FWD ? min(max(bead(k) + (side ? -1 : 1), 0), n - 1) : bead(k); };
+  auto ebead = [&](int k) { return FWD ? min(bead(k) + 1, n - 1) : bead(k); };
   double a[P][KPL], e[P];
 #pragma unroll
   for (int s = 0; s < P; ++s) {
@@ -943,41 +943,37 @@ __device__ __forceinline__ int solve_sweep(int D, int n, int h, int side, int K,
     for (int j = 0; j < KPL; ++j) a[s][j] = buffer_ld(Sb, ko[j], so);
     e[s] = buffer_ld(Eb, eo, ebead(s) * D8);
   }
-  for (int k0 = 0; k0 < Kmax; k0 += P) {
+  for (int k0 = 0; k0 < K; k0 += P) {
 #pragma unroll
     for (int s = 0; s < P; ++s) {
       const int k = k0 + s;
-      if (k < Kmax) {  // block-uniform
-        if (k < K) {   // the side's waves
-          const double* u = zb + cur * QK;
-          double t0 = 0.0, t1 = 0.0;
+      if (k < K) {  // block-uniform
+        const double* u = zb + cur * QK;
+        double t0 = 0.0, t1 = 0.0;
 #pragma unroll
-          for (int j = 0; j < KPL; j += 2) {
-            t0 += a[s][j] * u[q + Q * j];
-            if (j + 1 < KPL) t1 += a[s][j + 1] * u[q + Q * (j + 1)];
-          }
-          const double t = row_sum<Q>(t0 + t1), ev = e[s];
-          const int so = bead(k + P) * DD8, i = bead(k);
-#pragma unroll
-          for (int j = 0; j < KPL; ++j) a[s][j] = buffer_ld(Sb, ko[j], so);
-          e[s] = buffer_ld(Eb, eo, ebead(k + P) * D8);
-          double* nz = zb + (cur ^ 1) * QK;
-          if (FWD) {
-            if (wr) {
-              dst[(int64_t)i * D + r] = t;
-              // side 1 brings its c t alone to the middle bead, which side 0 gives its v
-              const bool coupled = side || k >= 1, own = !(side && k == K - 1);
-              nz[r] = (own ? ev : 0.0) + (coupled ? c * t : 0.0);
-            }
-          } else {
-            const double y = ev + c * t;
-            if (wr) {
-              dst[(int64_t)i * D + r] = y;
-              nz[r] = y;
-            }
-          }
-          cur ^= 1;
+        for (int j = 0; j < KPL; j += 2) {
+          t0 += a[s][j] * u[q + Q * j];
+          if (j + 1 < KPL) t1 += a[s][j + 1] * u[q + Q * (j + 1)];
         }
+        const double t = row_sum<Q>(t0 + t1), ev = e[s];
+        const int so = bead(k + P) * DD8, i = bead(k);
+#pragma unroll
+        for (int j = 0; j < KPL; ++j) a[s][j] = buffer_ld(Sb, ko[j], so);
+        e[s] = buffer_ld(Eb, eo, ebead(k + P) * D8);
+        double* nz = zb + (cur ^ 1) * QK;
+        if (FWD) {
+          if (wr) {
+            dst[(int64_t)i * D + r] = t;
+            nz[r] = ev + (k >= 1 ? c * t : 0.0);
+          }
+        } else {
+          const double y = ev + c * t;
+          if (wr) {
+            dst[(int64_t)i * D + r] = y;
+            nz[r] = y;
+          }
+        }
+        cur ^= 1;
         lds_sync<NT>();
       }
     }
@@ -985,38 +981,41 @@ __device__ __forceinline__ int solve_sweep(int D, int n, int h, int side, int K,
   return cur;
 }
 
+// Inverse iteration's fixed generic start
+__device__ __forceinline__ double start_entry(int64_t e) {
+  return 1.0 + 0.37 * (double)((e * 7919) % 101) / 101.0;
+}
+
 // Inverse iteration for the eigenvalue of H nearest the factorisation shift sig:
 // v <- (H - sig)^-1 v / |.|, eta = sig + 1 / (v . (H - sig)^-1 v) for the normalised v.
 // work holds [v | y] per chain (2 n D); fresh = 1 starts from a fixed generic vector,
 // otherwise the previous v is continued.  Stops after iters iterations, or earlier once eta
 // changes by at most tol relative; chains with act[c] == 0 are left as they are.
-// D <= Q KPL.
-template <int Q, int KPL, int P, int HALVES>
-__global__ void __launch_bounds__(HALVES * kRingThreads) ring_eta1_kernel(
+// More than 32 dofs, D <= Q KPL; one end, h = n - 1.
+template <int Q, int KPL, int P>
+__global__ void __launch_bounds__(kRingThreads) ring_eta1_kernel(
     int D, const int* __restrict__ nn, const int64_t* __restrict__ boff,
     const double* __restrict__ betan, const double* __restrict__ sinv, double* __restrict__ work,
     const double* __restrict__ shift, int iters, int fresh, double tol,
     const int* __restrict__ act, double* __restrict__ eta1) {
   static_assert(Q * (kRingThreads / Q) == kRingThreads && (Q == 2 || Q == 4 || Q == 8), "lanes per row");
-  constexpr int NT = HALVES * kRingThreads, QK = Q * KPL;
+  constexpr int NT = kRingThreads, QK = Q * KPL;
   __shared__ double red[NT];
-  __shared__ double zbs[HALVES][2 * QK], zm[QK];
+  __shared__ double zb[2 * QK], zm[QK];
   const int cix = blockIdx.x, n = nn[cix], tid = threadIdx.x;
   if (act && !act[cix]) return;  // block-uniform
-  const int side = HALVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / kRingThreads);
-  const int ht = tid - side * kRingThreads, h = ring_middle(D, n);
+  const int h = n - 1;
   const int64_t tot = (int64_t)n * D;
   const double c = 1.0 / (betan[cix] * betan[cix]);
   double* v = work + 2 * boff[cix] * D;
   double* y = v + tot;
   const double* S = sinv + (size_t)boff[cix] * D * D;
   const double sig = shift ? shift[cix] : 0.0;
-  double* zb = zbs[side];
-  if (ht < 2 * QK) zb[ht] = 0.0;
+  if (tid < 2 * QK) zb[tid] = 0.0;
   if (tid < QK) zm[tid] = 0.0;
   double nrm = 0.0;
   for (int64_t e = tid; e < tot; e += NT) {
-    const double t = fresh ? 1.0 + 0.37 * (double)((e * 7919) % 101) / 101.0 : v[e];
+    const double t = fresh ? start_entry(e) : v[e];
     v[e] = t;
     nrm += t * t;
   }
@@ -1024,19 +1023,14 @@ __global__ void __launch_bounds__(HALVES * kRingThreads) ring_eta1_kernel(
   for (int64_t e = tid; e < tot; e += NT) v[e] /= nrm;
   __syncthreads();
   double eta = 0.0, prev = 0.0;
-  const int nup = h, ndn = n - 1 - h;
   for (int it = 0; it < iters; ++it) {
-    if (ht < D) zb[ht] = v[side ? tot - D + ht : ht];  // z_0 and z_{n-1} in the sides' buffers 0
+    if (tid < D) zb[tid] = v[tid];
     __syncthreads();
-    const int cur = solve_sweep<Q, KPL, P, NT, true>(D, n, h, side, side ? ndn : nup, max(nup, ndn), ht, c,
-                                               S, v, y, zb, 0);
-    // the middle bead: z_h from both sides, y_h = S_h^-1 z_h by side 0, for both sides' way back
-    if (!side && ht < D) zm[ht] = zb[cur * QK + ht];
+    const int cur = solve_sweep<Q, KPL, P, NT, true>(D, n, h, h, tid, c, S, v, y, zb, 0);
+    if (tid < D) zm[tid] = zb[cur * QK + tid];  // z_h; y_h = S_h^-1 z_h
     __syncthreads();
-    if (side && h >= 1 && ht < D) zm[ht] += zb[cur * QK + ht];
-    if (HALVES == 2) __syncthreads();
-    if (!side) {
-      const int r = ht / Q, q = ht - r * Q;
+    {
+      const int r = tid / Q, q = tid - r * Q;
       const double* Sh = S + ((int64_t)h * D + min(r, D - 1)) * D;
       double t = 0.0;
 #pragma unroll
@@ -1044,15 +1038,11 @@ __global__ void __launch_bounds__(HALVES * kRingThreads) ring_eta1_kernel(
       t = row_sum<Q>(t);
       if (q == 0 && r < D) {
         y[(int64_t)h * D + r] = t;
-#pragma unroll
-        for (int b = 0; b < HALVES; ++b) zbs[b][r] = t;
+        zb[r] = t;
       }
     }
     __syncthreads();  // and the t of every lane, in y, before the backward sweep reads them
-    // y_0 = t_0, and nothing comes back to side 1 where h = 0: bead 0 is coupled to no other
-    const int kup = max(nup - 1, 0), kdn = h ? ndn : 0;
-    solve_sweep<Q, KPL, P, NT, false>(D, n, h, side, side ? kdn : kup, max(kup, kdn), ht, c, S, y, y,
-                                      zb, 0);
+    solve_sweep<Q, KPL, P, NT, false>(D, n, h, max(h - 1, 0), tid, c, S, y, y, zb, 0);  // y_0 = t_0
     __syncthreads();
     double mu = 0.0, yy = 0.0;
     for (int64_t e = tid; e < tot; e += NT) {
@@ -1067,6 +1057,173 @@ __global__ void __launch_bounds__(HALVES * kRingThreads) ring_eta1_kernel(
     if (it > 2 && fabs(eta - prev) <= tol * fabs(eta)) break;  // block-uniform
     prev = eta;
   }
+  if (tid == 0) eta1[cix] = eta;
+}
+
+// The same up to 32 dofs, D <= 2 KPL: wave 0 takes the beads below h, wave 1 those above.  Two
+// lanes per block row, KPL consecutive columns each in 16-byte loads (a row's overrun reads the
+// next rows, or zeros past the chain's end, against zeros of the LDS vector), so a step is KPL
+// FMAs, one DPP move and one LDS round trip inside the wave, with no barrier.  v . y and |y|^2
+// are summed in the backward sweep and the normalisation goes into the next forward one: the two
+// vectors' buffers change places instead of three more passes over them.
+// Loads in flight: P (KPL / 2 + 1 or 2) of the 63 that a wave can have.
+// Bound by the serial chain where a chain is alone, else by the blocks' bytes (2.6 TB/s).  ms per
+// iteration of chains of 1024 beads, 27 dofs: one 0.49, 256 0.90; with four waves a side, eight
+// lanes per row and a barrier per step 0.63 and 1.03.
+typedef double d2 __attribute__((ext_vector_type(2)));
+template <int KPL, int P>
+__global__ void __launch_bounds__(128) ring_eta1_wave_kernel(
+    int D, const int* __restrict__ nn, const int64_t* __restrict__ boff,
+    const double* __restrict__ betan, const double* __restrict__ sinv, double* __restrict__ work,
+    const double* __restrict__ shift, int iters, int fresh, double tol,
+    const int* __restrict__ act, double* __restrict__ eta1) {
+  __shared__ __attribute__((aligned(16))) double zs[2][2 * KPL], zm[2 * KPL];
+  __shared__ double red[2][2];
+  const int cix = blockIdx.x, n = nn[cix], tid = threadIdx.x, lane = tid & 63;
+  if (act && !act[cix]) return;  // block-uniform
+  const int side = __builtin_amdgcn_readfirstlane(tid >> 6), h = ring_middle(D, n);
+  const int r = lane >> 1, q = lane & 1, rr = min(r, D - 1);
+  const bool wr = q == 0 && r < D;
+  const int64_t tot = (int64_t)n * D;
+  const int DD8 = D * D * 8, D8 = D * 8;
+  const double c = 1.0 / (betan[cix] * betan[cix]);
+  double* const v = work + 2 * boff[cix] * D;
+  const double sig = shift ? shift[cix] : 0.0;
+  const __amdgpu_buffer_rsrc_t Sb = raw_buffer(sinv + (size_t)boff[cix] * D * D, (int64_t)n * DD8);
+  const int ao = rr * D8 + q * KPL * 8, eo = rr * 8;
+  double* z = zs[side];
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  // sums over the workgroup's threads, two at a time
+  auto sum2 = [&](double& a, double& b) {
+    for (int o = 32; o > 0; o >>= 1) {
+      a += __shfl_xor(a, o);
+      b += __shfl_xor(b, o);
+    }
+    __syncthreads();
+    if (lane == 0) {
+      red[side][0] = a;
+      red[side][1] = b;
+    }
+    __syncthreads();
+    a = red[0][0] + red[1][0];
+    b = red[0][1] + red[1][1];
+  };
+  auto load = [&](double (&a)[KPL], int bead) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < KPL; j += 2) {
+      const d2 w = __builtin_bit_cast(d2, __builtin_amdgcn_raw_buffer_load_b128(Sb, ao + 8 * j, bead * DD8, 0));
+      a[j] = w.x;
+      a[j + 1] = w.y;
+    }
+  };
+  auto row = [&](const double (&a)[KPL], const double* u) __attribute__((always_inline)) {
+    double t0 = 0.0, t1 = 0.0;
+#pragma unroll
+    for (int j = 0; j < KPL; j += 2) {
+      const d2 w = *reinterpret_cast<const d2*>(u + q * KPL + j);
+      t0 = fma(a[j], w.x, t0);
+      t1 = fma(a[j + 1], w.y, t1);
+    }
+    const double t = t0 + t1;
+    return t + dpp_mov<0xB1>(t);  // the row's other lane
+  };
+  double sc = 0.0, zero = 0.0;  // sc src is the normalised v
+  for (int64_t e = tid; e < tot; e += 128) {
+    const double t = fresh ? start_entry(e) : v[e];
+    if (fresh) v[e] = t;
+    sc += t * t;
+  }
+  if (lane < 2 * KPL) z[lane] = zm[lane] = 0.0;
+  sum2(sc, zero);
+  sc = 1.0 / sqrt(sc);
+  double *src = v, *dst = v + tot;
+  const int K = side ? n - 1 - h : h;
+  // the K steps of this side; the previous vectors at sc src, this iteration's in dst
+  auto sweep = [&](auto Fwd, int K, double& mu, double& yy) __attribute__((always_inline)) {
+    constexpr bool FWD = decltype(Fwd)::value;
+    const __amdgpu_buffer_rsrc_t Vb = raw_buffer(src, tot * 8), Tb = raw_buffer(dst, tot * 8);
+    auto bead = [&](int k) {
+      const int i = FWD ? (side ? n - 1 - k : k) : (side ? h + 1 + k : h - 1 - k);
+      return min(max(i, 0), n - 1);
+    };
+    auto next = [&](int k) { return min(max(bead(k) + (side ? -1 : 1), 0), n - 1); };
+    double a[P][KPL], e[P], ve[P];
+    auto fetch = [&](int s, int k) __attribute__((always_inline)) {
+      load(a[s], bead(k));
+      ve[s] = buffer_ld(Vb, eo, (FWD ? next(k) : bead(k)) * D8);
+      if (!FWD) e[s] = buffer_ld(Tb, eo, bead(k) * D8);
+    };
+#pragma unroll
+    for (int s = 0; s < P; ++s) fetch(s, s);
+    for (int k0 = 0; k0 < K; k0 += P) {
+#pragma unroll
+      for (int s = 0; s < P; ++s) {
+        const int k = k0 + s;
+        if (k < K) {  // wave-uniform
+          const double t = row(a[s], z), vi = sc * ve[s], ti = FWD ? 0.0 : e[s];
+          fetch(s, k + P);
+          double out, nz;
+          if (FWD) {
+            // side 1 brings its c t alone to the middle bead, which side 0 gives its v
+            const bool coupled = side || k >= 1, own = !(side && k == K - 1);
+            out = t;
+            nz = (own ? vi : 0.0) + (coupled ? c * t : 0.0);
+          } else {
+            out = nz = ti + c * t;
+            mu += wr ? out * vi : 0.0;
+            yy += wr ? out * out : 0.0;
+          }
+          wave_sync();  // every lane has read z
+          if (wr) {
+            dst[(int64_t)bead(k) * D + r] = out;
+            z[r] = nz;
+          }
+          wave_sync();
+        }
+      }
+    }
+  };
+  double eta = 0.0, prev = 0.0;
+  for (int it = 0; it < iters; ++it) {
+    double mu = 0.0, yy = 0.0, ah[KPL];
+    if (lane < D) z[lane] = sc * src[side ? tot - D + lane : lane];  // z_0 and z_{n-1}
+    load(ah, h);
+    wave_sync();
+    sweep(std::true_type{}, K, mu, yy);
+    __syncthreads();
+    if (side == 0) {  // the middle bead: y_h = S_h^-1 z_h, from where both sides go back
+      if (lane < D) zm[lane] = zs[0][lane] + (h >= 1 ? zs[1][lane] : 0.0);
+      wave_sync();
+      const double t = row(ah, zm);
+      if (wr) {
+        dst[(int64_t)h * D + r] = t;
+        zs[0][r] = zs[1][r] = t;
+        mu += t * (sc * src[(int64_t)h * D + r]);
+        yy += t * t;
+      }
+    }
+    // y_0 = t_0, and nothing comes back to bead 1 of n = 2 (h = 0): bead 0 is coupled to no other
+    if (wr && K > 0 && (side == 0 || h == 0)) {
+      const int64_t o = (side ? D : 0) + r;
+      const double t = dst[o];
+      mu += t * (sc * src[o]);
+      yy += t * t;
+    }
+    __syncthreads();
+    sweep(std::false_type{}, side ? (h ? K : 0) : max(K - 1, 0), mu, yy);
+    sum2(mu, yy);  // and every y is written
+    sc = 1.0 / sqrt(yy);
+    double* sw = src;
+    src = dst;
+    dst = sw;
+    eta = sig + 1.0 / mu;
+    if (it > 2 && fabs(eta - prev) <= tol * fabs(eta)) break;  // block-uniform
+    prev = eta;
+  }
+  for (int64_t e = tid; e < tot; e += 128) v[e] = sc * src[e];
   if (tid == 0) eta1[cix] = eta;
 }
 
@@ -1637,13 +1794,15 @@ int ring_lowest_eigen(rp_ring* r, const std::vector<int>& ng, double* eta) {
     cleanup();
     return rc;
   }
-  // lanes per block row, prefetch depth and sides of the block solve: 8 x 4 columns, 12 steps
-  // ahead, from both ends for D <= 32; 4 x 16 columns, 4 steps ahead (the registers of a deeper
-  // ring) up to kMaxD
+  // above 32 dofs: 4 lanes x 16 columns per block row, 4 steps ahead (the registers of a deeper
+  // prefetch)
   auto eta1 = [&](const double* shift, int iters, int fresh, double tol, const int* act) -> int {
-    auto kern = r->D <= 32 ? ring_eta1_kernel<8, 4, 12, 2> : ring_eta1_kernel<4, 16, 4, 1>;
-    kern<<<C, kRingThreads * (r->D <= 32 ? 2 : 1), 0, r->s>>>(r->D, r->d_n.p, r->d_boff.p, r->d_betan.p, r->d_sinv.p,
-                                       r->d_work.p, shift, iters, fresh, tol, act, r->d_eta.p);
+    auto kern = r->D <= 28   ? ring_eta1_wave_kernel<14, 7>
+                : r->D <= 32 ? ring_eta1_wave_kernel<16, 6>
+                             : ring_eta1_kernel<4, 16, 4>;
+    kern<<<C, r->D <= 32 ? 128 : kRingThreads, 0, r->s>>>(r->D, r->d_n.p, r->d_boff.p, r->d_betan.p,
+                                                         r->d_sinv.p, r->d_work.p, shift, iters, fresh,
+                                                         tol, act, r->d_eta.p);
     RP_HIP(hipGetLastError());
     return RP_OK;
   };
@@ -1656,8 +1815,8 @@ int ring_lowest_eigen(rp_ring* r, const std::vector<int>& ng, double* eta) {
   std::vector<double> mu(C), sh(C, 0.0);
   std::vector<int> act(C);
   // inverse iteration on the unshifted factors, from a fixed generic start: two iterations for
-  // an upper bound that the first multisection round can work with (six gave it to a per cent,
-  // and cost 5.4 ms of 34.6 on 256 chains of the 27-dof EVB for 4 ms of later rounds)
+  // an upper bound that the first multisection round can work with (six cost
+  // 256 chains of the 27-dof EVB 3 ms more of 34.6 than the later rounds gave back)
   if ((rc = eta1(nullptr, 2, 1, 0.0, nullptr)) || (rc = fetch_eta(mu))) return cleanup(), rc;
   // chains with negative eigenvalues: four more, then Rayleigh-quotient refinement toward the
   // one nearest zero
