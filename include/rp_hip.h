@@ -206,7 +206,8 @@ int rp_batch_family_shape(rp_batch *b, int fam, int *waves, int *units_per_wave,
 /* launch shape: steps per launch (>= 1; 0 keeps the current value) and the wave budget of a
  * workgroup (2, 4 or 8 for every family; 0 keeps each family's value; 8 applies to families of
  * at most 16 MFMA units, 2 to families of at most 2 units with at most 2 dof tiles, the others
- * take 4).  Until a budget is set, polymers per workgroup are picked by occupancy.
+ * take 4).  Until a budget is set, polymers per workgroup are picked by occupancy, and batches of
+ * at most one workgroup per compute unit get helper waves.
  * rp_batch_autotune times, on the live batch (state saved and
  * restored), 2, 4 and 8 waves per family from each family's own launch timings, then the
  * steps-per-launch candidates; it keeps the fastest and reports the steps and the most
@@ -298,7 +299,8 @@ int rp_ring_set_preconditioner(rp_ring *r, double sigma);
  * at once, resident on the device (iterates, gradients and correction pairs stay in HBM;
  * gradients from the adjoint).  x_inout as rp_ring_set_x; action[c] = U_M at the optimum;
  * iters[c]; status[c] = 0 converged, 1 abnormal line search, 2 iteration cap (maxiter, or
- * 200000 evaluations when maxiter = 0).  The optimum is left as the ring's x. */
+ * 200000 evaluations when maxiter = 0).  The optimum is left as the ring's x; the search's
+ * vectors, 5 + 2 (m + 1) of the chains' total size, stay allocated until the ring is destroyed. */
 int rp_instanton(rp_ring *r, double pgtol, double factr, int m, int maxiter, double *x_inout,
                  double *action, int *iters, int *status);
 /* adjoint sensitivity dU_M/dtheta of each chain to the potential parameters
