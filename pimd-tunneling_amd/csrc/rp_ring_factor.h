@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(128, 2) ring_factor_kernel(
     wt[e] = r < D && q < D ? 1.0 / sqrt(massd[r] * massd[q]) : 0.0;
   }
   __syncthreads();
-  const __amdgpu_buffer_rsrc_t Bb = raw_buffer(blocks + (size_t)boff[c] * D * D, (int64_t)n * DD8);
+  const double* const chain = blocks + (size_t)boff[c] * D * D;
   int vo[RT][4], co[RT];  // byte offsets of the lane's rows and columns, clamped to the block
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
@@ -60,14 +60,15 @@ __global__ void __launch_bounds__(128, 2) ring_factor_kernel(
     for (int j = 0; j < 4; ++j) vo[t][j] = min(16 * t + 4 * j + g, D - 1) * D * 8;
   }
   d4 acc[RT][RT], nxt[RT][RT];
+  // a buffer per block: a chain's blocks may take more than its 32-bit offsets reach
   auto load = [&](int bead) __attribute__((always_inline)) {
-    const int so = bead * DD8;
+    const __amdgpu_buffer_rsrc_t Bb = raw_buffer(chain + (size_t)bead * D * D, DD8);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int ct = 0; ct < RT; ++ct)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) nxt[rt][ct][j] = buffer_ld(Bb, vo[rt][j] + co[ct], so);
+        for (int j = 0; j < 4; ++j) nxt[rt][ct][j] = buffer_ld(Bb, vo[rt][j] + co[ct], 0);
   };
   double mant = 1.0;  // the determinant so far: mant 2^ex, and the negative pivots
   int ex = 0, neg = 0;

@@ -1,4 +1,5 @@
-"""Ring entry points at the edges of their input: what is not finite."""
+"""Ring entry points at the edges of their input: what is not finite, and chains whose blocks
+take more bytes than 32 bits count."""
 import numpy as np
 import pytest
 
@@ -30,3 +31,33 @@ def test_inertia_of_a_chain_that_is_not_finite(natom, value, bead):
     with pytest.raises(RpError):
         ring.logdet(skip_lowest=True)
     ring.close()
+
+
+def test_determinant_of_a_chain_beyond_4_gib_of_blocks():
+    """530,000 beads of 32 dofs are 4.3 GB of blocks; the beads past the 4 GiB mark sit elsewhere
+    in the potential than all others.  The quartic's dofs are separable and alike here, so the
+    determinant is a scalar recurrence over the beads to the 32nd power: with the reference's
+    coupling S_0 = a_0, S_1 = a_1, S_i = a_i - 1 / (betan^4 S_{i-1}).  Bar, relative to a
+    logarithm of 1.5e8: a few roundings of 1.1e-16 in each of 1.7e7 pivots, all alike and so
+    adding up, are 1e-8, the logarithm's own rounding is as much; 2e-15 is 3e-7.  One wrong
+    block of the 5,712 in question is 7."""
+    D, n, mark, betan = 32, 530_000, 2 ** 32 // (32 * 32 * 8), 100.0
+    sp = specs.quartic(natom=D)
+    h, x0, m = sp.dp[0], sp.dp[1], sp.mass[0]
+    x = np.full((D, n), x0)
+    x[:, mark:] = 0.8 * x0
+    ring = Ring(Pes(sp), sp.mass, [n], [betan], sp.well1, sp.well2)
+    ring.set_x([x])
+    ld, nn, _ = ring.logdet(skip_lowest=False)
+    with pytest.raises(RpError):  # the block solve's offsets stay within 31 bits
+        ring.logdet(skip_lowest=True)
+    ring.close()
+    a = (4.0 * h / x0 ** 2 * (3.0 * x[0] ** 2 / x0 ** 2 - 1.0) / m + 2.0 / betan ** 2).tolist()
+    want, s = np.log(a[0]), a[1]
+    piv = [s]
+    for v in a[2:]:
+        s = v - 1.0 / (betan ** 4 * s)
+        piv.append(s)
+    want = D * (want + np.sum(np.log(piv)))
+    assert nn[0] == 0 and abs(want) > 1e8
+    assert abs(ld[0] - want) <= 2e-15 * abs(want), (ld[0], want)
