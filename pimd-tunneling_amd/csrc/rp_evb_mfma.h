@@ -62,11 +62,19 @@ __host__ __device__ inline int evb_kick_lds_size(int DC, uint32_t moved) {
   return 2 + 4 * DC + DC * (DC + 1) + (moved ? DC * evb_diff_stride(moved) : 0);
 }
 
-// K-chunks of 4 dofs with a dof that the wells' permutation moves, one bit each
+// K-chunks of 4 dofs with a dof whose column differs between the wells, one bit each: those of
+// an atom that the map does not send to itself, or that another atom (of a map which is no
+// permutation) or no atom is sent to, as rp_pes_create inverts it
 inline uint32_t evb_moved(const rp_pes* pes) {
+  const int na = pes->natom, nd = pes->ndim;
   uint32_t moved = 0;
-  for (int d = 0; d < pes->ndof; ++d)
-    if (pes->ip[d / pes->ndim] != d / pes->ndim) moved |= 1u << (d / 4);
+  for (int a = 0; a < na; ++a) {
+    int from = -1;  // the last atom sent to a
+    for (int k = 0; k < na; ++k)
+      if (pes->ip[k] == a) from = k;
+    if (from != a)
+      for (int d = a * nd; d < (a + 1) * nd; ++d) moved |= 1u << (d / 4);
+  }
   return moved;
 }
 
@@ -74,7 +82,7 @@ inline uint32_t evb_moved(const rp_pes* pes) {
 // (evb_kick_lds_size): vectors and matrices zero-padded to DC = 16 DT, matrix rows of
 // stride DC + 1 (the y GEMM reads a column of 16 rows per lane group: an odd stride puts
 // them in distinct banks).  The second matrix is the difference WtB - WtA: the wells differ by
-// a permutation of atoms, so its columns are zero at every atom the permutation leaves.
+// a permutation of atoms, so its columns are zero at every atom the permutation leaves (evb_moved).
 template <int M, int DT>
 __device__ __forceinline__ void stage_evb_kick(const double* __restrict__ dp, double* PL, uint32_t moved,
                                                int tid, int nthreads) {
