@@ -258,12 +258,14 @@ int rp_ring_hvp_device(rp_ring *r, const double *v, double *hv);
  * grad.  rp_ring_hvp_stream: x becomes the ring's coordinates, hv = H(x) v, times the chains'
  * weights w[nchain] unless NULL.  rp_ring_weight_stream: out = w[c] g over every chain.
  * rp_ring_dot_stream: out[c] = a . b over chain c.  A potential that lives on the host gets
- * RP_ERR_ARG from the first two. */
+ * RP_ERR_ARG from the first two, a stream of another GPU from all of them.  rp_ring_device: the
+ * GPU that holds the ring. */
 int rp_ring_action_stream(rp_ring *r, const double *x, double *energy, double *grad, void *stream);
 int rp_ring_hvp_stream(rp_ring *r, const double *x, const double *v, const double *w, double *hv,
                        void *stream);
 int rp_ring_weight_stream(rp_ring *r, const double *w, const double *g, double *out, void *stream);
 int rp_ring_dot_stream(rp_ring *r, const double *a, const double *b, double *out, void *stream);
+int rp_ring_device(const rp_ring *r, int *device);
 /* UMhessian (:155-217) of chain `chain`: the reference's answer(ndof+1, n*ndof), LAPACK
  * lower band storage in column-major order (AB(1+i-j, j) at band[j*(ndof+1) + i-j], 0-based),
  * bead blocks from ndof forward-over-reverse sweeps; singlewell reuses bead 1's block

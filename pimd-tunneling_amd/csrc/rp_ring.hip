@@ -1238,6 +1238,7 @@ struct rp_ring {
   std::vector<int64_t> off, boff;
   int64_t tot = 0, nbeads = 0;
   int nmax = 0;  // the longest chain
+  int dev = 0;  // the GPU that holds the ring
   hipStream_t s = nullptr;
   hipEvent_t ev = nullptr;  // the last stream-ordered call's work (rp_ring_*_stream)
   DevBuf<double> d_x, d_g, d_v, d_hv, d_e, d_ab, d_betan, d_massd, d_blocks, d_sinv, d_work, d_ld,
@@ -1431,6 +1432,7 @@ extern "C" int rp_ring_create(rp_pes* pes, const double* mass, int nchain, const
   for (int at = 0; at < r->natom; ++at)
     for (int j = 0; j < r->ndim; ++j) massd[at * r->ndim + j] = mass[at];
   if ((rc = [&]() -> int {
+        RP_HIP(hipGetDevice(&r->dev));
         RP_HIP(hipStreamCreateWithFlags(&r->s, hipStreamNonBlocking));
         int q;
         if ((q = r->d_x.alloc(r->tot)) || (q = r->d_g.alloc(r->tot)) || (q = r->d_v.alloc(r->tot)) ||
@@ -1602,10 +1604,25 @@ extern "C" int rp_ring_hvp_device(rp_ring* r, const double* v, double* hv) {
   return RP_OK;
 }
 
+extern "C" int rp_ring_device(const rp_ring* r, int* device) {
+  RP_REQUIRE(r && device, "rp_ring_device: bad arguments");
+  *device = r->dev;
+  return RP_OK;
+}
+
 // Stream-ordered entry points: the work is queued on the caller's stream, ordered with every
 // other call on the ring by one event (the caller's stream waits for what the ring last
 // queued, the ring's own stream for this).
+// A kernel on another GPU's stream would run there, on buffers of this one.
+static int stream_check(const rp_ring* r, hipStream_t s) {
+  hipDevice_t dev = -1;
+  RP_HIP(hipStreamGetDevice(s, &dev));
+  RP_REQUIRE(dev == r->dev, "rp_ring_*_stream: the stream belongs to GPU %d, the ring to GPU %d", (int)dev, r->dev);
+  return RP_OK;
+}
 static int stream_begin(rp_ring* r, hipStream_t s) {
+  int rc = stream_check(r, s);
+  if (rc) return rc;
   if (!r->ev) RP_HIP(hipEventCreateWithFlags(&r->ev, hipEventDisableTiming));
   else RP_HIP(hipStreamWaitEvent(s, r->ev, 0));
   return RP_OK;
@@ -1647,6 +1664,8 @@ extern "C" int rp_ring_hvp_stream(rp_ring* r, const double* x, const double* v, 
 extern "C" int rp_ring_weight_stream(rp_ring* r, const double* w, const double* g, double* out,
                                      void* stream) {
   RP_REQUIRE(r && w && g && out, "rp_ring_weight_stream: bad arguments");
+  const int rc = stream_check(r, (hipStream_t)stream);
+  if (rc) return rc;
   ring_weight_kernel<<<vec_grid(r), kVecThreads, 0, (hipStream_t)stream>>>(r->d_off.p, r->d_n.p, r->D, w, g, out);
   RP_HIP(hipGetLastError());
   return RP_OK;
@@ -1654,6 +1673,8 @@ extern "C" int rp_ring_weight_stream(rp_ring* r, const double* w, const double* 
 
 extern "C" int rp_ring_dot_stream(rp_ring* r, const double* a, const double* b, double* out, void* stream) {
   RP_REQUIRE(r && a && b && out, "rp_ring_dot_stream: bad arguments");
+  const int rc = stream_check(r, (hipStream_t)stream);
+  if (rc) return rc;
   ring_dot_kernel<<<r->nchain, kRingThreads, 0, (hipStream_t)stream>>>(r->d_off.p, r->d_n.p, r->D, a, b, out);
   RP_HIP(hipGetLastError());
   return RP_OK;

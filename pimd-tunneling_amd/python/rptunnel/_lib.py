@@ -109,6 +109,7 @@ _SIGS = {
     "rp_ring_hvp_stream": [vp, vp, vp, vp, vp, vp],
     "rp_ring_weight_stream": [vp, vp, vp, vp, vp],
     "rp_ring_dot_stream": [vp, vp, vp, vp, vp],
+    "rp_ring_device": [vp, ip],
     "rp_ring_hessian_band": [vp, C.c_int, C.c_int, dp],
     "rp_ring_logdet": [vp, C.c_int, C.c_int, dp, ip, dp],
     "rp_ring_lowest_eigs": [vp, C.c_int, C.c_int, dp],

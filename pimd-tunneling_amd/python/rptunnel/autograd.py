@@ -8,8 +8,9 @@ forward-over-reverse Hessian-vector product (rp_ring_hvp), so first and second
 derivatives of any scalar built from the actions come from the hand-written kernels.
 A tensor on the GPU stays there: the library's stream-ordered entry points
 (rp_ring_action_stream, rp_ring_hvp_stream and the per-chain weights and dot products) queue
-their kernels on torch's current stream, so nothing waits for the host.  CPU tensors, and
-potentials that live on the host, go through the host entry points.
+their kernels on torch's current stream, so nothing waits for the host.  CPU tensors, tensors
+on another GPU than the ring's, and potentials that live on the host go through the host entry
+points.
 
 The Ring is the function's workspace: every evaluation loads x into its device coordinates
 and leaves them there (keep an optimised instanton in a Ring of its own).  The gradient made
@@ -36,7 +37,8 @@ def _flat(chains) -> torch.Tensor:
 
 
 def _on_device(ring: Ring, x: torch.Tensor) -> bool:
-    return x.is_cuda and ring.pes.spec is not None  # a host potential has no spec
+    # on the ring's own GPU, and no host potential (which has no spec)
+    return x.is_cuda and x.device.index == ring.device and ring.pes.spec is not None
 
 
 def _f64(t: torch.Tensor) -> torch.Tensor:

@@ -34,6 +34,9 @@ class Ring:
                                        L.ptr(self.betan), L.ptr(self.a), L.ptr(self.b),
                                        int(fixedends), C.byref(h)))
         self.h = h
+        dev = C.c_int(0)
+        L.check(L.lib().rp_ring_device(h, C.byref(dev)))
+        self.device = dev.value  # the GPU that holds the ring
         self.off = np.concatenate([[0], np.cumsum([k * D for k in self.n])])
 
     def close(self):

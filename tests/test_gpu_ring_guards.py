@@ -1,9 +1,10 @@
-"""Ring entry points at the edges of their input: what is not finite, and chains whose blocks
-take more bytes than 32 bits count."""
+"""Ring entry points at the edges of their input: what is not finite, chains whose blocks take
+more bytes than 32 bits count, tensors that are not on the ring's GPU."""
 import numpy as np
 import pytest
+import torch
 
-from rptunnel import Pes, Ring, RpError, specs
+from rptunnel import Pes, Ring, RpError, autograd, specs
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +62,30 @@ def test_determinant_of_a_chain_beyond_4_gib_of_blocks():
     want = D * (want + np.sum(np.log(piv)))
     assert nn[0] == 0 and abs(want) > 1e8
     assert abs(ld[0] - want) <= 2e-15 * abs(want), (ld[0], want)
+
+
+def test_tensors_on_another_gpu_keep_off_the_ring_streams(monkeypatch):
+    """A tensor whose GPU is not the ring's goes through the host entry points, first and second
+    derivatives too, and comes back to its own GPU; none of the stream-ordered calls sees it.
+    With one GPU at hand the ring is made to name another one."""
+    sp = specs.coupled2d()
+    ns = [5, 33]
+    ring = Ring(Pes(sp), sp.mass, ns, [9.0, 7.0], sp.well1, sp.well2)
+    x0 = torch.from_numpy(np.random.default_rng(2).standard_normal(2 * sum(ns)))
+    v = torch.linspace(-1.0, 1.0, x0.numel(), dtype=torch.float64)
+
+    def derivatives():
+        x = x0.cuda().requires_grad_(True)
+        u = autograd.ring_action(x, ring)
+        (g,) = torch.autograd.grad((u * u).sum(), x, create_graph=True)
+        (h,) = torch.autograd.grad(g @ v.cuda(), x)
+        assert u.device == g.device == h.device == x.device
+        return [t.detach().cpu() for t in (u, g, h)]
+
+    assert ring.device == torch.cuda.current_device()
+    want = derivatives()
+    ring.device += 1
+    monkeypatch.setattr(autograd, "_call", lambda *a: pytest.fail("a stream-ordered call"))
+    for got, ref in zip(derivatives(), want):
+        assert torch.allclose(got, ref, rtol=1e-12, atol=0.0)
+    ring.close()
