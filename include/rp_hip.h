@@ -258,8 +258,8 @@ int rp_ring_hvp_device(rp_ring *r, const double *v, double *hv);
  * grad.  rp_ring_hvp_stream: x becomes the ring's coordinates, hv = H(x) v, times the chains'
  * weights w[nchain] unless NULL.  rp_ring_weight_stream: out = w[c] g over every chain.
  * rp_ring_dot_stream: out[c] = a . b over chain c.  A potential that lives on the host gets
- * RP_ERR_ARG from the first two, a stream of another GPU from all of them.  rp_ring_device: the
- * GPU that holds the ring. */
+ * RP_ERR_ARG from the first two, a stream under capture RP_ERR_STATE, a stream of another GPU
+ * RP_ERR_ARG from all of them.  rp_ring_device: the GPU that holds the ring. */
 int rp_ring_action_stream(rp_ring *r, const double *x, double *energy, double *grad, void *stream);
 int rp_ring_hvp_stream(rp_ring *r, const double *x, const double *v, const double *w, double *hv,
                        void *stream);

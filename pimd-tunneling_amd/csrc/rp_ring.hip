@@ -1623,6 +1623,14 @@ static int stream_check(const rp_ring* r, hipStream_t s) {
 static int stream_begin(rp_ring* r, hipStream_t s) {
   int rc = stream_check(r, s);
   if (rc) return rc;
+  // under capture the ring's own stream would join the caller's graph without an end, and a
+  // replay would not be ordered with the ring's other calls
+  if (s) {  // the default stream is never captured
+    hipStreamCaptureStatus cap;
+    RP_HIP(hipStreamIsCapturing(s, &cap));
+    if (cap != hipStreamCaptureStatusNone)
+      return set_error(RP_ERR_STATE, "rp_ring_*_stream: a ring's evaluations cannot be captured");
+  }
   if (!r->ev) RP_HIP(hipEventCreateWithFlags(&r->ev, hipEventDisableTiming));
   else RP_HIP(hipStreamWaitEvent(s, r->ev, 0));
   return RP_OK;

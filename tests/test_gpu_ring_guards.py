@@ -1,5 +1,5 @@
 """Ring entry points at the edges of their input: what is not finite, chains whose blocks take
-more bytes than 32 bits count, tensors that are not on the ring's GPU."""
+more bytes than 32 bits count, tensors that are not on the ring's GPU, streams under capture."""
 import numpy as np
 import pytest
 import torch
@@ -88,4 +88,38 @@ def test_tensors_on_another_gpu_keep_off_the_ring_streams(monkeypatch):
     monkeypatch.setattr(autograd, "_call", lambda *a: pytest.fail("a stream-ordered call"))
     for got, ref in zip(derivatives(), want):
         assert torch.allclose(got, ref, rtol=1e-12, atol=0.0)
+    ring.close()
+
+
+@pytest.mark.parametrize("used_before", [False, True])
+def test_evaluations_are_refused_under_capture(used_before):
+    """A ring's evaluation under capture is an error that leaves the capture, the graph and the
+    ring as they were: the graph replays what else it holds, the ring's later calls are right."""
+    sp = specs.coupled2d()
+    ns = [5, 33]
+    ring = Ring(Pes(sp), sp.mass, ns, [9.0, 7.0], sp.well1, sp.well2)
+    rng = np.random.default_rng(2)
+    chains = [0.3 * rng.standard_normal((2, n)) for n in ns]
+    flat = torch.from_numpy(ring.pack(chains)).cuda()
+    if used_before:
+        autograd.ring_action(flat + 1.0, ring)
+    a = torch.arange(4.0, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        b = a + 1.0
+        with pytest.raises(RpError, match="captured"):
+            autograd.ring_action(flat, ring)
+        c = b * 2.0
+    for k in range(3):
+        a.fill_(float(k))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.all(c == 2.0 * (k + 1))
+        x = (flat * (1.0 + k)).requires_grad_(True)
+        u = autograd.ring_action(x, ring)
+        (g,) = torch.autograd.grad(u.sum(), x)
+        gw, ew = ring.UMforceenergy([(1.0 + k) * v for v in chains])
+        assert np.allclose(u.detach().cpu().numpy(), ew, rtol=1e-13, atol=0.0)
+        assert np.allclose(g.cpu().numpy(), ring.pack(gw), rtol=1e-12, atol=1e-15)
     ring.close()
