@@ -8,6 +8,7 @@
 #include <cstring>
 
 #include "rp_evb_mfma.h"
+#include "rp_multisect.h"
 #include "rp_ring.h"
 #include <algorithm>
 
@@ -1803,7 +1804,7 @@ static int ring_factor(rp_ring* r, int ntask, const double* shift, const int* ch
 // Sylvester's inertia: lo with no eigenvalue below it (0 to start), hi with at least one (the
 // Rayleigh quotient of a few unshifted inverse iterations, an upper bound on eta_1), and h1,
 // the largest shift seen with exactly one below it (so eta_2 >= h1).  Rounds of multisection
-// (three shifts per chain in one launch) narrow it until inverse iteration shifted to lo,
+// (seven shifts or more per chain in one launch) narrow it until inverse iteration shifted to lo,
 // which converges to the eigenvalue nearest lo, i.e. eta_1, contracts by
 // (hi - lo) / (h1 - lo) <= 1/4 per iteration; that iteration then gives eta_1 to the last
 // bits.  A chain whose bracket closes first takes its midpoint.
@@ -1813,8 +1814,7 @@ int ring_lowest_eigen(rp_ring* r, const std::vector<int>& ng, double* eta) {
   if ((int64_t)r->nmax * r->D * r->D * 8 >= ((int64_t)1 << 31))
     return set_error(RP_ERR_ARG, "ring log-determinant: a chain's block factors exceed 2 GiB");
   if (r->d_work.n < 2 * (size_t)r->tot && (rc = r->d_work.alloc(2 * (size_t)r->tot))) return rc;
-  constexpr int M = 7, kFill = 512;  // shifts per chain and multisection round; tasks at least
-  const size_t ntask = std::max((size_t)M * C, (size_t)kFill);
+  const size_t ntask = multisect_tasks(C);
   DevBuf<double> d_shift, d_tld;
   DevBuf<int> d_act, d_map, d_cnt;
   auto cleanup = [&]() { d_shift.free(); d_tld.free(); d_act.free(); d_map.free(); d_cnt.free(); };
@@ -1892,19 +1892,12 @@ int ring_lowest_eigen(rp_ring* r, const std::vector<int>& ng, double* eta) {
     std::vector<double> tsh;
     for (int c = 0; c < C; ++c)
       if (open[c] && needs_more(c)) left.push_back(c);
-    // a round of up to kFill tasks takes as long as its longest chain, so a few chains get more
-    // shifts each: on 256 chains of the 27-dof EVB the last two rounds, 12 chains and one, took
-    // 1.65 ms each with seven
-    const int m = left.empty() ? M : std::max(M, std::min(63, kFill / (int)left.size()));
-    for (int c : left) {
+    const int m = multisect_shifts((int)left.size());
+    for (int c : left)
       for (int k = 1; k <= m; ++k) {
         map.push_back(c);
-        // the first round's shifts crowd toward hi (eta_1 is usually within a few per cent
-        // of the Rayleigh quotient), later rounds split the bracket evenly
-        const double f = round == 0 ? 1.0 - std::ldexp(1.0, -k * M / m) : (double)k / (m + 1);
-        tsh.push_back(lo[c] + (hi[c] - lo[c]) * f);
+        tsh.push_back(multisect_shift(lo[c], hi[c], round == 0, k, m));
       }
-    }
     if (map.empty()) break;
     const std::vector<int> ord = longest_first(r, map);
     permute(map, ord);
