@@ -208,10 +208,10 @@ int rp_batch_family_shape(rp_batch *b, int fam, int *waves, int *units_per_wave,
  * at most 16 MFMA units, 2 to families of at most 2 units with at most 2 dof tiles, the others
  * take 4).  Until a budget is set, polymers per workgroup are picked by occupancy, and batches of
  * at most one workgroup per compute unit get helper waves.
- * rp_batch_autotune times, on the live batch (state saved and
- * restored), 2, 4 and 8 waves per family from each family's own launch timings, then the
- * steps-per-launch candidates; it keeps the fastest and reports the steps and the most
- * frequent wave count. */
+ * rp_batch_autotune times, on the live batch (state saved and restored), each family by itself
+ * with no budget set and with 2, 4 and 8 waves, then the steps-per-launch candidates; a budget is
+ * set only where it is faster than none.  It reports the steps and the most frequent wave
+ * budget, as rp_batch_family_shape gives it. */
 int rp_batch_set_launch(rp_batch *b, int steps_per_launch, int waves);
 /* enable = 1: rp_batch_run replays each family's block of steps_per_launch steps as a captured
  * HIP graph, between that family's timing events, when it draws from the Philox streams.

@@ -57,6 +57,7 @@ struct rp_batch {
   std::vector<hipStream_t> side;
   std::vector<int> lane;
   hipEvent_t fork = nullptr;
+  bool in_turn = false;  // launch the families one after another all the same (autotune)
   // rp_batch_set_graphs: each family's launch of a step block (the last family's followed by
   // the step counter update) captured as a HIP graph and replayed between its timing events; a
   // graph is rebuilt when anything it captured changes.  Off by default: a block is one kernel
@@ -608,8 +609,9 @@ static int run_block(rp_batch* b, int steps, int64_t imin, const double* dn, int
       RP_HIP(hipEventRecord(b->fev[2 * fi + 1], b->s));
     }
   } else {
-    auto stream = [&](size_t fi) { return b->lane[fi] ? b->side[b->lane[fi] - 1] : b->s; };
-    if (!b->side.empty()) {
+    const bool apart = !b->side.empty() && !b->in_turn;
+    auto stream = [&](size_t fi) { return apart && b->lane[fi] ? b->side[b->lane[fi] - 1] : b->s; };
+    if (apart) {
       RP_HIP(hipEventRecord(b->fork, b->s));
       for (hipStream_t st : b->side) RP_HIP(hipStreamWaitEvent(st, b->fork, 0));
     }
@@ -634,10 +636,11 @@ static int run_block(rp_batch* b, int steps, int64_t imin, const double* dn, int
     size_t fi = b->fam.size();
     while (fi > 0 && !rc) rc = launch(--fi);
     // s waits for what the other streams got, once it has its own; after a failure too
-    for (hipStream_t st : b->side) {
-      RP_HIP(hipEventRecord(b->fork, st));
-      RP_HIP(hipStreamWaitEvent(b->s, b->fork, 0));
-    }
+    if (apart)
+      for (hipStream_t st : b->side) {
+        RP_HIP(hipEventRecord(b->fork, st));
+        RP_HIP(hipStreamWaitEvent(b->s, b->fork, 0));
+      }
     if (rc) return rc;
   }
   RP_HIP(hipStreamSynchronize(b->s));  // which waits for every family
@@ -921,27 +924,37 @@ extern "C" int rp_batch_autotune(rp_batch* b, int trial_steps, int* best_steps, 
     return restore();
   };
   const int64_t steps0 = b->steps_done;
-  // 1. waves per family, from each family's own hipEvent-timed launches
+  // 1. waves per family, from each family's own hipEvent-timed launches, one family at a time:
+  // no budget set (0: groups by occupancy, helper waves for small batches; launch_batch_kind),
+  // and the budgets that fit.  A budget takes over only where it is faster by more than two runs
+  // of one kernel differ.  Each is run once before it is timed: its first launch loads its code.
   const size_t nf = b->fam.size();
   std::vector<double> best_ms(nf, 1e300), fam_ms;
-  std::vector<int> best_w(nf, 4);
+  std::vector<int> best_w(nf, 0);
+  auto set_waves = [&](Family& f, int w) {
+    f.waves = w ? fitted_waves(b, f, w) : default_waves(b->DT, f.NPAD);
+    f.waves_set = w != 0;
+  };
   double sec = 0.0;
-  for (int w : {2, 4, 8}) {
-    for (Family& f : b->fam) {
-      f.waves = fitted_waves(b, f, w);
-      f.waves_set = true;
-    }
-    if ((rc = trial(std::min(b->steps_per_launch, trial_steps), fam_ms, sec))) return rc;
+  b->in_turn = true;
+  for (int w : {0, 2, 4, 8}) {
+    for (Family& f : b->fam) set_waves(f, w);
+    for (int k = 0; k < 2; ++k)
+      if ((rc = trial(std::min(b->steps_per_launch, trial_steps), fam_ms, sec))) {
+        b->in_turn = false;
+        return rc;
+      }
     for (size_t fi = 0; fi < nf; ++fi)
-      if (b->fam[fi].waves == w && fam_ms[fi] < best_ms[fi]) {
+      if (w == 0 || (b->fam[fi].waves == w && fam_ms[fi] < (best_w[fi] ? 1.0 : 0.97) * best_ms[fi])) {
         best_ms[fi] = fam_ms[fi];
         best_w[fi] = w;
       }
   }
+  b->in_turn = false;
   int nw[9] = {0};
   for (size_t fi = 0; fi < nf; ++fi) {
-    b->fam[fi].waves = best_w[fi];
-    ++nw[best_w[fi]];
+    set_waves(b->fam[fi], best_w[fi]);
+    ++nw[b->fam[fi].waves];
   }
   // 2. steps per launch
   const int cands[] = {8, 32, 128};
