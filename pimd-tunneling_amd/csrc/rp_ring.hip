@@ -28,27 +28,18 @@ struct RingArgs {
   const double* massd;     // per dof
 };
 
-// A barrier that orders LDS only, so global loads and stores stay in flight across it (a
-// one-wave workgroup needs no hardware barrier at all: its LDS operations complete in issue
-// order).
-template <int T>
+// A barrier that orders LDS only, so global loads and stores stay in flight across it
 __device__ __forceinline__ void lds_sync() {
-  if constexpr (T == 64) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  } else {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int NT = kRingThreads>
 __device__ __forceinline__ double block_sum(double v, double* red) {
   const int tid = threadIdx.x;
   red[tid] = v;
   __syncthreads();
-  for (int s = NT / 2; s > 0; s >>= 1) {
+  for (int s = kRingThreads / 2; s > 0; s >>= 1) {
     if (tid < s) red[tid] += red[tid + s];
     __syncthreads();
   }
@@ -117,7 +108,7 @@ __global__ void __launch_bounds__(kRingTile) ring_um_kernel(RingArgs A, const do
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e;
-  lds_sync<kRingTile>();
+  lds_sync();
   if (threadIdx.x == 0) {
     double t = 0.0;
 #pragma unroll
@@ -593,7 +584,6 @@ __global__ void __launch_bounds__(kRingThreads) ring_param_grad_kernel(RingArgs 
 // kept for inverse iteration on the eigenvalue nearest zero.
 namespace {
 constexpr int kMaxD = 56;  // ndof bound of the log-determinant workspace (LDS)
-constexpr int kPinP = 3;   // elements per thread whose step operands are read up front
 
 // 1/x of a pivot: the hardware reciprocal estimate (about 26 correct bits) refined by two
 // Newton-Raphson steps r <- r + r (1 - x r), each doubling the correct bits.  The full
@@ -622,31 +612,29 @@ __device__ __forceinline__ double buffer_ld(__amdgpu_buffer_rsrc_t b, int voff, 
 #include "rp_ring_factor.h"
 
 // The factorisation for more than 32 dofs, from bead 0 to bead n-1.
-// T threads per chain.  Thread t owns the elements e = t + T q (q < P) of every D x D block,
-// so the Hessian block of the next bead is loaded into registers while the current one is
-// eliminated, and the Schur update uses the previous inverse where it sits in LDS.  The
-// Gauss-Jordan inverse runs without pivoting, double-buffered in LDS (one barrier per pair
-// of eliminations): the pivot of elimination k is the k-th pivot of the matrix's LDL^T
+// A workgroup per chain.  The next bead's Hessian block is loaded into registers while the
+// current one is eliminated, and the Schur update uses the previous inverse where it sits in
+// LDS.  The Gauss-Jordan inverse runs without pivoting, double-buffered in LDS (one barrier per
+// pair of eliminations): the pivot of elimination k is the k-th pivot of the matrix's LDL^T
 // factorisation (a ratio of leading principal minors), so their logs sum to log|det| and
 // their signs give the inertia (Sylvester).
 //
-// SYM: the lower triangle only.  The Gauss-Jordan iterates keep M[j][i] = s M[i][j], with
-// s = -1 exactly when one of i, j has been swept (a pivot already eliminated) and +1
-// otherwise, so thread t owns lower element t (r >= cc, row-major) and writes both it and its
-// mirror: P elements per thread cover D (D + 1) / 2 instead of D^2, the reads are the same,
-// and the LDS tile (PT elements per thread) still holds the whole matrix.  Threads beyond the
-// triangle own the pad element (D, D).
-template <int P, int T, bool SYM = false, int PT = P>
-__global__ void __launch_bounds__(T) ring_logdet_kernel(
+// Only the lower triangle is worked out.  The Gauss-Jordan iterates keep M[j][i] = s M[i][j],
+// with s = -1 exactly when one of i, j has been swept (a pivot already eliminated) and +1
+// otherwise, so thread t owns the lower elements t + kRingThreads q (r >= cc, row-major) and
+// writes each and its mirror: P elements per thread cover D (D + 1) / 2, and the LDS tile (PT
+// elements per thread) holds the whole matrix.  Threads beyond the triangle own the pad
+// element (D, D).
+template <int P, int PT>
+__global__ void __launch_bounds__(kRingThreads) ring_logdet_kernel(
     int D, const int* __restrict__ nn, const int64_t* __restrict__ boff,
     const double* __restrict__ betan, const double* __restrict__ massd,
     const double* __restrict__ blocks, const double* __restrict__ shift, double* __restrict__ sinv,
     double* __restrict__ logdet, int* __restrict__ nneg, const int* __restrict__ chain_of) {
-  // every LDS element t + T q exists, and so does every r D + k <= t + T q + D - 1 read for
-  // it (and k D + cc < D^2 <= T P); the elements beyond D*D hold values nobody reads back,
-  // which keeps every load and store unconditional (no branch, so the loads of the next
-  // block stay in flight).  Sized by T P, so several workgroups share a CU's LDS.
-  constexpr int kTile = T * PT + kMaxD;
+  // the pad element and what is read for it lie past D^2 <= kRingThreads PT and hold values
+  // nobody reads back, which keeps every load and store unconditional (no branch, so the loads
+  // of the next block stay in flight).  Sized by PT, so several workgroups share a CU's LDS.
+  constexpr int kTile = kRingThreads * PT + kMaxD;
   __shared__ double Sb[2][kTile];
   // one task per workgroup: chain c (task t of a chain_of map, else chain t) factored at
   // the shift of task t; outputs per task
@@ -658,18 +646,13 @@ __global__ void __launch_bounds__(T) ring_logdet_kernel(
   double wgt[P], diag[P], nxt[P];
 #pragma unroll
   for (int q = 0; q < P; ++q) {
-    const int e = tid + T * q;
-    if constexpr (SYM) {
-      int r = 0;
-      while ((r + 1) * (r + 2) / 2 <= e && r < D) ++r;  // row of lower element e
-      const bool pad = r >= D;
-      er[q] = pad ? D : r;
-      ec[q] = pad ? D : e - r * (r + 1) / 2;
-    } else {
-      er[q] = e / D;
-      ec[q] = e - er[q] * D;
-    }
-    ei[q] = SYM ? er[q] * D + ec[q] : e;
+    const int e = tid + kRingThreads * q;
+    int r = 0;
+    while ((r + 1) * (r + 2) / 2 <= e && r < D) ++r;  // row of lower element e
+    const bool pad = r >= D;
+    er[q] = pad ? D : r;
+    ec[q] = pad ? D : e - r * (r + 1) / 2;
+    ei[q] = er[q] * D + ec[q];
     mi[q] = ec[q] * D + er[q];
     eg[q] = min(ei[q], DD - 1);  // clamped index of the global block loads
     const int rm = min(er[q], D - 1), cm = min(ec[q], D - 1);
@@ -693,14 +676,14 @@ __global__ void __launch_bounds__(T) ring_logdet_kernel(
       const double prev = M[e];
       const double val = coupled ? v - c2 * prev : v;
       M[e] = val;
-      if constexpr (SYM) M[mi[q]] = val;  // A_i and S_{i-1}^-1 are symmetric
+      M[mi[q]] = val;  // A_i and S_{i-1}^-1 are symmetric
     }
     // the next bead's block (a valid address for the last bead too), in flight during the
     // elimination
     const double* nb = base + (size_t)min(i + 1, n - 1) * DD;
 #pragma unroll
     for (int q = 0; q < P; ++q) nxt[q] = nb[eg[q]];
-    lds_sync<T>();
+    lds_sync();
     // eliminations two pivots at a time (a 2 x 2 pivot block, inverted explicitly, is two
     // successive Gauss-Jordan steps), so a bead takes ceil(D/2) barriers; the pivots of the
     // pair are a and det/a, the same two LDL^T pivots as one at a time
@@ -712,11 +695,6 @@ __global__ void __launch_bounds__(T) ring_logdet_kernel(
       double* B = Sb[cur ^ 1];
       if (k + 1 < D) {
         const int l = k + 1;
-        // every element's operands are read before the pivot block's inverse, and the empty
-        // asm below needs them all: otherwise the compiler moves each read into the branch
-        // that uses it, and a step waits on one LDS round trip per element and operand.
-        // Pinned up to kPinP elements per thread: beyond that the held operands cost
-        // occupancy (P = 6 would go from 3 to 2 waves per SIMD)
         double u0s[P], u1s[P], w0s[P], w1s[P], aes[P];
         auto operands = [&](int q) {
           const int r = er[q], cc = ec[q];
@@ -726,10 +704,6 @@ __global__ void __launch_bounds__(T) ring_logdet_kernel(
           w1s[q] = A[l * D + cc];
           aes[q] = A[ei[q]];
         };
-        if constexpr (P <= kPinP) {
-#pragma unroll
-          for (int q = 0; q < P; ++q) operands(q);
-        }
         const double a = A[k * D + k], b = A[k * D + l], cq = A[l * D + k], d = A[l * D + l];
         const double det = fma(a, d, -b * cq), id = pivot_recip(det);
         const double p00 = d * id, p01 = -b * id, p10 = -cq * id, p11 = a * id;  // block^-1
@@ -737,14 +711,9 @@ __global__ void __launch_bounds__(T) ring_logdet_kernel(
           pnum = tid == k ? a : tid == l ? det : pnum;
           pden = tid == k ? 1.0 : tid == l ? a : pden;
         }
-        if constexpr (P <= kPinP) {
-#pragma unroll
-          for (int q = 0; q < P; ++q)
-            asm volatile("" ::"v"(u0s[q]), "v"(u1s[q]), "v"(w0s[q]), "v"(w1s[q]), "v"(aes[q]));
-        }
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-          if constexpr (P > kPinP) operands(q);
+          operands(q);
           const int e = ei[q], r = er[q], cc = ec[q];
           // every case is a' - u~ P w~ with P = block^-1: a pivot row (r in K) takes
           // u~ = -e_r (row r of P A[K][cc]), a pivot column w~ = e_cc (-A[r][K] P, or P
@@ -759,42 +728,27 @@ __global__ void __launch_bounds__(T) ring_logdet_kernel(
           const double pw0 = p00 * w0 + p01 * w1, pw1 = p10 * w0 + p11 * w1;  // P A[K][cc]
           const double v = ae - (u0 * pw0 + u1 * pw1);
           B[e] = v;
-          if constexpr (SYM) B[mi[q]] = (r <= l) != (cc <= l) ? -v : v;  // swept: 0..l
+          B[mi[q]] = (r <= l) != (cc <= l) ? -v : v;  // swept: 0..l
         }
       } else {
-        double mrks[P], mkcs[P], aes[P];  // read first, as in the pair step
-        auto operands = [&](int q) {
-          mrks[q] = A[er[q] * D + k];
-          mkcs[q] = A[k * D + ec[q]];
-          aes[q] = A[ei[q]];
-        };
-        if constexpr (P <= kPinP) {
-#pragma unroll
-          for (int q = 0; q < P; ++q) operands(q);
-        }
         const double p = A[k * D + k], ip = pivot_recip(p);
         if (tid < 64) {
           pnum = tid == k ? p : pnum;
           pden = tid == k ? 1.0 : pden;
         }
-        if constexpr (P <= kPinP) {
-#pragma unroll
-          for (int q = 0; q < P; ++q) asm volatile("" ::"v"(mrks[q]), "v"(mkcs[q]), "v"(aes[q]));
-        }
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-          if constexpr (P > kPinP) operands(q);
           const int e = ei[q], r = er[q], cc = ec[q];
-          const double mrk = mrks[q], mkc = mkcs[q], a = aes[q];
+          const double mrk = A[r * D + k], mkc = A[k * D + cc], a = A[e];
           const double vr = cc == k ? ip : mkc * ip;
           const double vo = cc == k ? -mrk * ip : a - mrk * mkc * ip;
           const double v = r == k ? vr : vo;
           B[e] = v;
-          if constexpr (SYM) B[mi[q]] = (r <= k) != (cc <= k) ? -v : v;  // swept: 0..k
+          B[mi[q]] = (r <= k) != (cc <= k) ? -v : v;  // swept: 0..k
         }
       }
       cur ^= 1;
-      lds_sync<T>();
+      lds_sync();
     }
     // pivots: log|p| and the sign count; threads k < D <= 56 of wave 0 hold pivot k
     if (tid < 64) {
@@ -812,19 +766,13 @@ __global__ void __launch_bounds__(T) ring_logdet_kernel(
       double* out = sinv + (size_t)(boff[c] + i) * DD;
       const double* Minv = Sb[cur];
       // each thread stores the elements it overwrites first in the next bead (no barrier
-      // between): under SYM its lower element and the mirror, else its own elements
-      if constexpr (SYM) {
+      // between): its lower element and the mirror
 #pragma unroll
-        for (int q = 0; q < P; ++q)
-          if (ei[q] < DD) {
-            out[ei[q]] = Minv[ei[q]];
-            out[mi[q]] = Minv[mi[q]];
-          }
-      } else {
-#pragma unroll
-        for (int q = 0; q < P; ++q)
-          if (tid + T * q < DD) out[tid + T * q] = Minv[tid + T * q];
-      }
+      for (int q = 0; q < P; ++q)
+        if (ei[q] < DD) {
+          out[ei[q]] = Minv[ei[q]];
+          out[mi[q]] = Minv[mi[q]];
+        }
     }
   }
   if (tid == 0) {
@@ -878,8 +826,8 @@ template <typename F>
 int with_logdet_kernel(int D, F&& f) {
   if (D <= 16) return f(ring_factor_kernel<1>, 128);
   if (D <= 32) return f(ring_factor_kernel<2>, 128);
-  if (D * D <= 1536) return f(ring_logdet_kernel<4, 256, true, 6>, 256);  // D (D + 1) / 2 <= 1024
-  return f(ring_logdet_kernel<7, 256, true, 13>, 256);  // D (D + 1) / 2 <= 1792
+  if (D * D <= 1536) return f(ring_logdet_kernel<4, 6>, kRingThreads);  // D (D + 1) / 2 <= 1024
+  return f(ring_logdet_kernel<7, 13>, kRingThreads);  // D (D + 1) / 2 <= 1792
 }
 // the middle bead of its elimination
 __host__ __device__ inline int ring_middle(int D, int n) { return D <= 32 ? (n - 1) >> 1 : n - 1; }
@@ -900,14 +848,18 @@ __device__ __forceinline__ double dpp_mov(double v) {
   return __builtin_amdgcn_update_dpp(0.0, v, CTRL, 0xF, 0xF, false);
 }
 
-// the sum over each aligned group of Q (2, 4 or 8) lanes, in every lane of the group
-template <int Q>
-__device__ __forceinline__ double row_sum(double s) {
-  s += dpp_mov<0xB1>(s);                         // quad_perm [1,0,3,2]: lane ^ 1
-  if constexpr (Q >= 4) s += dpp_mov<0x4E>(s);   // quad_perm [2,3,0,1]: lane ^ 2
-  if constexpr (Q >= 8) s += dpp_mov<0x141>(s);  // row_half_mirror: lane 7 - l of 8
-  return s;
+// the sum over each aligned group of four lanes, in every lane of the group
+__device__ __forceinline__ double quad_sum(double s) {
+  s += dpp_mov<0xB1>(s);        // quad_perm [1,0,3,2]: lane ^ 1
+  return s + dpp_mov<0x4E>(s);  // quad_perm [2,3,0,1]: lane ^ 2
 }
+
+// Above 32 dofs: Q lanes per block row, KPL columns each (kMaxD <= Q KPL), and loads P steps
+// ahead (the registers of a deeper prefetch)
+namespace eta1_wide {
+constexpr int Q = 4, KPL = 16, P = 4, QK = Q * KPL;
+static_assert(Q * kMaxD <= kRingThreads && kMaxD <= QK, "a workgroup holds every row");
+}  // namespace eta1_wide
 
 // One sweep of K steps; returns the LDS buffer (of the two in zb) that holds its last vector.
 // src: v (forward) or the t the forward sweep left in dst (backward).  The per-step barrier
@@ -915,11 +867,11 @@ __device__ __forceinline__ double row_sum(double s) {
 // r = tid / Q, lane q), each holding the KPL columns k = q + Q j of its row; a row's sum is a
 // DPP butterfly inside its Q lanes.  Byte offsets within a chain fit 31 bits (the host checks
 // n D^2 8 < 2^31).
-template <int Q, int KPL, int P, int NT, bool FWD>
+template <bool FWD>
 __device__ __forceinline__ int solve_sweep(int D, int n, int h, int K, int ht, double c,
                                            const double* __restrict__ S, const double* src,
                                            double* dst, double* zb, int cur) {
-  constexpr int QK = Q * KPL;
+  using namespace eta1_wide;
   const int r = ht / Q, q = ht - r * Q;
   const int rr = min(r, D - 1);
   const bool wr = q == 0 && r < D;
@@ -956,7 +908,7 @@ __device__ __forceinline__ int solve_sweep(int D, int n, int h, int K, int ht, d
           t0 += a[s][j] * u[q + Q * j];
           if (j + 1 < KPL) t1 += a[s][j + 1] * u[q + Q * (j + 1)];
         }
-        const double t = row_sum<Q>(t0 + t1), ev = e[s];
+        const double t = quad_sum(t0 + t1), ev = e[s];
         const int so = bead(k + P) * DD8, i = bead(k);
 #pragma unroll
         for (int j = 0; j < KPL; ++j) a[s][j] = buffer_ld(Sb, ko[j], so);
@@ -975,7 +927,7 @@ __device__ __forceinline__ int solve_sweep(int D, int n, int h, int K, int ht, d
           }
         }
         cur ^= 1;
-        lds_sync<NT>();
+        lds_sync();
       }
     }
   }
@@ -992,15 +944,14 @@ __device__ __forceinline__ double start_entry(int64_t e) {
 // work holds [v | y] per chain (2 n D); fresh = 1 starts from a fixed generic vector,
 // otherwise the previous v is continued.  Stops after iters iterations, or earlier once eta
 // changes by at most tol relative; chains with act[c] == 0 are left as they are.
-// More than 32 dofs, D <= Q KPL; one end, h = n - 1.
-template <int Q, int KPL, int P>
+// More than 32 dofs; one end, h = n - 1.
 __global__ void __launch_bounds__(kRingThreads) ring_eta1_kernel(
     int D, const int* __restrict__ nn, const int64_t* __restrict__ boff,
     const double* __restrict__ betan, const double* __restrict__ sinv, double* __restrict__ work,
     const double* __restrict__ shift, int iters, int fresh, double tol,
     const int* __restrict__ act, double* __restrict__ eta1) {
-  static_assert(Q * (kRingThreads / Q) == kRingThreads && (Q == 2 || Q == 4 || Q == 8), "lanes per row");
-  constexpr int NT = kRingThreads, QK = Q * KPL;
+  using namespace eta1_wide;
+  constexpr int NT = kRingThreads;
   __shared__ double red[NT];
   __shared__ double zb[2 * QK], zm[QK];
   const int cix = blockIdx.x, n = nn[cix], tid = threadIdx.x;
@@ -1020,14 +971,14 @@ __global__ void __launch_bounds__(kRingThreads) ring_eta1_kernel(
     v[e] = t;
     nrm += t * t;
   }
-  nrm = sqrt(block_sum<NT>(nrm, red));
+  nrm = sqrt(block_sum(nrm, red));
   for (int64_t e = tid; e < tot; e += NT) v[e] /= nrm;
   __syncthreads();
   double eta = 0.0, prev = 0.0;
   for (int it = 0; it < iters; ++it) {
     if (tid < D) zb[tid] = v[tid];
     __syncthreads();
-    const int cur = solve_sweep<Q, KPL, P, NT, true>(D, n, h, h, tid, c, S, v, y, zb, 0);
+    const int cur = solve_sweep<true>(D, n, h, h, tid, c, S, v, y, zb, 0);
     if (tid < D) zm[tid] = zb[cur * QK + tid];  // z_h; y_h = S_h^-1 z_h
     __syncthreads();
     {
@@ -1036,22 +987,22 @@ __global__ void __launch_bounds__(kRingThreads) ring_eta1_kernel(
       double t = 0.0;
 #pragma unroll
       for (int j = 0; j < KPL; ++j) t += Sh[min(q + Q * j, D - 1)] * zm[q + Q * j];
-      t = row_sum<Q>(t);
+      t = quad_sum(t);
       if (q == 0 && r < D) {
         y[(int64_t)h * D + r] = t;
         zb[r] = t;
       }
     }
     __syncthreads();  // and the t of every lane, in y, before the backward sweep reads them
-    solve_sweep<Q, KPL, P, NT, false>(D, n, h, max(h - 1, 0), tid, c, S, y, y, zb, 0);  // y_0 = t_0
+    solve_sweep<false>(D, n, h, max(h - 1, 0), tid, c, S, y, y, zb, 0);  // y_0 = t_0
     __syncthreads();
     double mu = 0.0, yy = 0.0;
     for (int64_t e = tid; e < tot; e += NT) {
       mu += v[e] * y[e];
       yy += y[e] * y[e];
     }
-    mu = block_sum<NT>(mu, red);
-    yy = sqrt(block_sum<NT>(yy, red));
+    mu = block_sum(mu, red);
+    yy = sqrt(block_sum(yy, red));
     for (int64_t e = tid; e < tot; e += NT) v[e] = y[e] / yy;
     __syncthreads();
     eta = sig + 1.0 / mu;
@@ -1823,12 +1774,10 @@ int ring_lowest_eigen(rp_ring* r, const std::vector<int>& ng, double* eta) {
     cleanup();
     return rc;
   }
-  // above 32 dofs: 4 lanes x 16 columns per block row, 4 steps ahead (the registers of a deeper
-  // prefetch)
   auto eta1 = [&](const double* shift, int iters, int fresh, double tol, const int* act) -> int {
     auto kern = r->D <= 28   ? ring_eta1_wave_kernel<14, 7>
                 : r->D <= 32 ? ring_eta1_wave_kernel<16, 6>
-                             : ring_eta1_kernel<4, 16, 4>;
+                             : ring_eta1_kernel;
     kern<<<C, r->D <= 32 ? 128 : kRingThreads, 0, r->s>>>(r->D, r->d_n.p, r->d_boff.p, r->d_betan.p,
                                                          r->d_sinv.p, r->d_work.p, shift, iters, fresh,
                                                          tol, act, r->d_eta.p);
