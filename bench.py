@@ -295,7 +295,18 @@ def copy_probe(mib):
     print(json.dumps({"copy_probe_mib": mib, "bytes_read": n * 8, "bytes_written": n * 8}))
 
 
-def instanton_sample(pes, sp, nchain=256, reps=10, seed=4):
+def per_chain(columns, path=None):
+    """The spread of each column of a per-chain table, {name: [min, median, max]}; the table
+    itself goes to the JSON file at path, if any: 256 chains of six columns would be most of the
+    result line."""
+    if path:
+        with open(path, "w") as f:
+            json.dump({k: [float(f"{float(x):.10g}") for x in v] for k, v in columns.items()}, f)
+    return {k: [float(f"{float(q):.10g}") for q in (np.min(v), np.median(v), np.max(v))]
+            for k, v in columns.items()}
+
+
+def instanton_sample(pes, sp, nchain=256, reps=10, seed=4, table=None):
     """The batched instanton workload on the same EVB surface: nchain open chains with N
     uniform in [64, 1024] and beta in [1000, 8000] (RPI betan = beta/N, rpi_ser.f90:45).
 
@@ -311,7 +322,8 @@ def instanton_sample(pes, sp, nchain=256, reps=10, seed=4):
     V0 moved down to the instanton's lowest bead where it dips below V(well1);
     lndetJ at each instanton, lndetJ0 with every bead at well 1, and the splitting
     Delta = 2 theta / betan.  Reported: converged chains, iterations, wall time of each stage
-    and in total, and per chain S = betan U_M, lndetJ, lndetJ0 and Delta (cm^-1)."""
+    and in total, and the spread over the chains of S = betan U_M, lndetJ, lndetJ0 and Delta
+    (cm^-1); every chain's go to the JSON file `table`, if given."""
     from rptunnel import Ring
 
     rng = np.random.default_rng(seed)
@@ -405,9 +417,6 @@ def instanton_sample(pes, sp, nchain=256, reps=10, seed=4):
     theta = bn * np.exp(-skink) * np.sqrt(skink / (2.0 * 3.14159265358979)) / phi
     delta_cm = 2.0 * theta / bn * 219475.0
 
-    def r10(a):
-        return [float(f"{float(x):.10g}") for x in a]
-
     return {"workload": f"evb27 instantons: {nchain} chains, N in [64, 1024] (total {beads} beads), "
                         "beta in [1000, 8000]",
             "um_grad_bead_evals_per_s": beads / t_um,
@@ -430,8 +439,8 @@ def instanton_sample(pes, sp, nchain=256, reps=10, seed=4):
                                    "max_abs_S_difference": float(np.max(np.abs(pc_ds))),
                                    "chains_lower_S_than_plain": int(np.sum(pc_ds < 0.0))},
                 "negative_eigenvalues_at_instanton": {str(k): int(np.sum(nneg == k)) for k in np.unique(nneg)},
-                "per_chain": {"n": ns, "beta": r10(betas), "S": r10(skink), "lndetJ": r10(ldj),
-                              "lndetJ0": r10(ldj0), "delta_cm-1": r10(delta_cm)}}}
+                "min_median_max": per_chain({"n": ns, "beta": betas, "S": skink, "lndetJ": ldj,
+                                             "lndetJ0": ldj0, "delta_cm-1": delta_cm}, table)}}
 
 
 def water_sample(steps=16, warmup=8, ntraj=1024, n=128, nchain=256):
@@ -607,6 +616,8 @@ def main():
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-instanton", action="store_true",
                     help="skip the batched-instanton sample reported beside the headline")
+    ap.add_argument("--instanton-table", metavar="JSON",
+                    help="write S, lndetJ, lndetJ0 and the splitting of every instanton chain there")
     ap.add_argument("--no-equal", action="store_true",
                     help="skip the same-TI-on-both-paths sample reported beside the headline")
     ap.add_argument("--no-andersen", action="store_true",
@@ -708,7 +719,7 @@ def main():
     inst = None
     if not args.no_instanton:
         log("instanton sample (256 chains)")
-        inst = instanton_sample(pes, sp)
+        inst = instanton_sample(pes, sp, table=args.instanton_table)
 
     coupled = None
     if not args.no_coupled2d:
