@@ -1,8 +1,8 @@
 // rp_batch.hip -- host side of the batched engine (rp_batch_* in rp_hip.h).
 //
-// Polymers are grouped into families of equal (n, betan): one family shares the
-// transform T and the per-mode table, and is advanced by one launch of the fused
-// step kernel (rp_batch_kernel.h) with one workgroup per polymer.
+// Polymers are grouped into families of equal (n, betan): one family shares the tables of its
+// modes, and is advanced by one launch of the fused step kernel (rp_batch_kernel.h), whose
+// workgroups hold one polymer or several (launch_batch_kind).
 #include <algorithm>
 #include <chrono>
 #include <climits>

@@ -1,5 +1,4 @@
-// Batched-engine kernels for the water clusters (1, 2 or 6 molecules), on the full
-// (unfolded) transforms.
+// Batched-engine kernels for the water clusters (1, 2 or 6 molecules).
 #include "rp_batch_kernel.h"
 
 namespace rp {

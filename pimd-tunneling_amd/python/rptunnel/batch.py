@@ -117,7 +117,7 @@ class Batch:
         return list(zip(n[: nf.value].tolist(), cnt[: nf.value].tolist()))
 
     def family_shapes(self):
-        """Per family: (n, waves per workgroup, MFMA units per wave, folded transforms)."""
+        """Per family: (n, wave budget, MFMA units per wave of it, even n and no water cluster)."""
         out = []
         for f, (n, _) in enumerate(self.families()):
             w, u, fo = C.c_int(0), C.c_int(0), C.c_int(0)
