@@ -1567,9 +1567,10 @@ extern "C" int rp_ring_device(const rp_ring* r, int* device) {
 // queued, the ring's own stream for this).
 // A kernel on another GPU's stream would run there, on buffers of this one.
 static int stream_check(const rp_ring* r, hipStream_t s) {
-  hipDevice_t dev = -1;
-  RP_HIP(hipStreamGetDevice(s, &dev));
-  RP_REQUIRE(dev == r->dev, "rp_ring_*_stream: the stream belongs to GPU %d, the ring to GPU %d", (int)dev, r->dev);
+  int dev = -1;
+  if (s) RP_HIP(hipStreamGetDevice(s, &dev));
+  else RP_HIP(hipGetDevice(&dev));  // the default stream is the current GPU's
+  RP_REQUIRE(dev == r->dev, "rp_ring_*_stream: the stream belongs to GPU %d, the ring to GPU %d", dev, r->dev);
   return RP_OK;
 }
 static int stream_begin(rp_ring* r, hipStream_t s) {

@@ -47,6 +47,9 @@ def _f64(t: torch.Tensor) -> torch.Tensor:
 
 def _call(name: str, ring: Ring, like: torch.Tensor, *tensors) -> None:
     """One stream-ordered library call on torch's current stream of the tensors' GPU."""
+    if torch.cuda.current_device() != like.device.index:  # a default stream is the current GPU's
+        with torch.cuda.device(like.device):
+            return _call(name, ring, like, *tensors)
     stream = torch.cuda.current_stream(like.device).cuda_stream
     ptrs = [None if t is None else C.c_void_p(t.data_ptr()) for t in tensors]
     L.check(getattr(L.lib(), name)(ring.h, *ptrs, C.c_void_p(stream)))
